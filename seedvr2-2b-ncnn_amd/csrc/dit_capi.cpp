@@ -36,22 +36,21 @@ GemmProblem problem(const uint16_t* A, int lda, const uint16_t* W, int ldw, int 
     return p;
 }
 
-constexpr int VID_IN = 132, VID_IN_PAD = 192;   // patch channels 33 x 2 x 2; K padded to the GEMM step (64)
-constexpr int VID_OUT = 64, VID_OUT_PAD = 256;  // output channels 16 x 2 x 2; N padded to the GEMM tile
+constexpr int VID_OUT = 64;  // output channels 16 x 2 x 2
 
 }  // namespace
 
 struct dit_io {
     int device = 0;
-    uint16_t* vid_in_w = nullptr;   // [2560][192], columns 132.. zero
+    uint16_t* vid_in_w = nullptr;   // [2560][EMBED_K] in fragment order
     const float* vid_in_b = nullptr;
     const uint16_t* txt_in_w = nullptr;
     const float* txt_in_b = nullptr;
     const float* out_norm_w = nullptr;
     const float* out_ada_shift = nullptr;
     const float* out_ada_scale = nullptr;
-    uint16_t* vid_out_w = nullptr;  // [256][2560], rows 64.. zero
-    float* vid_out_b = nullptr;     // [256], 64.. zero
+    uint16_t* vid_out_w = nullptr;  // [64][2560] in fragment order
+    float* vid_out_b = nullptr;     // [64]
 };
 
 extern "C" {
@@ -69,18 +68,10 @@ int dit_io_create(awa_ctx* ctx, const dit_io_weights* w, dit_io** out, awa_strea
     io->device = ctx->device;
     io->vid_in_b = w->vid_in_b; io->txt_in_w = w->txt_in_w; io->txt_in_b = w->txt_in_b;
     io->out_norm_w = w->out_norm_w; io->out_ada_shift = w->out_ada_shift; io->out_ada_scale = w->out_ada_scale;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&io->vid_in_w), (size_t)DIM * VID_IN_PAD * 2);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&io->vid_out_w), (size_t)VID_OUT_PAD * DIM * 2);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&io->vid_out_b), VID_OUT_PAD * 4);
-    // zero, then copy the real rows / columns in (set-up, not in a captured sequence)
-    if (e == hipSuccess) e = hipMemsetAsync(io->vid_in_w, 0, (size_t)DIM * VID_IN_PAD * 2, s);
-    if (e == hipSuccess) e = hipMemsetAsync(io->vid_out_w, 0, (size_t)VID_OUT_PAD * DIM * 2, s);
-    if (e == hipSuccess) e = hipMemsetAsync(io->vid_out_b, 0, VID_OUT_PAD * 4, s);
-    if (e == hipSuccess)
-        e = hipMemcpy2DAsync(io->vid_in_w, VID_IN_PAD * 2, w->vid_in_w, VID_IN * 2, VID_IN * 2, DIM,
-                             hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(io->vid_out_w, w->vid_out_w, (size_t)VID_OUT * DIM * 2, hipMemcpyDeviceToDevice, s);
+    hipError_t e = hipMalloc(reinterpret_cast<void**>(&io->vid_in_w), (size_t)DIM * EMBED_K * 2);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&io->vid_out_w), (size_t)VID_OUT * DIM * 2);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&io->vid_out_b), VID_OUT * 4);
+    if (e == hipSuccess) e = launch_end_weights(w->vid_in_w, io->vid_in_w, w->vid_out_w, io->vid_out_w, s);
     if (e == hipSuccess) e = hipMemcpyAsync(io->vid_out_b, w->vid_out_b, VID_OUT * 4, hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) {
         set_err(ctx, "dit_io_create: %s", hipGetErrorString(e));
@@ -102,12 +93,7 @@ void dit_io_destroy(awa_ctx* ctx, dit_io* io) {
 
 namespace {
 // workspace bytes of each entry point (the offsets below follow the same layouts)
-size_t embed_ws_bytes(int Lv, int TXT) {
-    return align256((size_t)Lv * VID_IN_PAD * 2) + align256((size_t)TXT * 5120 * 2);
-}
-size_t final_ws_bytes(int Lv) {
-    return align256(2 * DIM * 4) + align256((size_t)Lv * DIM * 2) + align256((size_t)Lv * VID_OUT_PAD * 4);
-}
+size_t embed_ws_bytes(int TXT) { return (size_t)EMBED_TXT_SPLIT * TXT * DIM * 4; }
 size_t layer_ws_bytes(int M, int mlp) {
     return align256(12 * DIM * 4) + align256((size_t)M * DIM * 2) + align256((size_t)M * QKV * 2) +
            align256((size_t)M * DIM * 2) + align256((size_t)M * mlp * 2);
@@ -121,9 +107,9 @@ int dit_reserve(awa_ctx* ctx, const awa_geom* g, int mlp) {
         return AWA_EARG;
     }
     const int Lv = g->plan.Lv, TXT = g->plan.txt_len;
-    const size_t need = std::max(layer_ws_bytes(Lv + TXT, mlp), std::max(embed_ws_bytes(Lv, TXT), final_ws_bytes(Lv)));
     DeviceGuard dg(ctx->device);
-    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, need));
+    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes,
+                             std::max(layer_ws_bytes(Lv + TXT, mlp), embed_ws_bytes(TXT))));
     return awa_reserve(ctx, g, AWA_BF16);
 }
 
@@ -135,23 +121,15 @@ int dit_embed(awa_ctx* ctx, const dit_io* io, const float* d_grid, int T, int H,
     }
     DeviceGuard dg(ctx->device);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const int Lv = T * (H / 2) * (W / 2), M = Lv + TXT;
-    // workspace: patches [Lv][192] bf16 | text [TXT][5120] bf16
-    const size_t o_t = align256((size_t)Lv * VID_IN_PAD * 2);
-    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, embed_ws_bytes(Lv, TXT)));
-    uint16_t* patch = static_cast<uint16_t*>(ctx->ws);
-    uint16_t* txt = reinterpret_cast<uint16_t*>(static_cast<char*>(ctx->ws) + o_t);
-    HIPCK(ctx, launch_patchify(d_grid, T, H, W, patch, VID_IN_PAD, s));
-    HIPCK(ctx, launch_cast_f32_bf16(d_txt, txt, (int64_t)TXT * 5120, s));
-    // x = A W^T + b: the residual epilogue on a zeroed x, gate 1
-    HIPCK(ctx, launch_zero(d_x, (size_t)M * DIM * 4, s));
-    GemmBatch b{};
-    b.nprob = 2;
-    b.p[0] = problem(patch, VID_IN_PAD, io->vid_in_w, VID_IN_PAD, Lv, DIM, VID_IN_PAD, d_x, DIM);
-    b.p[0].bias = io->vid_in_b;
-    b.p[1] = problem(txt, 5120, io->txt_in_w, 5120, TXT, DIM, 5120, d_x + (size_t)Lv * DIM, DIM);
-    b.p[1].bias = io->txt_in_b;
-    HIPCK(ctx, launch_gemm(EPI_RESID, b, s));
+    EmbedArgs a{};
+    a.grid = d_grid; a.H = H; a.W2 = W / 2;
+    a.Lv = T * (H / 2) * (W / 2); a.TXT = TXT;
+    a.vid_w = io->vid_in_w; a.vid_b = io->vid_in_b;
+    a.txt = d_txt; a.txt_w = io->txt_in_w; a.txt_b = io->txt_in_b;
+    a.x = d_x;
+    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, embed_ws_bytes(TXT)));
+    a.part = static_cast<float*>(ctx->ws);
+    HIPCK(ctx, launch_embed(a, s));
     return AWA_OK;
 }
 
@@ -163,28 +141,14 @@ int dit_final(awa_ctx* ctx, const dit_io* io, const float* d_emb, const float* d
     }
     DeviceGuard dg(ctx->device);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const int Lv = T * (H / 2) * (W / 2);
-    // workspace: scale, shift [2][2560] f32 | h [Lv][2560] bf16 | y [Lv][256] f32
-    const size_t o_h = align256(2 * DIM * 4);
-    const size_t o_y = o_h + align256((size_t)Lv * DIM * 2);
-    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, final_ws_bytes(Lv)));
-    char* ws = static_cast<char*>(ctx->ws);
-    float* scale = reinterpret_cast<float*>(ws);
-    float* shift = scale + DIM;
-    uint16_t* h = reinterpret_cast<uint16_t*>(ws + o_h);
-    float* y = reinterpret_cast<float*>(ws + o_y);
-    HIPCK(ctx, launch_final_ada(d_emb, io->out_norm_w, io->out_ada_scale, io->out_ada_shift, scale, shift, s));
-    NormArgs na{};
-    na.x = d_x; na.h = h; na.M = Lv; na.split = Lv; na.eps = eps;
-    na.scale0 = scale; na.shift0 = shift;
-    HIPCK(ctx, launch_norm_ada(na, s));
-    HIPCK(ctx, launch_zero(y, (size_t)Lv * VID_OUT_PAD * 4, s));
-    GemmBatch b{};
-    b.nprob = 1;
-    b.p[0] = problem(h, DIM, io->vid_out_w, DIM, Lv, VID_OUT_PAD, DIM, y, VID_OUT_PAD);
-    b.p[0].bias = io->vid_out_b;
-    HIPCK(ctx, launch_gemm(EPI_RESID, b, s));
-    HIPCK(ctx, launch_unpatchify(y, VID_OUT_PAD, T, H, W, d_out, s));
+    FinalArgs a{};
+    a.x = d_x; a.emb = d_emb;
+    a.norm_w = io->out_norm_w; a.ada_scale = io->out_ada_scale; a.ada_shift = io->out_ada_shift;
+    a.W = io->vid_out_w; a.bias = io->vid_out_b;
+    a.rows = T * (H / 2) * (W / 2); a.H = H; a.W2 = W / 2;
+    a.eps = eps;
+    a.out = d_out;
+    HIPCK(ctx, launch_final(a, s));
     return AWA_OK;
 }
 

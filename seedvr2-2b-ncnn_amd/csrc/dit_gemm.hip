@@ -427,21 +427,24 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmBatch b) {
 
 }  // namespace
 
+int device_cus() {
+    // looked up once per device (threads may race to store the same value)
+    static std::atomic<int> n_cu[64];
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    if (dev < 0 || dev >= 64) return 256;
+    int c = n_cu[dev].load(std::memory_order_relaxed);
+    if (c == 0 && hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
+        n_cu[dev].store(c, std::memory_order_relaxed);
+    return c > 0 ? c : 256;
+}
+
 // Tiles of 256 x 256 or 256 x 224 (rows of A), whichever needs fewer
 // workgroup rounds times rows per tile on the device's CUs: with 5498 rows,
 // 2560 output features give 220 tiles of 256 rows (1 round, 36 CUs idle) or
 // 250 of 224 (1 round, 12 % less work per tile).
 hipError_t launch_gemm(int epi, GemmBatch& b, hipStream_t s) {
-    // CU count per device, looked up once (threads may race to store the same value)
-    static std::atomic<int> n_cu[64];
-    int dev = 0, cus = 256;
-    (void)hipGetDevice(&dev);
-    if (dev >= 0 && dev < 64) {
-        int c = n_cu[dev].load(std::memory_order_relaxed);
-        if (c == 0 && hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
-            n_cu[dev].store(c, std::memory_order_relaxed);
-        if (c > 0) cus = c;
-    }
+    const int cus = device_cus();
     auto tiles_for = [&](int bm) {
         long t = 0;
         for (int i = 0; i < b.nprob; i++) t += (long)(b.p[i].N / BN) * ((b.p[i].M + bm - 1) / bm);

@@ -27,6 +27,8 @@ struct GemmBatch {
     int tiles0, total_tiles;
 };
 
+// compute units of the current device (256 if it cannot be asked)
+int device_cus();
 hipError_t launch_gemm(int epi, GemmBatch& b, hipStream_t s);
 
 // h[m] = bf16(RMSNorm(x[m]) * scale + shift); rows >= split use the second
@@ -60,12 +62,43 @@ hipError_t launch_gemv_f32(const float* W, const float* b, const float* x, float
                            int silu, hipStream_t s);
 hipError_t launch_sinusoid(float t, float* e, int dim, hipStream_t s);
 
-// grid (T, H, W, 33) fp32 -> [T (H/2) (W/2)][kpad] bf16 patches, (ph, pw, c) order
-hipError_t launch_patchify(const float* grid, int T, int H, int W, uint16_t* out, int kpad, hipStream_t s);
-// [T (H/2) (W/2)][ldy] fp32 (first 64 columns) -> (T, H, W, 16) fp32
-hipError_t launch_unpatchify(const float* y, int ldy, int T, int H, int W, float* out, hipStream_t s);
-// output-layer modulation vectors: scale = w (emb[6d+1] + ada_scale), shift = emb[6d] + ada_shift
-hipError_t launch_final_ada(const float* emb, const float* w, const float* ada_scale, const float* ada_shift,
-                            float* scale, float* shift, hipStream_t s);
+// The model's ends (dit_ends.hip).  x [Lv + TXT][2560] from the latent grid
+// (T, H, 2 W2, 33) and the text features [TXT][5120].
+constexpr int EMBED_K = 160;  // 132 patch channels and zeros up to whole k32 steps
+constexpr int EMBED_TXT_SPLIT = 16;  // parts of the text projection's K
+struct EmbedArgs {
+    const float* grid;
+    int H, W2;
+    int Lv, TXT;
+    const uint16_t* vid_w;  // [2560][EMBED_K] in fragment order
+    const float* vid_b;
+    const float* txt;
+    const uint16_t* txt_w;  // [2560][5120]
+    const float* txt_b;
+    float* x;
+    float* part;     // workspace: [EMBED_TXT_SPLIT][TXT][2560] partial products of the text
+    int txt_blocks;  // filled by launch_embed
+};
+hipError_t launch_embed(const EmbedArgs& a, hipStream_t s);
+// out (T, H, 2 W2, 16) from the first `rows` rows of x and the timestep embedding
+struct FinalArgs {
+    const float* x;
+    const float* emb;
+    const float* norm_w;
+    const float* ada_scale;
+    const float* ada_shift;
+    const uint16_t* W;  // [64][2560] in fragment order
+    const float* bias;  // [64]
+    int rows, H, W2;
+    float eps;
+    float* out;
+    int rpw;  // rows per workgroup, filled by launch_final
+};
+hipError_t launch_final(const FinalArgs& a, hipStream_t s);
+// The video weights of both ends, [2560][132] and [64][2560], in the fragment
+// order that launch_embed and launch_final read: EMBED_K per input row (zeros
+// past 132), DIM per output row.
+hipError_t launch_end_weights(const uint16_t* vid_in, uint16_t* vid_in_frag, const uint16_t* vid_out,
+                              uint16_t* vid_out_frag, hipStream_t s);
 
 }  // namespace awa
