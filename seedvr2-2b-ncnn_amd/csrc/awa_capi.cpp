@@ -89,7 +89,7 @@ hipError_t dalloc(T** p, size_t n) {
 
 void free_geom_buffers(awa_geom* g) {
     void* ptrs[] = {g->d_slices, g->d_cumf, g->d_vidx, g->d_tile_base, g->d_tile_win,
-                    g->d_items, g->d_f32_units, g->d_sched_start, g->d_sched_desc, g->d_vfreq, g->d_tfreq,
+                    g->d_items, g->d_f32_work, g->d_sched_start, g->d_sched_desc, g->d_vfreq, g->d_tfreq,
                     g->d_vcs, g->d_tcs, g->d_tile_meta, g->d_vrow};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -98,6 +98,14 @@ void free_geom_buffers(awa_geom* g) {
 }  // namespace
 
 namespace awa {
+
+void item_desc(const GeomPlan& P, int h, int i, int32_t d[8]) {
+    const int w = P.items[4 * i];
+    const int32_t v[8] = {h | (w << 8), P.items[4 * i + 1], P.items[4 * i + 2], P.cumf[w],
+                          P.tile_base[w], P.tile_base[w + 1] - P.tile_base[w],
+                          P.n_vid_tiles + (P.txt_sets == 1 ? 0 : w) * P.ntt, P.cumf[w + 1] - P.cumf[w]};
+    std::copy(v, v + 8, d);
+}
 
 // 64-row tiles of every window plus the text tiles, and the work items of the
 // attention kernel (one window, two query tiles).
@@ -137,17 +145,30 @@ void plan_tiles(GeomPlan& P) {
         }
     }
     P.n_items = (int)P.items.size() / 4;
-    // fp32 units: every query tile of every item, longest windows first
-    std::vector<int> units;
-    for (int i = 0; i < P.n_items; i++)
-        for (int half = 0; half < 2; half++)
-            if (P.items[4 * i + 1 + half] >= 0) units.push_back(2 * i + half);
-    auto nkey = [&](int u) {
-        const int w = P.items[4 * (u >> 1)];
-        return P.tile_base[w + 1] - P.tile_base[w];
-    };
-    std::stable_sort(units.begin(), units.end(), [&](int x, int y) { return nkey(x) > nkey(y); });
-    P.f32_units.assign(units.begin(), units.end());
+    // fp32 workgroups: (window, head) groups longest first onto the least
+    // loaded XCD, each XCD's list longest window first
+    constexpr int XCDS = 8;
+    auto nkey = [&](int w) { return P.tile_base[w + 1] - P.tile_base[w] + P.ntt; };
+    std::vector<int> first(P.nwin + 1, 0);
+    for (int i = 0; i < P.n_items; i++) first[P.items[4 * i] + 1] = i + 1;
+    for (int w = 0; w < P.nwin; w++) first[w + 1] = std::max(first[w + 1], first[w]);
+    std::vector<int> order(P.nwin);
+    for (int w = 0; w < P.nwin; w++) order[w] = w;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return nkey(x) > nkey(y); });
+    std::vector<std::vector<std::pair<int, int>>> list(XCDS);  // (head, item)
+    long load[XCDS] = {};
+    for (int w : order)
+        for (int h = 0; h < HEADS; h++) {
+            const int x = (int)(std::min_element(load, load + XCDS) - load);
+            load[x] += (long)nkey(w) * (first[w + 1] - first[w]);
+            for (int i = first[w]; i < first[w + 1]; i++) list[x].push_back({h, i});
+        }
+    size_t len = 0;
+    for (const auto& l : list) len = std::max(len, l.size());
+    P.f32_work.assign(len * XCDS * 8, -1);
+    for (int x = 0; x < XCDS; x++)
+        for (size_t k = 0; k < list[x].size(); k++)
+            item_desc(P, list[x][k].first, list[x][k].second, &P.f32_work[(k * XCDS + x) * 8]);
 }
 
 // Static schedule of the persistent bf16 attention
@@ -257,11 +278,8 @@ void plan_schedule(GeomPlan& P, int n_slots) {
     int n = 0;
     for (int sl = 0; sl < n_slots; sl++) {
         for (int id : slot_work[sl]) {
-            const int h = id / P.n_items, i = id % P.n_items, w = P.items[4 * i];
-            const int32_t d[8] = {h | (w << 8), P.items[4 * i + 1], P.items[4 * i + 2], P.cumf[w],
-                                  P.tile_base[w], P.tile_base[w + 1] - P.tile_base[w],
-                                  P.n_vid_tiles + (P.txt_sets == 1 ? 0 : w) * P.ntt,
-                                  P.cumf[w + 1] - P.cumf[w]};
+            int32_t d[8];
+            item_desc(P, id / P.n_items, id % P.n_items, d);
             P.sched_desc.insert(P.sched_desc.end(), d, d + 8);
             n++;
         }
@@ -288,9 +306,9 @@ int upload_plan(awa_ctx* ctx, awa_geom* g, hipStream_t s) {
     HIPCK(ctx, dalloc(&g->d_tile_base, P.tile_base.size()));
     HIPCK(ctx, dalloc(&g->d_tile_win, P.tile_win.size()));
     HIPCK(ctx, dalloc(&g->d_items, P.items.size()));
-    HIPCK(ctx, dalloc(&g->d_f32_units, P.f32_units.size()));
-    if (!P.f32_units.empty())
-        HIPCK(ctx, hipMemcpyAsync(g->d_f32_units, P.f32_units.data(), P.f32_units.size() * 4,
+    HIPCK(ctx, dalloc(&g->d_f32_work, P.f32_work.size()));
+    if (!P.f32_work.empty())
+        HIPCK(ctx, hipMemcpyAsync(g->d_f32_work, P.f32_work.data(), P.f32_work.size() * 4,
                                   hipMemcpyHostToDevice, s));
     HIPCK(ctx, hipMemcpyAsync(g->d_tile_base, P.tile_base.data(), P.tile_base.size() * 4,
                               hipMemcpyHostToDevice, s));
@@ -430,7 +448,9 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     pa.nq_v = d_nq_v; pa.nk_v = d_nk_v; pa.nq_t = d_nq_t; pa.nk_t = d_nk_t;
     pa.tile_meta = g->d_tile_meta; pa.vrow = g->d_vrow;
     pa.vcs = g->d_vcs; pa.tcs = g->d_tcs;
-    pa.Qp = base; pa.Kp = base + off_k; pa.Vp = bf16 ? nullptr : base + off_v;
+    // bf16: Q and K; fp32: K, V and the blocks' factors (in Q's place)
+    pa.Qp = bf16 ? base : nullptr; pa.Kp = base + off_k; pa.Vp = bf16 ? nullptr : base + off_v;
+    pa.kexp = reinterpret_cast<float*>(base); pa.vexp = pa.kexp + (size_t)HEADS * P.n_tiles * 4;
     pa.n_vid_tiles = P.n_vid_tiles; pa.ntt = P.ntt; pa.txt_sets = P.txt_sets; pa.txt_len = P.txt_len;
     pa.n_tiles = P.n_tiles; pa.eps = eps;
     pa.qscale = (1.0f / std::sqrt(128.0f)) * 1.4426950408889634f;
@@ -448,8 +468,10 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.tpart = reinterpret_cast<float*>(base + off_t);
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;
     sa.n_tiles = P.n_tiles; sa.n_items = P.n_items; sa.nwin = P.nwin;
-    sa.scale_log2e = 1.0f;  // the pack kernel folded the scale into Q
-    sa.f32_units = g->d_f32_units; sa.n_f32_units = (int)P.f32_units.size();
+    sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size() / 8;
+    sa.kexp = pa.kexp; sa.vexp = pa.vexp;
+    sa.tile_meta = g->d_tile_meta; sa.vcs = g->d_vcs; sa.tcs = g->d_tcs; sa.nq_v = d_nq_v; sa.nq_t = d_nq_t;
+    sa.eps = eps; sa.qscale = pa.qscale;
     HIPCK(ctx, launch_sdpa(dtype, sa, s));
     HIPCK(ctx, mark());
 

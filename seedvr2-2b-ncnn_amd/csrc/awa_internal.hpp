@@ -7,11 +7,11 @@
 // Per head h and tile k the packed buffers hold
 //   Qp[h][k][slot 0..63][d 0..127]   normalised + rotated queries
 //   Kp[h][k][slot 0..63][d 0..127]   normalised + rotated keys
-//   Vp[h][k][d 0..127][slot 0..63]   values, transposed inside the tile (fp32 only)
-// in the storage type of the op (bf16 or fp32).  Unused slots are zero.
-// Queries carry the softmax scale times log2(e), so scores come out in log2
-// units.  The bf16 attention kernel reads V from vqkv / tqkv itself, through
-// the geometry's row table (awa_geom::d_vrow).
+// in bf16.  Unused slots are zero.  Queries carry the softmax scale times
+// log2(e), so scores come out in log2 units.  The bf16 attention kernel reads V
+// from vqkv / tqkv itself, through the geometry's row table
+// (awa_geom::d_vrow).  For fp32 storage only K and V are packed, as split fp16
+// tiles in fragment order (f32_kfrag).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -57,6 +57,50 @@ __device__ inline uint32_t bf16x2_rne(float lo, float hi) {
     typedef float f32x2_t __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t));
 }
+
+// x / r, correctly rounded, from rinv = 1 / r (correctly rounded): q = x rinv
+// is within an ulp of x / r, and one correction step with the exact residual
+// fma(-q, r, x) rounds it correctly (Markstein, IBM J. Res. Dev. 34(1), 1990).
+// Three instructions where the IEEE division takes about ten.
+__device__ inline float div_by(float x, float r, float rinv) {
+    const float q = x * rinv;
+    return __builtin_fmaf(__builtin_fmaf(-q, r, x), rinv, q);
+}
+
+// The fp32 path's split operands: x 2^a = hi + lo (two fp16), 2^a =
+// split_scale(largest finite magnitude of the block) bringing that magnitude
+// to [2^14, 2^15).  Infinities take no part in the scale and split into
+// infinity and NaN.
+__device__ inline float finite_abs(float x) {
+    const float v = fabsf(x);
+    return v < __builtin_inff() ? v : 0.f;
+}
+__device__ inline float split_scale(float mx) {
+    // exponents below -100 are held there, so that the scale is finite
+    const int e = max((int)(__float_as_uint(mx) >> 23) - 127, -100);
+    return __uint_as_float((uint32_t)(127 + 14 - e) << 23);
+}
+__device__ inline void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+    typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, f16x2_t));
+    // x - hi in one instruction each (fp32 with an fp16 operand)
+    float ra, rb;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(hi), "v"(b));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){ra, rb}, f16x2_t));
+}
+__device__ inline void split8(const float (&x)[8], uint32_t (&hi)[4], uint32_t (&lo)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) split2(x[2 * i], x[2 * i + 1], hi[i], lo[i]);
+}
+// Fragment order of a packed fp32 tile (32 fragments of 1 KiB, lane l's 16 bytes
+// at 16 l), by 32-key halves of 16 KiB.  K: key block b (16 keys), k32 step s of
+// the channels, hi (0) or lo (1); lane 16 q + r: key 16 b + r, channels
+// 32 s + 8 q .. + 7.  V^T: half ks, channel block db; lane: channel 16 db + r,
+// keys 32 ks + {4 q + e, 16 + 4 q + e}, e = 0 .. 3.
+__host__ __device__ inline constexpr int f32_kfrag(int b, int s, int lo) { return (b * 4 + s) * 2 + lo; }
+__host__ __device__ inline constexpr int f32_vfrag(int ks, int db, int lo) { return (ks * 8 + db) * 2 + lo; }
 
 // Integer restatement of awa_window.cpp:15-78 along one axis.  The reference
 // forms shifted bounds as int((i - 0.5) * wX) in double; for integer i and wX
@@ -112,11 +156,13 @@ struct GeomPlan {
     std::vector<int32_t> tile_win;   // n_vid_tiles, window of each video tile
     std::vector<int32_t> tile_meta;  // n_tiles*2: RoPE-table row of slot 0, valid rows
     std::vector<int32_t> items;      // n_items*4: window, first q tile, second q tile (-1), 0
-    // Work units of the fp32 attention kernel (one workgroup per unit and
-    // head): 2 item + query tile of the item, units of windows with more key
-    // tiles first (workgroups are dispatched in index order, and window sizes
+    // Workgroups of the fp32 attention kernel, 8 values each as in sched_desc
+    // below (first value -1: idle).  Consecutive workgroups go to the 8 XCDs
+    // in turn, so entry b belongs to XCD b % 8: all items of one (window,
+    // head) sit on one XCD, whose L2 holds that window's K and V tiles, and
+    // each XCD's list has the windows with more key tiles first (window sizes
     // can differ several-fold: the longest must start first).
-    std::vector<int32_t> f32_units;
+    std::vector<int32_t> f32_work;
     // Persistent schedule of the bf16 attention kernel: one workgroup per
     // resident slot (two per CU); slot s runs on XCD s % 8 and processes the
     // work items sched_start[s] .. sched_start[s+1]) of sched_desc, longest
@@ -127,6 +173,10 @@ struct GeomPlan {
     std::vector<int32_t> sched_start;  // n_slots+1
     std::vector<int32_t> sched_desc;   // 8 per item, n_items*HEADS items
 };
+// The 8 values of work item i of head h: {head | window << 8, first query tile,
+// second query tile (-1: none), cumf[window]}, {first video tile of the window,
+// its video tile count, its first text tile, its token count}.
+void item_desc(const GeomPlan& P, int h, int i, int32_t d[8]);
 // Host planning (awa_capi.cpp): the tiles and work items of a geometry with
 // nwin, cumf, txt_len and txt_sets set, then the attention kernel's
 // schedule over n_slots workgroups (a multiple of 8 is used).
@@ -201,7 +251,7 @@ struct awa_geom {
     int32_t* d_tile_base = nullptr;
     int32_t* d_tile_win = nullptr;
     int32_t* d_items = nullptr;
-    int32_t* d_f32_units = nullptr;  // GeomPlan::f32_units
+    int32_t* d_f32_work = nullptr;  // GeomPlan::f32_work
     int32_t* d_sched_start = nullptr;
     int32_t* d_sched_desc = nullptr;
     float* d_vfreq = nullptr;
@@ -271,9 +321,11 @@ struct PackArgs {
     const uint32_t* vrow;      // row table
     const float2* vcs;
     const float2* tcs;
-    void* Qp;
+    void* Qp;              // bf16 storage only (the fp32 attention normalises its own queries)
     void* Kp;
     void* Vp;              // fp32 storage only (the bf16 attention reads V from vqkv / tqkv)
+    // fp32 storage: [HEADS][n_tiles][4], of each 16-row block with split_scale 2^a: 2^-a of K, -a of V
+    float *kexp, *vexp;
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles;
     float eps;
     float qscale;          // folded into Q: softmax scale 1/sqrt(128) times log2(e)
@@ -300,8 +352,15 @@ struct SdpaArgs {
     float* tpart;          // [nwin][txt_len][2560] fp32 text partials
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles, n_items, nwin;
     float scale_log2e;     // multiplier of the scores (1 when Q carries the scale)
-    const int32_t* f32_units;  // fp32 kernel: GeomPlan::f32_units
-    int n_f32_units;
+    // fp32 kernel: its workgroups, the packed blocks' factors, and what the
+    // queries' normalisation and rotation need (as in PackArgs)
+    const int32_t* f32_work;
+    int n_f32_work;
+    const float *kexp, *vexp;
+    const int32_t* tile_meta;
+    const float2 *vcs, *tcs;
+    const float *nq_v, *nq_t;
+    float eps, qscale;
 };
 hipError_t launch_sdpa(int dtype, const SdpaArgs& a, hipStream_t s);
 hipError_t launch_sdpa_f32(const SdpaArgs& a, hipStream_t s);   // awa_sdpa_f32.hip

@@ -9,9 +9,10 @@
 // normalises q and k per head (dit_vk.cpp:54-61: r = sqrt(sum x^2 / 128 +
 // eps), y = x / r * g), rotates channel pairs (2i, 2i+1) for i < 63
 // (dit_vk.cpp:62-71; pair 63 of the table is the identity) and writes the
-// packed tiles the SDPA kernel reads: Qp/Kp row-major per tile and, for fp32
-// storage only, Vp transposed per tile (layout in awa_internal.hpp; the bf16
-// attention kernel reads V from vqkv / tqkv itself).  HBM-bound: every byte it
+// packed tiles the SDPA kernel reads: Qp/Kp row-major per tile for bf16, split
+// K and V tiles for fp32 storage (layouts in awa_internal.hpp; the bf16
+// attention kernel reads V, the fp32 one Q from vqkv / tqkv itself).
+// HBM-bound: every byte it
 // needs is read once and every packed byte written once; all loads of a
 // thread are issued before the first use.
 #include "awa_internal.hpp"
@@ -84,19 +85,10 @@ __device__ inline float row_sum16(float v) {
     v = dpp_add(v, 0x141);
     return dpp_add(v, 0x140);
 }
-// x / r, correctly rounded, from rinv = 1 / r (correctly rounded): q = x rinv
-// is within an ulp of x / r, and one correction step with the exact residual
-// fma(-q, r, x) rounds it correctly (Markstein, IBM J. Res. Dev. 34(1), 1990).
-// Three instructions where the IEEE division takes about ten.
-__device__ inline float div_by(float x, float r, float rinv) {
-    const float q = x * rinv;
-    return __builtin_fmaf(__builtin_fmaf(-q, r, x), rinv, q);
-}
-
-// V staging tile in LDS (fp32), [slot][d] with a row pitch of VP = 129
-// 4-byte words, so that the row writes and the transposing column reads below
-// both hit distinct banks.
-constexpr int VP = 129;
+// V staging tile in LDS (fp32), [slot][d] with a row pitch of VP words: four
+// rows apart is 16 banks of 64, so the transposing reads below (16 channels x
+// 4 slots four rows apart) hit distinct banks.
+constexpr int VP = 132;
 
 constexpr int RPT = TILE / 16;  // rows per thread of the bf16 kernel (16 rows per 256-thread pass)
 
@@ -123,24 +115,27 @@ __device__ inline void store_cs(float4* lds_cs, const float4 (&t)[CS_PT], int ti
 }
 
 // fp32 storage: one workgroup per (QR rows of a 64-row tile, head), QR / 16
-// rows per thread (16 threads per row, each an 8-channel chunk).  QR = 64
-// (whole tiles) when the grid fills the device; QR = 16 (four workgroups per
-// tile and head) for small geometries, whose whole-tile grid has fewer
-// workgroups than the device has CUs (220 at 360p).  Correctly rounded
-// arithmetic (IEEE sqrt, division by div_by); V is packed transposed through
-// LDS: the workgroup's QR slots of every channel row of the V^T tile.
+// rows per thread (16 threads per row, each an 8-channel chunk), K and V only
+// (the attention kernel normalises and rotates its queries itself, which saves
+// a read and a write of Q).  QR = 64 (whole tiles) when the grid fills the
+// device; QR = 16 (four workgroups per tile and head) for small geometries,
+// whose whole-tile grid has fewer workgroups than the device has CUs (220 at
+// 360p).  Correctly rounded arithmetic (IEEE sqrt, division by div_by).  Both
+// leave as split fp16 tiles in fragment order (f32_kfrag), each 16-row block
+// scaled by its own power of two (split_scale of its largest finite
+// magnitude), whose inverse or exponent goes to kexp / vexp; V is transposed through LDS.
 // whole-tile workgroups from this many (tile, head) pairs on (measured: quarters
-// faster up to 1,200 pairs (360p 12.0 -> 10.2 us, 720p 31 -> 26), whole tiles
-// from 1,900 (1080p 79 against 86 us))
+// faster up to 1,200 pairs, whole tiles from 1,900)
 constexpr long F32_WHOLE_MIN = 1536;
 template <int QR>
 __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     using IO = Io<float>;
     constexpr int NQ = TILE / QR;                 // workgroups per (tile, head)
-    constexpr int RT = QR / 16;                   // rows per thread
+    constexpr int RT = QR / 16;                   // 16-row blocks of the workgroup: rows per thread
     constexpr int NCS = QR * CS_Q4 / 256;         // table float4 per thread
-    __shared__ uint32_t vs[QR * VP];
+    __shared__ __align__(16) float vs[QR * VP];
     __shared__ float4 lds_cs[QR * CS_Q4];
+    __shared__ float mxs[4][2 * RT];
 
     const int nblk = a.n_tiles * HEADS * NQ;
     const int lid = xcd_remap(nblk);  // a tile's workgroups: neighbouring ids, one XCD
@@ -150,7 +145,7 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     const int h = rem / NQ, qt = rem - (rem / NQ) * NQ;
     const int tid = threadIdx.x;
     const int c = tid & 15;                  // 8-channel chunk of the head row
-    const int rl = tid >> 4;                 // first row of the thread in the workgroup
+    const int rl = tid >> 4;                 // row of the thread in each 16-row block
 
     // Two levels of loads: the tile's record (RoPE-table row of slot 0,
     // valid rows) and the thread's row indices from the row table, then every
@@ -166,11 +161,10 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     const size_t cs_row0 = (size_t)meta.x;  // table row of slot 0
     const float* src = reinterpret_cast<const float*>(is_txt ? a.tqkv : a.vqkv);
     const float4* cst = reinterpret_cast<const float4*>(is_txt ? a.tcs : a.vcs);
-    const float* gq = is_txt ? a.nq_t : a.nq_v;
     const float* gk = is_txt ? a.nk_t : a.nk_v;
     const int col = h * HEAD_D + c * 8;
 
-    // the workgroup's (cos, sin) rows for LDS, then the rows' q, k, v
+    // the workgroup's (cos, sin) rows for LDS, then the rows' k, v
     float4 cst_t[NCS];
 #pragma unroll
     for (int it = 0; it < NCS; it++) {
@@ -184,84 +178,114 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         // and drop padding queries, so padding rows reach no output.
         cst_t[it] = cst[(cs_row0 + min(row, nvalid - 1)) * CS_Q4 + (i % CS_Q4)];
     }
-    IO::Raw rq[RT], rk[RT], rv[RT];
+    IO::Raw rk[RT], rv[RT];
 #pragma unroll
     for (int kk = 0; kk < RT; kk++) {  // padding slots: the window's last row
         const float* row = src + (size_t)ridx[kk] + col;
-        rq[kk] = IO::load(row);
         rk[kk] = IO::load(row + DIM);
         rv[kk] = IO::load(row + 2 * DIM);
     }
-    float gqv[8], gkv[8];
+    float gkv[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        gqv[i] = gq[c * 8 + i];
-        gkv[i] = gk[c * 8 + i];
-    }
+    for (int i = 0; i < 8; i++) gkv[i] = gk[c * 8 + i];
 #pragma unroll
     for (int it = 0; it < NCS; it++) lds_cs[it * 256 + tid] = cst_t[it];
     __syncthreads();
 
-    const size_t tile_off = ((size_t)h * a.n_tiles + tile) * TILE * HEAD_D;
-    float* Qt = reinterpret_cast<float*>(a.Qp) + tile_off;
-    float* Kt = reinterpret_cast<float*>(a.Kp) + tile_off;
-    float* Vt = reinterpret_cast<float*>(a.Vp) + tile_off;
-
+    float k[RT][8];
+    float mx[2 * RT];  // largest magnitudes of the thread's part of K and V blocks
 #pragma unroll
     for (int kk = 0; kk < RT; kk++) {
         const int lr = rl + 16 * kk;       // row in the workgroup
-        const int r = qt * QR + lr;        // slot in the tile
         const float4 cs0 = lds_cs[lr * CS_Q4 + 2 * c], cs1 = lds_cs[lr * CS_Q4 + 2 * c + 1];
-        float q[8], k[8];
-        IO::widen(rq[kk], q);
-        IO::widen(rk[kk], k);
-        float sq = 0.f, sk = 0.f;
+        IO::widen(rk[kk], k[kk]);
+        float sk = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            sq += q[i] * q[i];
-            sk += k[i] * k[i];
-        }
-        sq = row_sum16(sq);
+        for (int i = 0; i < 8; i++) sk += k[kk][i] * k[kk][i];
         sk = row_sum16(sk);
-        const float nq = sqrtf(sq / (float)HEAD_D + a.eps);
         const float nk = sqrtf(sk / (float)HEAD_D + a.eps);
-        const float iq = 1.f / nq, ik = 1.f / nk;
+        const float ik = 1.f / nk;
         const float csv[8] = {cs0.x, cs0.y, cs0.z, cs0.w, cs1.x, cs1.y, cs1.z, cs1.w};
+        mx[2 * kk] = mx[2 * kk + 1] = 0.f;
 #pragma unroll
         for (int p = 0; p < 4; p++) {
             const float cn = csv[2 * p], sn = csv[2 * p + 1];
-            const float q0 = div_by(q[2 * p], nq, iq) * gqv[2 * p];
-            const float q1 = div_by(q[2 * p + 1], nq, iq) * gqv[2 * p + 1];
-            const float k0 = div_by(k[2 * p], nk, ik) * gkv[2 * p];
-            const float k1 = div_by(k[2 * p + 1], nk, ik) * gkv[2 * p + 1];
-            q[2 * p] = (q0 * cn - q1 * sn) * a.qscale;
-            q[2 * p + 1] = (q1 * cn + q0 * sn) * a.qscale;
-            k[2 * p] = k0 * cn - k1 * sn;
-            k[2 * p + 1] = k1 * cn + k0 * sn;
+            const float k0 = div_by(k[kk][2 * p], nk, ik) * gkv[2 * p];
+            const float k1 = div_by(k[kk][2 * p + 1], nk, ik) * gkv[2 * p + 1];
+            k[kk][2 * p] = k0 * cn - k1 * sn;
+            k[kk][2 * p + 1] = k1 * cn + k0 * sn;
         }
-        IO::store8(Qt + (size_t)r * HEAD_D + c * 8, q);
-        IO::store8(Kt + (size_t)r * HEAD_D + c * 8, k);
         float v[8];
         IO::widen(rv[kk], v);
-        uint32_t* vrow = vs + lr * VP;
 #pragma unroll
-        for (int i = 0; i < 8; i++) vrow[c * 8 + i] = __float_as_uint(v[i]);
+        for (int i = 0; i < 8; i++) {
+            mx[2 * kk] = fmaxf(mx[2 * kk], finite_abs(k[kk][i]));
+            mx[2 * kk + 1] = fmaxf(mx[2 * kk + 1], finite_abs(v[i]));
+        }
+        float4* vrow = reinterpret_cast<float4*>(vs + lr * VP + c * 8);
+        vrow[0] = rv[kk].a;
+        vrow[1] = rv[kk].b;
+    }
+    // block maxima: 16 rows, so all four waves
+#pragma unroll
+    for (int i = 0; i < 2 * RT; i++) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], o));
+        if ((tid & 63) == 0) mxs[tid >> 6][i] = mx[i];
     }
     __syncthreads();
-
-    // Transposed V: Vt[d][slot] for the workgroup's QR slots, 4 QR contiguous
-    // bytes per channel row (thread unit: channel d, 4-slot chunk sc).
-    constexpr int NSC = QR / 4;
 #pragma unroll
-    for (int it = 0; it < QR * HEAD_D / 4 / 256; it++) {
-        const int u = it * 256 + tid;
-        const int d = u / NSC, sc = u % NSC;
-        float4 o;
-        o.x = __uint_as_float(vs[(sc * 4 + 0) * VP + d]);
-        o.y = __uint_as_float(vs[(sc * 4 + 1) * VP + d]);
-        o.z = __uint_as_float(vs[(sc * 4 + 2) * VP + d]);
-        o.w = __uint_as_float(vs[(sc * 4 + 3) * VP + d]);
-        *reinterpret_cast<float4*>(Vt + (size_t)d * TILE + qt * QR + sc * 4) = o;
+    for (int i = 0; i < 2 * RT; i++)
+        mx[i] = split_scale(fmaxf(fmaxf(mxs[0][i], mxs[1][i]), fmaxf(mxs[2][i], mxs[3][i])));
+
+    const size_t ht = (size_t)h * a.n_tiles + tile;
+    if (tid < 2 * RT) {
+        const float f = split_scale(fmaxf(fmaxf(mxs[0][tid], mxs[1][tid]), fmaxf(mxs[2][tid], mxs[3][tid])));
+        const size_t b = ht * 4 + qt * RT + (tid >> 1);
+        if (tid & 1) a.vexp[b] = (float)(127 - (int)(__float_as_uint(f) >> 23));
+        else a.kexp[b] = 1.f / f;
+    }
+    unsigned char* Kt = reinterpret_cast<unsigned char*>(a.Kp) + ht * (TILE * HEAD_D * 4);
+    unsigned char* Vt = reinterpret_cast<unsigned char*>(a.Vp) + ht * (TILE * HEAD_D * 4);
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int kk = 0; kk < RT; kk++) {  // lane 16 (c % 4) + rl of fragments (block, step c / 4)
+#pragma unroll
+        for (int i = 0; i < 8; i++) k[kk][i] *= mx[2 * kk];
+        split8(k[kk], hi, lo);
+        unsigned char* d = Kt + f32_kfrag(qt * RT + kk, c >> 2, 0) * 1024 + (16 * (c & 3) + rl) * 16;
+        *reinterpret_cast<uint4*>(d) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *reinterpret_cast<uint4*>(d + 1024) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+    // V^T fragments: a 16-row block is half of a lane's eight keys
+    const int r16 = tid & 15, q = (tid >> 4) & 3;
+    if constexpr (RT == 4) {
+#pragma unroll
+        for (int it = 0; it < 4; it++) {
+            const int u = it * 4 + (tid >> 6), ks = u >> 3, db = u & 7;  // wave-uniform
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[e] = vs[(32 * ks + 16 * (e >> 2) + 4 * q + (e & 3)) * VP + 16 * db + r16] *
+                       (ks ? mx[5 + 2 * (e >> 2)] : mx[1 + 2 * (e >> 2)]);
+            split8(v, hi, lo);
+            unsigned char* d = Vt + f32_vfrag(ks, db, 0) * 1024 + (tid & 63) * 16;
+            *reinterpret_cast<uint4*>(d) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+            *reinterpret_cast<uint4*>(d + 1024) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        }
+    } else {
+        const int db = 2 * (tid >> 6);  // two channel blocks per wave
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            v[e] = vs[(4 * q + (e & 3)) * VP + 16 * (db + (e >> 2)) + r16] * mx[1];
+        split8(v, hi, lo);
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            unsigned char* d = Vt + f32_vfrag(qt >> 1, db + b, 0) * 1024 + (tid & 63) * 16 + 8 * (qt & 1);
+            *reinterpret_cast<uint2*>(d) = make_uint2(hi[2 * b], hi[2 * b + 1]);
+            *reinterpret_cast<uint2*>(d + 1024) = make_uint2(lo[2 * b], lo[2 * b + 1]);
+        }
     }
 }
 

@@ -17,7 +17,7 @@
 // ds_read_b64_tr_b16; the fp32 kernel reads a V^T tile packed per window.
 //
 // bf16 storage -> v_mfma_f32_32x32x16_bf16 (fp32 accumulation); fp32
-// storage -> v_mfma_f32_32x32x2f32 in awa_sdpa_f32.hip (a file of its own:
+// storage -> split fp16 MFMAs in awa_sdpa_f32.hip (a file of its own:
 // this one is compiled with the MFMA accumulators in VGPRs, which the bf16
 // kernel's softmax wants and which made the fp32 kernel spill).
 //

@@ -1,14 +1,32 @@
 // awa_sdpa_f32.hip — varlen window attention with fp32 storage on CDNA4 matrix
-// cores (v_mfma_f32_32x32x2f32).
+// cores (v_mfma_f32_16x16x32_f16 on split operands).
 //
 // The fp32 counterpart of sdpa_bf16_kernel (awa_sdpa.hip), for AWA_F32
-// storage: the reference's fp32 attention (dit_vk.cpp:406-439) at fp32
-// MFMA precision.  One workgroup (4 wave64) per (work item, head): a work
-// item is one window and up to two of its 64-row query tiles, each wave owns
-// 32 queries; the window's K and V^T tiles stream through LDS (double
-// buffered).  Scores are formed transposed, S^T = K Q^T, so that a lane owns
-// one query column and the online softmax needs one cross-lane exchange;
-// the probabilities leave the accumulator in the B-operand layout of
+// storage: the reference's fp32 attention (dit_vk.cpp:406-439).  Every matrix
+// operand x is carried as two fp16 values, hi = fp16(x 2^a) and lo =
+// fp16(x 2^a - hi), which hold 23 of fp32's 24 significand bits (hi's rounding
+// error is a multiple of 2^-24 of it, lo keeps 11 bits of that and a sign), and
+// a product is three MFMAs, lo hi + hi lo + hi hi, accumulated in fp32; the
+// dropped lo lo is 2^-24 of the product.  The fp16 MFMA does 16 times the work of
+// the fp32 one, so three of them still do over five times.  Against 64 bits
+// the result is no further off than a chain of fp32 MFMAs, whose 32 (here 12)
+// roundings of the running sum per score outweigh the operands' last bit
+// (relative error 2.9e-7 against 4.3e-7 on N(0, 1) inputs at 360p, 3.3e-7
+// against 5.0e-7 at 1080p).
+//
+// The powers of two 2^a bring every block of 16 rows (K and V: set by the pack
+// kernel per block and head; Q: per row) to at most 2^15, so fp16's range
+// bounds nothing: an element 2^-17 of its block's largest still has its 23
+// bits, and smaller ones are held to 2^-40 of the largest.  They are undone
+// exactly: in the factor of the scores, in P before its split, and in the
+// normalisation of O.  P = exp2(s - m) is split like the rest.
+//
+// The query rows are normalised and rotated here (each is read by one
+// workgroup), K and V come from the pack kernel as hi and lo tiles in fragment
+// order (f32_kfrag in awa_internal.hpp): the LDS DMA copies it linearly and a
+// wave's fragment read is 1 KiB of consecutive LDS.  Scores are formed
+// transposed, S^T = K Q^T, so that a lane owns one query column; the
+// probabilities leave the accumulator in the B-operand layout of
 // O^T = V^T P^T.  Video query rows are scattered back to token order
 // (dit_vk.cpp:445-455); text query rows go to per-window fp32 partials that
 // the coalesce kernel averages in window order (dit_vk.cpp:440-444).
@@ -18,270 +36,514 @@ namespace awa {
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void* lptr_t;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(4))) f32x2 cfloat2_t;
 
-// The key/query tile sequence of one window: its video tiles, then the text
-// tiles of its text set.
-struct WinTiles {
-    int vbase, nvt, tbase, ntt, f, txt;
+// A work entry (GeomPlan::f32_work): one head, one window and one or two of its
+// query tiles; the window's tiles are its video tiles, then the text tiles of
+// its text set.
+struct Item {
+    int h, w, kq0, kq1, vbase, nvt, tbase, ntt, f, txt;
     __device__ int tile(int kk) const { return kk < nvt ? vbase + kk : tbase + (kk - nvt); }
     __device__ int nvalid(int kk) const {
         return kk < nvt ? min(TILE, f - TILE * kk) : min(TILE, txt - TILE * (kk - nvt));
     }
+    // 32-key units: of the video rows, then of the text rows (a tile's empty
+    // second half is none)
+    __device__ int vid_units() const { return (f + 31) >> 5; }
+    __device__ int units() const { return vid_units() + ((txt + 31) >> 5); }
+    // half tile (2 tile + half) and valid keys of unit u
+    __device__ int unit_half(int u) const {
+        const int nv = vid_units();
+        return u < nv ? 2 * vbase + u : 2 * tbase + (u - nv);
+    }
+    __device__ int unit_valid(int u) const {
+        const int nv = vid_units();
+        return u < nv ? f - 32 * u : txt - 32 * (u - nv);
+    }
 };
 
-__device__ inline WinTiles window_tiles(const SdpaArgs& a, int w) {
-    WinTiles t;
-    t.vbase = a.tile_base[w];
-    t.nvt = a.tile_base[w + 1] - t.vbase;
-    t.ntt = a.ntt;
-    t.tbase = a.n_vid_tiles + (a.txt_sets == 1 ? 0 : w) * a.ntt;
-    t.f = a.cumf[w + 1] - a.cumf[w];
-    t.txt = a.txt_len;
-    return t;
+// Maximum / sum over the four lanes l % 16 + 16 i (a row of the fragment
+// layouts), without LDS.
+__device__ inline float max4(float v) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ inline float sum4(float v) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Hardware dispatches workgroup b to XCD b % 8.  Remap so that each XCD gets
-// a contiguous range of (head, item) ids: consecutive items of one head are
-// mostly the same window and share its K/V tiles through that XCD's L2.
+// P is at most 2^M_STALE (the running maximum stays until a tile's exceeds it by
+// more, so that O is rarely rescaled), times 2^P_SHIFT: below 2^16, and down to
+// 2^-22 in fp16's normal range.  A V block is taken as no smaller than 2^V_FLOOR
+// of the window's largest in P's exponent, which keeps P out of fp32's
+// subnormals (the row sum needs it) and lies far below what fp16 holds of V.
+constexpr float P_SHIFT = 8.f, M_STALE = 7.f, V_FLOOR = -60.f;
 
-// Destination of query slot `slot` of query tile kq (nullptr: padding slot).
-__device__ inline void* query_dst(const SdpaArgs& a, const WinTiles& wt, int w, int h, int kq,
-                                  int slot, size_t elem) {
-    if (slot >= wt.nvalid(kq)) return nullptr;
-    if (kq < wt.nvt) {
-        const int g = a.cumf[w] + TILE * kq + slot;
-        const size_t tok = (size_t)a.vidx[g];
-        return reinterpret_cast<char*>(a.vattn) + (tok * DIM + (size_t)h * HEAD_D) * elem;
-    }
-    const int i = TILE * (kq - wt.nvt) + slot;
-    return a.tpart + ((size_t)w * a.txt_len + i) * DIM + (size_t)h * HEAD_D;
+constexpr uint32_t FU_BYTES = 32 * HEAD_D * 4;  // a K or V unit (32 keys): hi and lo, 16 KiB
+constexpr uint32_t V_RING = 2 * FU_BYTES;       // LDS stage: two K units, then two V units
+constexpr uint32_t STAGE_BYTES = 4 * FU_BYTES;  // 64 KiB
+
+// A wave's quarter of a unit (4 KiB) by LDS DMA, linear: instruction offset j
+// moves the global address and the LDS destination alike.  From asm, with the
+// kernel's own waits (unit_barrier) before any wave reads the unit.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ inline void dma_quarter(const void* unit, uint32_t part, uint32_t lane16, uint32_t m) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(unit), 0, FU_BYTES, 0x00020000);
+    asm volatile(
+        "s_mov_b32 m0, %[m]\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %[v], %[r], %[so] offen lds\n\t"
+        "buffer_load_dwordx4 %[v], %[r], %[so] offen offset:1024 lds\n\t"
+        "buffer_load_dwordx4 %[v], %[r], %[so] offen offset:2048 lds\n\t"
+        "buffer_load_dwordx4 %[v], %[r], %[so] offen offset:3072 lds"
+        :
+        : [v] "v"(lane16), [r] "s"(r), [so] "s"(part), [m] "s"(m + part)
+        : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// This wave's DMA has landed and its LDS reads are done, then the barrier.
+__device__ inline void unit_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Eighteen wait states between MFMAs and the first use of their results, tied to
+// the registers (the compiler places the eight or so that this MFMA needs by
+// itself; next to a unit's MFMAs the rest is nothing).
+template <int N>
+__device__ inline void mfma_fence(f32x4 (&s)[N][1]) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2)
+        asm volatile("s_nop %c2" : "+v"(s[i][0]), "+v"(s[i + 1][0]) : "n"(i ? 0 : 15));
+    asm volatile("s_nop 1");
+}
+template <int N>
+__device__ inline void mfma_fence(f32x4 (&s)[N][2]) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2)
+        asm volatile("s_nop %c4" : "+v"(s[i][0]), "+v"(s[i][1]), "+v"(s[i + 1][0]), "+v"(s[i + 1][1]) : "n"(i ? 0 : 15));
+    asm volatile("s_nop 1");
 }
 
-constexpr int KP32 = 132;                 // LDS pitch of a K row (floats)
-constexpr int VP32 = 68;                  // LDS pitch of a V^T row (floats)
-constexpr int KS32 = TILE * KP32;
-constexpr int STAGE32 = KS32 + HEAD_D * VP32;  // one K and one V^T tile: 68.6 KiB
-
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
-// One workgroup per (64-row query tile, head).  With v_mfma_f32_16x16x4_f32 a
-// wave holds 16 queries' Q (32 floats), O^T (32) and one key tile's scores (16)
-// in few registers, so two waves share each SIMD:
-//   kSplit = false: four waves (wave w owns the tile's queries 16 w .. + 15)
-//     and one LDS tile stage (68.6 KiB): two workgroups per CU;
-//   kSplit = true: eight waves in two halves of four, half 0 taking the
-//     window's key tiles [0, nk0), half 1 the rest (nk0 = ceil(nk / 2)), each
-//     through its own stage: one workgroup per CU, and a long window's key
-//     tiles take half as long; at the end half 1 leaves its row maxima, sums
-//     and O^T in its stage and half 0 merges them.
-// The launch takes the split form for small grids (at most two workgroups per
-// CU, where the longest query tile sets the time), else the other.
+// One workgroup per (two query tiles of a window, head), 128 queries: four
+// waves of 32 (or, for an odd window's last tile, of 16).  64 KiB of LDS and at
+// most 256 registers: two workgroups per CU, two waves per SIMD.  Fewer
+// queries per wave would read the fragments more often than LDS can deliver
+// (32 queries: 85 of 128 bytes per clock at full MFMA rate).
 //
-// Lane l = 16 g + j (j: the lane's query; g: its group of four).
-//   S^T = K Q^T per 16-key block kb and k-step s (32 steps of 4 channels):
-//     A: K[16 kb + j][32 g + s], B: Q[j][32 g + s] (step s pairs channel
-//     32 g + s across the four lane groups: any channel order that A and B
-//     share gives the same dot products), out: lane l holds keys
-//     16 kb + 4 g + r (r = 0..3) of query j.
-//   O^T += V^T P^T per 16-channel block db and key step (kb, r):
-//     A: V^T[16 db + j][16 kb + 4 g + r], B: P[j][16 kb + 4 g + r], which is
-//     exactly score register r of block kb: the probabilities never move.
-//     out: lane l holds channels 16 db + 4 g + r of query j.
-// A query's scores are spread over lanes j, j + 16, j + 32, j + 48: its row
-// maximum and sum take two cross-lane steps.
-template <bool kSplit>
-__global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArgs a) {
-    constexpr int HALVES = kSplit ? 2 : 1;
-    __shared__ __align__(16) float lds[HALVES * STAGE32];
-    // Workgroup b: head b % 20 of query tile GeomPlan::f32_units[b / 20]
-    // (2 item + tile of the item), the tiles of windows with more key tiles
-    // first: workgroups are dispatched in index order, and window sizes can
-    // differ several-fold (the slowest workgroup sets the time).
-    const int lid = (int)blockIdx.x;
-    if (lid >= a.n_f32_units * HEADS) return;
-    const int h = lid % HEADS;
-    const int unit = a.f32_units[lid / HEADS];
-    const int4 it = reinterpret_cast<const int4*>(a.items)[unit >> 1];
-    const int kq = (unit & 1) ? it.z : it.y;
-    const int w = it.x;
-    const WinTiles wt = window_tiles(a, w);
-    const int nk = wt.nvt + wt.ntt;
+// Measured (1080p shifted, 1,304 workgroups of 6-22 units, kernel trace): 323
+// us as fp32 MFMAs, 130 here; 360p 49.5 -> 35 us.  With every window cut to two
+// units it still takes 56 us: the workgroup's ends (its queries' rows from
+// memory, their normalisation and split, the first units' latency, the output
+// rows) are over a third of the time, the units between run at about 60 % of the
+// MFMA rate.  Neither the softmax's instructions (a quarter fewer: 134 -> 128 us)
+// nor HBM (112 MB read, 69 written) sets it.
+//
+// The window's keys run in 32-key units u, each in two phases in which the
+// matrix core and the VALU work side by side:
+//   A(u)  MFMA  S(u+1) = K(u+1) Q^T
+//         VALU  P(u) = exp2(S(u) - m), its row sums and its split
+//   B(u)  MFMA  O^T += V^T(u) P^T(u)
+//         VALU  row maxima of S(u+1)
+// K and V units reach LDS by DMA into rings of two; unit u's barrier makes
+// K(u+1) and V(u) visible and frees the slots of K(u) and V(u-1), which the
+// DMA of K(u+2) and V(u+1) refills under both phases.  Past the last unit
+// phase A forms scores from whatever its slot holds, which nothing uses.
+//   kSplit: eight waves in two halves of four, half 0 taking the window's
+//     units [0, n0), half 1 the rest (n0 = ceil(n / 2)), each through its own
+//     stage: one workgroup per CU, and a long window takes half as long; at the
+//     end half 1 leaves its row maxima, sums and O^T in LDS and half 0 merges
+//     them.  For grids of at most one workgroup per CU, where the longest
+//     window sets the time.
+//
+// Lane l = 16 q + r.  Fragments (A or B operand, 16 rows x 32 k): lane holds
+// row r, k 8 q .. + 7.
+//   S^T block (kb: 16 keys, qb: 16 queries): A = K, B = Q, 4 k32 steps of
+//     channels; out: keys 16 kb + 4 q + t of query r in register t.
+//   O^T block (db: 16 channels, qb): A = V^T, B = P, one k32 step: keys
+//     {4 q + e, 16 + 4 q + e}, e = 0..3, which are exactly the lane's score
+//     registers of the unit's two blocks.
+template <int NQ, bool kSplit>
+__device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char* lds) {
+    const int h = wt.h;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int half = kSplit ? wave >> 2 : 0, w4 = wave & 3;
+    const int r16 = lane & 15, q = lane >> 4;
+    const int nu = wt.units();
+    const int n0 = kSplit ? (nu + 1) >> 1 : nu;  // iterations: half 0 has n0 units, half 1 nu - n0
+    const int ubeg = half ? n0 : 0, uend = half ? nu : n0;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int half = kSplit ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0;
-    const int htid = tid & 255;  // thread index within the half
-    const int j = lane & 15, g = lane >> 4;
-    const int qslot = 16 * (wave & 3) + j;
-    float* stage = lds + half * STAGE32;
-    const int nk0 = kSplit ? (nk + 1) >> 1 : nk;  // iterations: half 0 has nk0 tiles, half 1 nk - nk0
-    const int kbeg = half ? nk0 : 0, kend = half ? nk : nk0;
+    const uint32_t ldsb = (uint32_t)(uintptr_t)(lptr_t)lds + half * STAGE_BYTES;
+    const unsigned char* stage = lds + half * STAGE_BYTES;
+    const unsigned char* Kh = reinterpret_cast<const unsigned char*>(a.Kp) + (size_t)h * a.n_tiles * (2 * FU_BYTES);
+    const unsigned char* Vh = reinterpret_cast<const unsigned char*>(a.Vp) + (size_t)h * a.n_tiles * (2 * FU_BYTES);
+    // 2^-a (K) and -a (V) of each 16-row block; read through the scalar cache
+    // (constant address space): a vector load's wait would also wait for the
+    // units' DMA
+    const cfloat2_t* ke = (const cfloat2_t*)(a.kexp) + (size_t)h * a.n_tiles * 2;
+    const cfloat2_t* ve2 = (const cfloat2_t*)(a.vexp) + (size_t)h * a.n_tiles * 2;
+    const float* ve = a.vexp + (size_t)h * a.n_tiles * 4;
+    // unit u into a ring slot (0, 1: this half's even and odd units)
+    auto fetch_k = [&](int u, int slot) __attribute__((always_inline)) {
+        if (u < uend)
+            dma_quarter(Kh + (size_t)wt.unit_half(u) * FU_BYTES, 4096u * w4, 16u * lane, ldsb + slot * FU_BYTES);
+    };
+    auto fetch_v = [&](int u, int slot) __attribute__((always_inline)) {
+        if (u < uend)
+            dma_quarter(Vh + (size_t)wt.unit_half(u) * FU_BYTES, 4096u * w4, 16u * lane,
+                        ldsb + V_RING + slot * FU_BYTES);
+    };
+    fetch_k(ubeg, 0);
+    fetch_k(ubeg + 1, 1);
+    fetch_v(ubeg, 0);
 
-    const size_t head_off = (size_t)h * a.n_tiles * TILE * HEAD_D;
-    const float* Qh = reinterpret_cast<const float*>(a.Qp) + head_off;
-    const float* Kh = reinterpret_cast<const float*>(a.Kp) + head_off;
-    const float* Vh = reinterpret_cast<const float*>(a.Vp) + head_off;
-
-    // B operand of S^T: Q[qslot][32 g + s], s = 0..31
-    float qf[32];
-    {
-        const float* qrow = Qh + ((size_t)wt.tile(kq) * TILE + qslot) * HEAD_D + 32 * g;
+    // ---- this wave's queries: 16-row blocks NQ w4 + qb of the item, every load
+    // issued before the first use
+    // element offsets of the queries' rows in vqkv / tqkv
+    uint32_t row_ofs[NQ];
+    float4 xr[NQ][8], cs[NQ][8];
+    int2 meta[NQ];
 #pragma unroll
-        for (int s = 0; s < 32; s += 4) {
-            const f32x4v v = *reinterpret_cast<const f32x4v*>(qrow + s);
-            qf[s] = v[0]; qf[s + 1] = v[1]; qf[s + 2] = v[2]; qf[s + 3] = v[3];
-        }
+    for (int qb = 0; qb < NQ; qb++) {
+        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
+        const int row_tile = kq >= wt.nvt ? a.n_vid_tiles + (kq - wt.nvt) : wt.vbase + kq;
+        row_ofs[qb] = a.vrow[(size_t)row_tile * TILE + vrow_pos(slot)];
+        meta[qb] = reinterpret_cast<const int2*>(a.tile_meta)[wt.tile(kq)];
     }
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
+        const bool txt = kq >= wt.nvt;
+        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + row_ofs[qb] + h * HEAD_D + 8 * q;
+        const float4* cst = reinterpret_cast<const float4*>(txt ? a.tcs : a.vcs) +
+                            ((size_t)meta[qb].x + min(slot, meta[qb].y - 1)) * (CS_STRIDE / 2) + 2 * q;
+#pragma unroll
+        for (int i = 0; i < 8; i++) xr[qb][i] = *reinterpret_cast<const float4*>(row + 32 * (i >> 1) + 4 * (i & 1));
+#pragma unroll
+        for (int i = 0; i < 8; i++) cs[qb][i] = cst[8 * (i >> 1) + (i & 1)];
+    }
+    // the largest V exponent of the window: P V is accumulated in its units
+    float vmax = -1000.f;
+    for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) vmax = fmaxf(vmax, ve[4 * wt.tile(i >> 2) + (i & 3)]);
 
-    // The half's next tile's K and V^T travel through registers (eight
-    // 16-byte pieces of each per thread) while its current tile is computed.
-    f32x4v rk[8], rv[8];
-    auto load_tile = [&](int kk) __attribute__((always_inline)) {
-        const size_t t = (size_t)wt.tile(kk) * TILE * HEAD_D;
-        const f32x4v* ks = reinterpret_cast<const f32x4v*>(Kh + t);
-        const f32x4v* vs = reinterpret_cast<const f32x4v*>(Vh + t);
+    f16x8 qh[NQ][4], ql[NQ][4];
+    float cq[NQ];
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        float x[32];
+        float ss = 0.f;
+        const float* gain = ((NQ * w4 + qb < 4 ? wt.kq0 : wt.kq1) >= wt.nvt ? a.nq_t : a.nq_v) + 8 * q;
+        float gr[32];
+#pragma unroll
+        for (int i = 0; i < 32; i++) gr[i] = gain[32 * (i >> 3) + (i & 7)];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            rk[i] = ks[htid + 256 * i];
-            rv[i] = vs[htid + 256 * i];
+            x[4 * i] = xr[qb][i].x; x[4 * i + 1] = xr[qb][i].y; x[4 * i + 2] = xr[qb][i].z; x[4 * i + 3] = xr[qb][i].w;
         }
-    };
-    auto store_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 32; i++) ss += x[i] * x[i];
+        ss = sum4(ss);
+        // x / n g, rotated, times the softmax scale
+        const float in = a.qscale / sqrtf(ss / (float)HEAD_D + a.eps);
+        float mx = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int c = htid + 256 * i;
-            *reinterpret_cast<f32x4v*>(stage + (c >> 5) * KP32 + (c & 31) * 4) = rk[i];      // K row c / 32
-            *reinterpret_cast<f32x4v*>(stage + KS32 + (c >> 4) * VP32 + (c & 15) * 4) = rv[i];  // V^T row c / 16
+            const float c4[4] = {cs[qb][i].x, cs[qb][i].y, cs[qb][i].z, cs[qb][i].w};
+#pragma unroll
+            for (int p = 0; p < 4; p += 2) {
+                const float x0 = x[4 * i + p] * in * gr[4 * i + p], x1 = x[4 * i + p + 1] * in * gr[4 * i + p + 1];
+                x[4 * i + p] = x0 * c4[p] - x1 * c4[p + 1];
+                x[4 * i + p + 1] = x1 * c4[p] + x0 * c4[p + 1];
+                mx = fmaxf(mx, fmaxf(fabsf(x[4 * i + p]), fabsf(x[4 * i + p + 1])));
+            }
+        }
+        const float f = split_scale(finite_abs(max4(mx)));
+        cq[qb] = 1.f / f;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            float y[8];
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = x[8 * st + i] * f;
+            split8(y, hi, lo);
+            qh[qb][st] = __builtin_bit_cast(f16x8, hi);
+            ql[qb][st] = __builtin_bit_cast(f16x8, lo);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one block's gains at a time: registers
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
+
+    f32x4 oacc[8][NQ];
+    float m_i[NQ], l_i[NQ];
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        m_i[qb] = -INFINITY;
+        l_i[qb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < 8; db++) oacc[db][qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+
+    f32x4 s[2][2][NQ];  // scores of an even and an odd unit: two 16-key blocks
+    f16x8 fr[2][4];     // fragments, read a step ahead of their MFMAs
+    const f16x8* frag = reinterpret_cast<const f16x8*>(stage) + lane;
+    // step st of the K unit in a slot: its two key blocks, hi and lo
+    auto read_k = [&](int slot, int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) fr[st & 1][e] = frag[slot * (FU_BYTES / 16) + 64 * f32_kfrag(e >> 1, st, e & 1)];
+    };
+    // step j of the V unit in a slot: channel blocks 2 j, 2 j + 1, hi and lo
+    auto read_v = [&](int slot, int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            fr[j & 1][e] = frag[(V_RING + slot * FU_BYTES) / 16 + 64 * f32_vfrag(0, 2 * j + (e >> 1), e & 1)];
+    };
+    // the MFMAs of step st of S += K Q^T, the small products first
+    auto score_step = [&](f32x4 (&sn)[2][NQ], int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int pr = 0; pr < 3; pr++)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int qb = 0; qb < NQ; qb++)
+                    sn[e][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        fr[st & 1][2 * e + (pr == 0)], pr == 1 ? ql[qb][st] : qh[qb][st],
+                        st == 0 && pr == 0 ? (f32x4){0.f, 0.f, 0.f, 0.f} : sn[e][qb], 0, 0, 0);
+    };
+    auto mask = [&](f32x4 (&sn)[2][NQ], int u) __attribute__((always_inline)) {
+        const int kv = wt.unit_valid(u);
+        if (kv < 32) {
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (16 * kb + 4 * q + r >= kv)
+#pragma unroll
+                        for (int qb = 0; qb < NQ; qb++) sn[kb][qb][r] = -INFINITY;
         }
     };
-
-    f32x4v oacc[8];
+    // row maximum of query block qb in a unit whose K blocks have factors kc
+    auto row_max = [&](const f32x4 (&sn)[2][NQ], int qb, f32x2 kc) __attribute__((always_inline)) {
+        float mx = -INFINITY;
 #pragma unroll
-    for (int db = 0; db < 8; db++) oacc[db] = (f32x4v){0.f, 0.f, 0.f, 0.f};
-    float m_i = -INFINITY, l_i = 0.f;
-
-    if (kbeg < kend) {
-        load_tile(kbeg);
-        store_tile();
-    }
-    __syncthreads();
-    for (int i = 0; i < nk0; i++) {  // the same iteration count in both halves
-        const int kk = kbeg + i;
-        const bool have = kk < kend, have_next = kk + 1 < kend;  // uniform per half
-        if (have_next) load_tile(kk + 1);
-        if (have) {
-            // ---- scores of the tile: four 16-key blocks
-            f32x4v sacc[4];
+        for (int kb = 0; kb < 2; kb++)
+            mx = fmaxf(mx, cq[qb] * kc[kb] * fmaxf(fmaxf(sn[kb][qb][0], sn[kb][qb][1]), fmaxf(sn[kb][qb][2], sn[kb][qb][3])));
+        return max4(mx);
+    };
+    // the running maximum stays until a unit's exceeds it by M_STALE
+    auto raise = [&](const float (&mloc)[NQ]) __attribute__((always_inline)) {
+        bool up = false;
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++) {
-                sacc[kb] = (f32x4v){0.f, 0.f, 0.f, 0.f};
-                const float* krow = stage + (16 * kb + j) * KP32 + 32 * g;
+        for (int qb = 0; qb < NQ; qb++) up |= mloc[qb] > m_i[qb] + M_STALE;
+        if (!__any(up)) return;
+        mfma_fence(oacc);
 #pragma unroll
-                for (int s = 0; s < 32; s += 4) {
-                    const f32x4v kv = *reinterpret_cast<const f32x4v*>(krow + s);
+        for (int qb = 0; qb < NQ; qb++) {
+            const float m_new = fmaxf(m_i[qb], mloc[qb]);
+            const float alpha = __builtin_amdgcn_exp2f(m_i[qb] - m_new);
+            l_i[qb] *= alpha;
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        sacc[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qf[s + e], sacc[kb], 0, 0, 0);
-                }
-            }
-            // ---- online softmax (scale folded into Q; keys past the tile's
-            // valid count get -inf)
-            const int kvalid = wt.nvalid(kk);
-            float mloc = -INFINITY;
-#pragma unroll
-            for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int key = 16 * kb + 4 * g + r;
-                    const float v = key < kvalid ? sacc[kb][r] * a.scale_log2e : -INFINITY;
-                    sacc[kb][r] = v;
-                    mloc = fmaxf(mloc, v);
-                }
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
-            const float m_new = fmaxf(m_i, mloc);  // finite: every tile has a valid key
-            const float alpha = __builtin_amdgcn_exp2f(m_i - m_new);
-            float psum = 0.f;
-#pragma unroll
-            for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float p = __builtin_amdgcn_exp2f(sacc[kb][r] - m_new);
-                    sacc[kb][r] = p;
-                    psum += p;
-                }
-            l_i = l_i * alpha + psum;  // this lane's keys; summed over the group at the end
-            m_i = m_new;
-#pragma unroll
-            for (int db = 0; db < 8; db++) oacc[db] *= alpha;
-            // ---- O^T += V^T P^T
-#pragma unroll
-            for (int db = 0; db < 8; db++) {
-                const float* vrow = stage + KS32 + (16 * db + j) * VP32 + 4 * g;
-#pragma unroll
-                for (int kb = 0; kb < 4; kb++) {
-                    const f32x4v vv = *reinterpret_cast<const f32x4v*>(vrow + 16 * kb);
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        oacc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r], sacc[kb][r], oacc[db], 0, 0, 0);
-                }
-            }
+            for (int db = 0; db < 8; db++) oacc[db][qb] *= alpha;
+            m_i[qb] = m_new;
         }
-        if (i + 1 < nk0) {
-            __syncthreads();  // every wave is done with its half's tile
-            if (have_next) store_tile();
-            __syncthreads();
+    };
+    f32x2 kc = {0.f, 0.f};  // K factors of the unit whose scores are pending
+    // one unit, its V in slot sl and the next one's K in slot sl ^ 1: scores
+    // s[sl] to P and O, the next unit's to s[sl ^ 1]
+    auto unit = [&](int u, int sl) __attribute__((always_inline)) {
+        f32x4 (&sc)[2][NQ] = s[sl];
+        f32x4 (&sn)[2][NQ] = s[sl ^ 1];
+        const int un = min(u + 1, uend - 1);  // past the end: any unit's factors
+        const f32x2 kcn = ke[wt.unit_half(un)];
+        // P leaves as exp2(s - m + vs): vs puts the block's V scale and
+        // P_SHIFT into the exponent, vi takes them back out of the row sum
+        f32x2 vs = ve2[wt.unit_half(u)], vi;
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+            vs[kb] = fmaxf(vs[kb] - vmax, V_FLOOR) + P_SHIFT;
+            vi[kb] = __builtin_amdgcn_exp2f(-vs[kb]);  // exact: whole exponents
         }
+        uint32_t hi[NQ][4], lo[NQ][4];
+        // ---- phase A
+        read_k(sl ^ 1, 0);
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            if (st < 3) read_k(sl ^ 1, st + 1);
+            else read_v(sl, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            score_step(sn, st);
+            // NQ of the unit's 2 NQ (query block, key block) pairs per two steps
+            if (NQ == 2 || (st & 1)) {
+                const int qb = NQ == 2 ? st >> 1 : 0, kb = NQ == 2 ? st & 1 : st >> 1;
+                const float c = cq[qb] * kc[kb], b = vs[kb] - m_i[qb];
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][qb][r], c, b));
+                // this lane's keys; summed over the row at the end
+                l_i[qb] = __builtin_fmaf((p[0] + p[1]) + (p[2] + p[3]), vi[kb], l_i[qb]);
+                split2(p[0], p[1], hi[qb][2 * kb], lo[qb][2 * kb]);
+                split2(p[2], p[3], hi[qb][2 * kb + 1], lo[qb][2 * kb + 1]);
+            }
+#pragma unroll
+            for (int g = 0; g < 6 * NQ; g++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);  // and some of the VALU work
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        mfma_fence(sn);
+        mask(sn, un);
+        f16x8 ph[NQ], pl[NQ];
+#pragma unroll
+        for (int qb = 0; qb < NQ; qb++) {
+            ph[qb] = __builtin_bit_cast(f16x8, hi[qb]);
+            pl[qb] = __builtin_bit_cast(f16x8, lo[qb]);
+        }
+        // ---- phase B
+        float mloc[NQ];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j < 3) read_v(sl, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int pr = 0; pr < 3; pr++)
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int qb = 0; qb < NQ; qb++)
+                        oacc[2 * j + e][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            fr[j & 1][2 * e + (pr == 0)], pr == 1 ? pl[qb] : ph[qb], oacc[2 * j + e][qb], 0, 0, 0);
+            if (j >= 1 && j <= NQ) mloc[j - 1] = row_max(sn, j - 1, kcn);
+#pragma unroll
+            for (int g = 0; g < 6 * NQ; g++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        kc = kcn;
+        if (u + 1 < uend) raise(mloc);
+    };
+
+    unit_barrier();
+    if (ubeg < uend) {  // the first unit's scores
+        kc = ke[wt.unit_half(ubeg)];
+        read_k(0, 0);
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            if (st < 3) read_k(0, st + 1);
+            score_step(s[0], st);
+        }
+        mfma_fence(s[0]);
+        mask(s[0], ubeg);
+        float mloc[NQ];
+#pragma unroll
+        for (int qb = 0; qb < NQ; qb++) mloc[qb] = row_max(s[0], qb, kc);
+        raise(mloc);
     }
-    float l = l_i + __shfl_xor(l_i, 16);
-    l += __shfl_xor(l, 32);
+    for (int i = 0; i < n0; i += 2)  // the same iteration count in both halves
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int u = ubeg + i + e;
+            unit_barrier();
+            fetch_k(u + 2, e);
+            fetch_v(u + 1, e ^ 1);
+            if (u < uend) unit(u, e);  // uniform per half
+        }
+    // the lane through an opaque copy: the addresses below are formed here and
+    // not held in registers across the loop
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    mfma_fence(oacc);
+    float l[NQ];
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) l[qb] = sum4(l_i[qb]);
     if constexpr (kSplit) {
         // merge: half 1 leaves its running maximum (-inf when it had no
         // tile), sum and O^T in its stage, half 0 rescales both to the common
-        // maximum
+        // maximum.  Rows of 16 NQ registers side by side per lane: 16-byte
+        // pieces of consecutive lanes.
         __syncthreads();
-        float* pub = lds + STAGE32;
+        f32x4* pub = reinterpret_cast<f32x4*>(lds + STAGE_BYTES) + (size_t)w4 * (8 * NQ * 64) + ln;
+        float* pml = reinterpret_cast<float*>(lds) + (size_t)w4 * (2 * NQ * 64) + ln;  // half 0's stage is free
         if (half == 1) {
 #pragma unroll
-            for (int db = 0; db < 8; db++)
-                *reinterpret_cast<f32x4v*>(pub + qslot * HEAD_D + 16 * db + 4 * g) = oacc[db];
-            if (g == 0) {
-                pub[TILE * HEAD_D + qslot] = m_i;
-                pub[TILE * HEAD_D + TILE + qslot] = l;
+            for (int qb = 0; qb < NQ; qb++) {
+#pragma unroll
+                for (int db = 0; db < 8; db++) pub[64 * (8 * qb + db)] = oacc[db][qb];
+                pml[64 * (2 * qb)] = m_i[qb];
+                pml[64 * (2 * qb + 1)] = l[qb];
             }
         }
         __syncthreads();
         if (half == 1) return;
-        const float m1 = pub[TILE * HEAD_D + qslot], l1 = pub[TILE * HEAD_D + TILE + qslot];
-        const float m = fmaxf(m_i, m1);
-        const float a0 = __builtin_amdgcn_exp2f(m_i - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
-        l = l * a0 + l1 * a1;
 #pragma unroll
-        for (int db = 0; db < 8; db++)
-            oacc[db] = oacc[db] * a0 + *reinterpret_cast<const f32x4v*>(pub + qslot * HEAD_D + 16 * db + 4 * g) * a1;
+        for (int qb = 0; qb < NQ; qb++) {
+            const float m1 = pml[64 * (2 * qb)], l1 = pml[64 * (2 * qb + 1)];
+            const float m = fmaxf(m_i[qb], m1);
+            const float a0 = __builtin_amdgcn_exp2f(m_i[qb] - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
+            l[qb] = l[qb] * a0 + l1 * a1;
+#pragma unroll
+            for (int db = 0; db < 8; db++) oacc[db][qb] = oacc[db][qb] * a0 + pub[64 * (8 * qb + db)] * a1;
+        }
     }
-    const float inv = 1.f / l;
-    float* dst = reinterpret_cast<float*>(query_dst(a, wt, w, h, kq, qslot, 4));
-    if (dst == nullptr) return;
+    // ---- O / l through LDS (each wave its own 16 rows of 512 bytes, 16-byte
+    // chunk c of row r at c ^ r), so that whole rows are stored (from the
+    // accumulator layout a store writes 64 bytes of 16 rows)
+    if constexpr (!kSplit) __syncthreads();  // every wave is done with the K and V units
+    f32x4* stg = reinterpret_cast<f32x4*>(lds + (kSplit ? 16384 : 0)) + w4 * (16 * 32);
+    const float c = __builtin_amdgcn_exp2f(vmax - P_SHIFT);
 #pragma unroll
-    for (int db = 0; db < 8; db++)
-        *reinterpret_cast<float4*>(dst + 16 * db + 4 * g) =
-            make_float4(oacc[db][0] * inv, oacc[db][1] * inv, oacc[db][2] * inv, oacc[db][3] * inv);
+    for (int qb = 0; qb < NQ; qb++) {
+        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1;
+        // 1 / l and the V scale; the factors separately, so that neither overflows
+        const float inv = 1.f / l[qb];
+#pragma unroll
+        for (int db = 0; db < 8; db++) stg[(ln & 15) * 32 + ((4 * db + (ln >> 4)) ^ (ln & 15))] = oacc[db][qb] * inv * c;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int row = 2 * i + (ln >> 5), ch = ln & 31, slot = 16 * (blk & 3) + row;
+            const f32x4 v = stg[row * 32 + (ch ^ row)];
+            const uint32_t ofs = __shfl(row_ofs[qb], row);
+            if (slot >= wt.nvalid(kq)) continue;  // padding
+            // video: the token's row of vattn (a row is a third of its qkv row)
+            float* dst = kq < wt.nvt ? reinterpret_cast<float*>(a.vattn) + ofs / 3
+                                     : a.tpart + ((size_t)wt.w * a.txt_len + TILE * (kq - wt.nvt) + slot) * DIM;
+            *reinterpret_cast<f32x4*>(dst + h * HEAD_D + 4 * ch) = v;
+        }
+    }
+}
+
+// Workgroup b: entry b of GeomPlan::f32_work.
+template <bool kSplit>
+__global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArgs a) {
+    __shared__ __align__(16) unsigned char lds[(kSplit ? 2 : 1) * STAGE_BYTES];
+    const int4 d0 = reinterpret_cast<const int4*>(a.f32_work)[2 * blockIdx.x];
+    const int4 d1 = reinterpret_cast<const int4*>(a.f32_work)[2 * blockIdx.x + 1];
+    if (d0.x < 0) return;  // an idle entry
+    Item it;
+    it.h = d0.x & 255; it.w = d0.x >> 8; it.kq0 = d0.y; it.kq1 = d0.z;
+    it.vbase = d1.x; it.nvt = d1.y; it.tbase = d1.z; it.f = d1.w;
+    it.ntt = a.ntt; it.txt = a.txt_len;
+    if (it.kq1 >= 0) run_item<2, kSplit>(a, it, lds);
+    else run_item<1, kSplit>(a, it, lds);
 }
 
 }  // namespace
 
 hipError_t launch_sdpa_f32(const SdpaArgs& a, hipStream_t s) {
-    const int nblk = a.n_f32_units * HEADS;
-    if (nblk == 0) return hipSuccess;
-    // n_slots: two per CU (the persistent bf16 schedule's slot count); the
-    // split form at most two workgroups per CU (measured: 360p 63 -> 53 us,
-    // while 720p and larger grids are faster with two 4-wave workgroups per CU)
-    if (nblk <= a.n_slots)
-        hipLaunchKernelGGL(sdpa_f32_kernel<true>, dim3(nblk), dim3(512), 0, s, a);
+    if (a.n_f32_work == 0) return hipSuccess;
+    // n_slots: two per CU (the persistent bf16 schedule's slot count)
+    if (a.n_f32_work <= a.n_slots / 2)
+        hipLaunchKernelGGL(sdpa_f32_kernel<true>, dim3(a.n_f32_work), dim3(512), 0, s, a);
     else
-        hipLaunchKernelGGL(sdpa_f32_kernel<false>, dim3(nblk), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(sdpa_f32_kernel<false>, dim3(a.n_f32_work), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -1,0 +1,80 @@
+"""GPU tests of the fp32 op's split operands (csrc/awa_sdpa_f32.hip) where its
+units, blocks and scales have edges.
+
+Keys run in 32-row units, queries in 16-row blocks of one or two 64-row tiles,
+and grids of at most one workgroup per CU split a window's units over two
+halves.  Reference: the C oracle in fp32.  Bar 5e-6 (2-norm): both sides carry a
+few 2^-24 of the scores' magnitude (up to about 16 in log2 units) into the
+exponent, so each is about 1e-6 off, and the bar leaves a factor of two over
+their sum.  Scaling V by a power of two scales every block's factor alike, so
+the output scales exactly, bit for bit.
+"""
+import numpy as np
+import pytest
+
+from conftest import seeded_awa_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def run(ctx, geom, vqkv, tqkv, gains):
+    import torch
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    va, ta = ctx.forward(geom, dev(vqkv), dev(tqkv), *[dev(g) for g in gains], eps=1e-5)
+    torch.cuda.synchronize()
+    return va.cpu().numpy(), ta.cpu().numpy()
+
+
+def rel(a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+# one window of h x w rows: 1 unit, a full unit, one row into the next, whole and
+# odd tiles; two windows per axis and enough of them for the unsplit form
+@pytest.mark.parametrize("h,w,nw,txt", [(1, 1, (1, 1, 1), 1), (1, 31, (1, 1, 1), 32), (4, 8, (1, 1, 1), 33),
+                                        (3, 11, (1, 1, 1), 64), (8, 16, (1, 1, 1), 65), (13, 5, (1, 1, 1), 31),
+                                        (10, 29, (1, 2, 2), 58), (30, 41, (1, 4, 4), 77)])
+@pytest.mark.parametrize("shifted", [0, 1])
+def test_f32_edges(oracle, ctx, h, w, nw, txt, shifted):
+    geom = ctx.build_geometry(1, h, w, nw, txt, shifted)
+    og = oracle.Geometry(1, h, w, nw, txt, shifted)
+    vqkv, tqkv, gains = seeded_awa_inputs(h * w, txt, 100 * h + w)
+    ref = oracle.awa_forward(vqkv, tqkv, og, *gains, eps=1e-5)
+    for a, b in zip(run(ctx, geom, vqkv, tqkv, gains), ref):
+        assert rel(a, b) <= 5e-6
+    geom.close()
+
+
+@pytest.mark.parametrize("k", [-90, -20, 20, 90])
+def test_v_scales_exactly(ctx, k):
+    """Far outside fp16's range, V's scale only moves the blocks' exponents."""
+    geom = ctx.build_geometry(1, 10, 29, (1, 2, 2), 58, 1)
+    vqkv, tqkv, gains = seeded_awa_inputs(290, 58, 5)
+    base = run(ctx, geom, vqkv, tqkv, gains)
+    for x in (vqkv, tqkv):
+        x[:, 5120:] *= np.float32(2.0 ** k)
+    for a, b in zip(run(ctx, geom, vqkv, tqkv, gains), base):
+        assert np.array_equal(a, b * np.float32(2.0 ** k))
+    geom.close()
+
+
+def test_mixed_scales(oracle, ctx):
+    """Row blocks of V 2^24 apart, single values 2^12 above their block, all-zero
+    rows of q, k and v, and gains far from 1."""
+    h, w, txt = 9, 23, 40
+    geom = ctx.build_geometry(1, h, w, (1, 1, 1), txt, 0)
+    og = oracle.Geometry(1, h, w, (1, 1, 1), txt, 0)
+    vqkv, tqkv, gains = seeded_awa_inputs(h * w, txt, 9)
+    vqkv[40:60, 5120:] *= 2.0 ** 24
+    vqkv[100, 5120::128] *= 2.0 ** 12
+    vqkv[7] = 0
+    tqkv[3] = 0
+    # q and k gains of video and text together: scores keep their size (with one
+    # of them alone text queries' scores reach 2^15, where the reference overflows)
+    for i, e in enumerate((-15, 15, -15, 15)):
+        gains[i] *= 2.0 ** e
+    ref = oracle.awa_forward(vqkv, tqkv, og, *gains, eps=1e-5)
+    for a, b in zip(run(ctx, geom, vqkv, tqkv, gains), ref):
+        assert np.isfinite(a).all() and rel(a, b) <= 5e-6
+    geom.close()
