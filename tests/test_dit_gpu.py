@@ -427,3 +427,23 @@ def test_model_directory_errors(ctx, awa, tmp_path):
                                     None, None, None, C.byref(h))
     assert rc != 0 and h.value is None
     assert "null stream" in awa.lib().awa_last_error(ctx.ptr).decode()
+
+
+# shapes that fall to each tile form of the GEMM (256 x 256 and 256 x 224, 256 x 128,
+# 128 x 256, 128 x 128, 128 x 64), with row counts at and around their edges
+@pytest.mark.parametrize("N,K", [(2560, 2560), (7680, 2560), (13824, 2560), (2560, 6912), (256, 64)])
+def test_gemm_tile_forms_agree(ctx, N, K):
+    """Every tile form sums an output's products in the same order (K steps of 32 in
+    sequence), so a row's results do not depend on how many rows are computed with
+    it: all bits agree with the largest call's, whose rows are checked against an
+    fp32 product (bf16 output rounding, 2^-8)."""
+    import torch
+    note(f"gemm tile forms N={N} K={K}")
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    A = torch.randn((5498, K), generator=g, device="cuda").bfloat16()
+    W = (0.05 * torch.randn((N, K), generator=g, device="cuda")).bfloat16()
+    full = ctx.gemm(A, W)
+    ref = torch.mm(A[-300:].float(), W.float().t().contiguous())
+    assert float((full[-300:].float() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    for M in (1, 63, 64, 65, 128, 257, 679, 897, 1418, 2778, 3100):
+        assert torch.equal(ctx.gemm(A[:M].contiguous(), W), full[:M]), M
