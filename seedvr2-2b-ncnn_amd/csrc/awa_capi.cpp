@@ -99,14 +99,6 @@ void free_geom_buffers(awa_geom* g) {
 
 namespace awa {
 
-void item_desc(const GeomPlan& P, int h, int i, int32_t d[8]) {
-    const int w = P.items[4 * i];
-    const int32_t v[8] = {h | (w << 8), P.items[4 * i + 1], P.items[4 * i + 2], P.cumf[w],
-                          P.tile_base[w], P.tile_base[w + 1] - P.tile_base[w],
-                          P.n_vid_tiles + (P.txt_sets == 1 ? 0 : w) * P.ntt, P.cumf[w + 1] - P.cumf[w]};
-    std::copy(v, v + 8, d);
-}
-
 // 64-row tiles of every window plus the text tiles, and the work items of the
 // attention kernel (one window, two query tiles).
 void plan_tiles(GeomPlan& P) {
@@ -145,30 +137,6 @@ void plan_tiles(GeomPlan& P) {
         }
     }
     P.n_items = (int)P.items.size() / 4;
-    // fp32 workgroups: (window, head) groups longest first onto the least
-    // loaded XCD, each XCD's list longest window first
-    constexpr int XCDS = 8;
-    auto nkey = [&](int w) { return P.tile_base[w + 1] - P.tile_base[w] + P.ntt; };
-    std::vector<int> first(P.nwin + 1, 0);
-    for (int i = 0; i < P.n_items; i++) first[P.items[4 * i] + 1] = i + 1;
-    for (int w = 0; w < P.nwin; w++) first[w + 1] = std::max(first[w + 1], first[w]);
-    std::vector<int> order(P.nwin);
-    for (int w = 0; w < P.nwin; w++) order[w] = w;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return nkey(x) > nkey(y); });
-    std::vector<std::vector<std::pair<int, int>>> list(XCDS);  // (head, item)
-    long load[XCDS] = {};
-    for (int w : order)
-        for (int h = 0; h < HEADS; h++) {
-            const int x = (int)(std::min_element(load, load + XCDS) - load);
-            load[x] += (long)nkey(w) * (first[w + 1] - first[w]);
-            for (int i = first[w]; i < first[w + 1]; i++) list[x].push_back({h, i});
-        }
-    size_t len = 0;
-    for (const auto& l : list) len = std::max(len, l.size());
-    P.f32_work.assign(len * XCDS * 8, -1);
-    for (int x = 0; x < XCDS; x++)
-        for (size_t k = 0; k < list[x].size(); k++)
-            item_desc(P, list[x][k].first, list[x][k].second, &P.f32_work[(k * XCDS + x) * 8]);
 }
 
 // Static schedule of the persistent bf16 attention
@@ -206,17 +174,21 @@ void plan_schedule(GeomPlan& P, int n_slots) {
     auto cost = [&](int id) { return (long)win_cost[P.items[4 * (id % P.n_items)]]; };
     for (int x = 0; x < XCDS; x++) {
         auto& wl = xwork[x];
-        std::stable_sort(wl.begin(), wl.end(), [&](int a, int b) { return cost(a) > cost(b); });
+        std::vector<std::pair<long, int>> by_cost;
+        for (int id : wl) by_cost.push_back({cost(id), id});
+        std::stable_sort(by_cost.begin(), by_cost.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
+        for (size_t k = 0; k < wl.size(); k++) wl[k] = by_cost[k].second;
         // longest first onto the least loaded slot
         std::vector<std::vector<int>> best(per_xcd);
         std::vector<long> sload(per_xcd, 0);
         long total = 0, cmax = 0;
         for (int id : wl) {
             const int k = (int)(std::min_element(sload.begin(), sload.end()) - sload.begin());
-            sload[k] += cost(id);
+            const long c = cost(id);
+            sload[k] += c;
             best[k].push_back(id);
-            total += cost(id);
-            cmax = std::max(cmax, cost(id));
+            total += c;
+            cmax = std::max(cmax, c);
         }
         // first fit decreasing under the smallest capacity it packs, when
         // that beats the longest-first makespan (items come in a few sizes,
@@ -226,10 +198,11 @@ void plan_schedule(GeomPlan& P, int n_slots) {
             std::vector<long> ld(per_xcd, 0);
             if (out) out->assign(per_xcd, {});
             for (int id : wl) {
+                const long c = cost(id);
                 int k = 0;
-                while (k < per_xcd && ld[k] + cost(id) > cap) k++;
+                while (k < per_xcd && ld[k] + c > cap) k++;
                 if (k == per_xcd) return false;
-                ld[k] += cost(id);
+                ld[k] += c;
                 if (out) (*out)[k].push_back(id);
             }
             return true;
@@ -275,16 +248,40 @@ void plan_schedule(GeomPlan& P, int n_slots) {
     }
     P.sched_start.assign(n_slots + 1, 0);
     P.sched_desc.clear();
+    std::vector<int32_t> desc_of((size_t)HEADS * P.n_items);
     int n = 0;
     for (int sl = 0; sl < n_slots; sl++) {
         for (int id : slot_work[sl]) {
-            int32_t d[8];
-            item_desc(P, id / P.n_items, id % P.n_items, d);
+            const int h = id / P.n_items, i = id % P.n_items, w = P.items[4 * i];
+            const int32_t d[8] = {h | (w << 8), P.items[4 * i + 1], P.items[4 * i + 2], P.cumf[w],
+                                  P.tile_base[w], P.tile_base[w + 1] - P.tile_base[w],
+                                  P.n_vid_tiles + (P.txt_sets == 1 ? 0 : w) * P.ntt,
+                                  P.cumf[w + 1] - P.cumf[w]};
             P.sched_desc.insert(P.sched_desc.end(), d, d + 8);
+            desc_of[id] = n;
             n++;
         }
         P.sched_start[sl + 1] = n;
     }
+
+    // fp32 workgroups: (window, head) groups onto the XCDs as above, each XCD's
+    // list longest window first
+    std::vector<int> order(P.nwin);
+    for (int w = 0; w < P.nwin; w++) order[w] = w;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return win_cost[x] > win_cost[y]; });
+    std::vector<int32_t> list[XCDS];
+    std::fill(xload.begin(), xload.end(), 0);
+    for (int w : order)
+        for (int h = 0; h < HEADS; h++) {
+            const int x = (int)(std::min_element(xload.begin(), xload.end()) - xload.begin());
+            xload[x] += (long)win_cost[w] * (long)items_of[w].size();
+            for (int i : items_of[w]) list[x].push_back(desc_of[h * P.n_items + i]);
+        }
+    size_t len = 0;
+    for (const auto& l : list) len = std::max(len, l.size());
+    P.f32_work.assign(len * XCDS, -1);
+    for (int x = 0; x < XCDS; x++)
+        for (size_t k = 0; k < list[x].size(); k++) P.f32_work[k * XCDS + x] = list[x][k];
 }
 
 }  // namespace awa
@@ -468,7 +465,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.tpart = reinterpret_cast<float*>(base + off_t);
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;
     sa.n_tiles = P.n_tiles; sa.n_items = P.n_items; sa.nwin = P.nwin;
-    sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size() / 8;
+    sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size();
     sa.kexp = pa.kexp; sa.vexp = pa.vexp;
     sa.tile_meta = g->d_tile_meta; sa.vcs = g->d_vcs; sa.tcs = g->d_tcs; sa.nq_v = d_nq_v; sa.nq_t = d_nq_t;
     sa.eps = eps; sa.qscale = pa.qscale;

@@ -156,8 +156,8 @@ struct GeomPlan {
     std::vector<int32_t> tile_win;   // n_vid_tiles, window of each video tile
     std::vector<int32_t> tile_meta;  // n_tiles*2: RoPE-table row of slot 0, valid rows
     std::vector<int32_t> items;      // n_items*4: window, first q tile, second q tile (-1), 0
-    // Workgroups of the fp32 attention kernel, 8 values each as in sched_desc
-    // below (first value -1: idle).  Consecutive workgroups go to the 8 XCDs
+    // Workgroups of the fp32 attention kernel: the number of a work item in
+    // sched_desc below (-1: idle).  Consecutive workgroups go to the 8 XCDs
     // in turn, so entry b belongs to XCD b % 8: all items of one (window,
     // head) sit on one XCD, whose L2 holds that window's K and V tiles, and
     // each XCD's list has the windows with more key tiles first (window sizes
@@ -173,13 +173,10 @@ struct GeomPlan {
     std::vector<int32_t> sched_start;  // n_slots+1
     std::vector<int32_t> sched_desc;   // 8 per item, n_items*HEADS items
 };
-// The 8 values of work item i of head h: {head | window << 8, first query tile,
-// second query tile (-1: none), cumf[window]}, {first video tile of the window,
-// its video tile count, its first text tile, its token count}.
-void item_desc(const GeomPlan& P, int h, int i, int32_t d[8]);
 // Host planning (awa_capi.cpp): the tiles and work items of a geometry with
 // nwin, cumf, txt_len and txt_sets set, then the attention kernel's
-// schedule over n_slots workgroups (a multiple of 8 is used).
+// schedule over n_slots workgroups (a multiple of 8 is used) and the fp32
+// kernel's list.
 void plan_tiles(GeomPlan& P);
 void plan_schedule(GeomPlan& P, int n_slots);
 // Row table (awa_geom::d_vrow): per row tile (the video tiles, then ntt

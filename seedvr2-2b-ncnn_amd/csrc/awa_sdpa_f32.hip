@@ -42,7 +42,7 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(4))) f32x2 cfloat2_t;
 
-// A work entry (GeomPlan::f32_work): one head, one window and one or two of its
+// A work item (GeomPlan::sched_desc): one head, one window and one or two of its
 // query tiles; the window's tiles are its video tiles, then the text tiles of
 // its text set.
 struct Item {
@@ -524,9 +524,10 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
 template <bool kSplit>
 __global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArgs a) {
     __shared__ __align__(16) unsigned char lds[(kSplit ? 2 : 1) * STAGE_BYTES];
-    const int4 d0 = reinterpret_cast<const int4*>(a.f32_work)[2 * blockIdx.x];
-    const int4 d1 = reinterpret_cast<const int4*>(a.f32_work)[2 * blockIdx.x + 1];
-    if (d0.x < 0) return;  // an idle entry
+    const int e = a.f32_work[blockIdx.x];
+    if (e < 0) return;  // an idle entry
+    const int4 d0 = reinterpret_cast<const int4*>(a.sched_desc)[2 * e];
+    const int4 d1 = reinterpret_cast<const int4*>(a.sched_desc)[2 * e + 1];
     Item it;
     it.h = d0.x & 255; it.w = d0.x >> 8; it.kq0 = d0.y; it.kq1 = d0.z;
     it.vbase = d1.x; it.nvt = d1.y; it.tbase = d1.z; it.f = d1.w;
