@@ -486,8 +486,9 @@ struct Tile {
     // us: a 64-deep K step with every CU busy, and a tile's ends
     float step, ends;
 };
-constexpr Tile TILES[] = {{8, 8, 2, 1.475f, 8.f}, {8, 7, 2, 1.375f, 8.f}, {8, 4, 3, 0.88f, 6.f},
-                          {4, 8, 3, 0.86f, 5.5f}, {4, 4, 4, 0.47f, 5.f},  {4, 2, 3, 0.30f, 4.f}};
+constexpr Tile TILES[] = {{8, 8, 2, 1.475f, 8.f}, {8, 7, 2, 1.375f, 8.f}, {8, 5, 3, 1.06f, 7.f},
+                          {8, 4, 3, 0.88f, 6.f},  {4, 8, 3, 0.86f, 5.5f}, {4, 6, 4, 0.60f, 5.5f},
+                          {4, 4, 4, 0.47f, 5.f},  {4, 2, 3, 0.30f, 4.f}};
 
 long tile_count(const GemmBatch& b, const Tile& t) {
     long n = 0;
@@ -499,7 +500,7 @@ long tile_count(const GemmBatch& b, const Tile& t) {
 // Estimated time of the batch with tiles t: rounds of one tile per CU, the last
 // one at 0.7 of a full round plus 0.3 of its share of tiles (its tiles start as
 // CUs fall free and run on a less loaded chip).  Within 15 % of the measured
-// times from 258 to 5498 rows, and it picks the fastest form or one within 7 % of
+// times from 258 to 5498 rows, and it picks the fastest form or one within 8 % of
 // it on all of them.
 float tile_cost(const GemmBatch& b, const Tile& t, int cus) {
     const float r = (float)tile_count(b, t) / cus;
@@ -536,8 +537,10 @@ hipError_t launch_gemm(int epi, GemmBatch& b, hipStream_t s) {
 #define GEMM_LAUNCH(E)    \
     GEMM_TILE(E, 8, 8, 2) \
     GEMM_TILE(E, 8, 7, 2) \
+    GEMM_TILE(E, 8, 5, 3) \
     GEMM_TILE(E, 8, 4, 3) \
     GEMM_TILE(E, 4, 8, 3) \
+    GEMM_TILE(E, 4, 6, 4) \
     GEMM_TILE(E, 4, 4, 4) \
     GEMM_TILE(E, 4, 2, 3) \
     return hipErrorInvalidValue;
