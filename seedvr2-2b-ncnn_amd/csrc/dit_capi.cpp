@@ -174,13 +174,9 @@ int dit_time_embedding(awa_ctx* ctx, float t, const float* d_w_in, const float* 
     DeviceGuard dg(ctx->device);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (!ctx->small) HIPCK(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->small), 8192 * sizeof(float)));
-    float* e0 = ctx->small;          // [256]
-    float* e1 = e0 + 256;            // [2560]
-    float* e2 = e1 + DIM;            // [2560]
-    HIPCK(ctx, launch_sinusoid(t, e0, 256, s));
-    HIPCK(ctx, launch_gemv_f32(d_w_in, d_b_in, e0, e1, 256, DIM, 1, s));
-    HIPCK(ctx, launch_gemv_f32(d_w_hid, d_b_hid, e1, e2, DIM, DIM, 1, s));
-    HIPCK(ctx, launch_gemv_f32(d_w_out, d_b_out, e2, d_emb, DIM, DIT_EMB, 0, s));
+    const float* w[3] = {d_w_in, d_w_hid, d_w_out};
+    const float* b[3] = {d_b_in, d_b_hid, d_b_out};
+    HIPCK(ctx, launch_time_mlp(t, w, b, ctx->small, ctx->small + DIM, d_emb, s));
     return AWA_OK;
 }
 

@@ -7,7 +7,8 @@
 //   ada        AdaCompose (ada_compose.cpp:165-235): emb[6d + K_MAP[k]] +
 //              branch vector, the 12 modulation vectors of a layer.
 //   pack_mlp   interleave proj_in / proj_in_gate rows for the fused SwiGLU.
-//   gemv_f32   the timestep MLP (M = 1 linears, dit_vk.cpp:303-309).
+//   time_in, gemv_f32   the timestep embedding and its MLP (M = 1 linears,
+//              dit_vk.cpp:295-309).
 #include <cmath>
 
 #include "dit_internal.hpp"
@@ -86,32 +87,59 @@ __global__ __launch_bounds__(256) void pack_mlp_kernel(const uint16_t* __restric
     for (int c = threadIdx.x; c < DIM / 8; c += 256) d4[c] = s4[c];
 }
 
-__global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ W,
-                                                       const float* __restrict__ b,
-                                                       const float* __restrict__ x,
-                                                       float* __restrict__ y, int in, int out,
-                                                       int silu) {
-    const int o = blockIdx.x * 4 + (threadIdx.x >> 6);
+// y = act(W x + b): R output rows per wave, x and the rows in 16-byte pieces per
+// lane, every load issued before the first use.  Bound by the weights (26 and
+// 157 MB): with one value per load and lane and a row per wave 20.6 and 50 us.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // weights are only known to hold floats
+template <int IN, int R>
+__device__ inline void gemv_rows(const float* __restrict__ W, const float* __restrict__ b, const float* __restrict__ x,
+                                 float* __restrict__ y, int out, int silu) {
+    constexpr int P = IN / 256;  // pieces per lane and row
+    const int o0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
     const int lane = threadIdx.x & 63;
-    if (o >= out) return;
-    const float* w = W + (size_t)o * in;
-    float acc = 0.f;
-    for (int i = lane; i < in; i += 64) acc += w[i] * x[i];
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        float v = acc + (b ? b[o] : 0.f);
-        if (silu) v = v / (1.f + expf(-v));
-        y[o] = v;
+    if (o0 >= out) return;
+    f32x4u w[R][P], xv[P];
+#pragma unroll
+    for (int r = 0; r < R; r++) {  // rows past the end repeat the last one
+        const float* row = W + (size_t)min(o0 + r, out - 1) * IN;
+#pragma unroll
+        for (int i = 0; i < P; i++) w[r][i] = *reinterpret_cast<const f32x4u*>(row + 4 * (i * 64 + lane));
     }
+#pragma unroll
+    for (int i = 0; i < P; i++) xv[i] = *reinterpret_cast<const f32x4u*>(x + 4 * (i * 64 + lane));
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < P; i++)
+            acc += w[r][i][0] * xv[i][0] + w[r][i][1] * xv[i][1] + w[r][i][2] * xv[i][2] + w[r][i][3] * xv[i][3];
+        acc = wave_sum(acc);
+        if (lane == 0 && o0 + r < out) {
+            float v = acc + b[o0 + r];
+            if (silu) v = v / (1.f + expf(-v));
+            y[o0 + r] = v;
+        }
+    }
+}
+
+template <int IN, int R>
+__global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ W, const float* __restrict__ b,
+                                                       const float* __restrict__ x, float* __restrict__ y, int out,
+                                                       int silu) {
+    gemv_rows<IN, R>(W, b, x, y, out, silu);
 }
 
 struct Sinusoid {
     float v[256];
 };
 
-__global__ void sinusoid_kernel(Sinusoid s, float* e, int dim) {
-    const int j = threadIdx.x;
-    if (j < dim) e[j] = s.v[j];
+// the first linear, its input in the kernel arguments
+__global__ __launch_bounds__(256) void time_in_kernel(Sinusoid s, const float* __restrict__ W,
+                                                      const float* __restrict__ b, float* __restrict__ y, int out) {
+    __shared__ float x[256];
+    x[threadIdx.x] = s.v[threadIdx.x];
+    __syncthreads();
+    gemv_rows<256, 1>(W, b, x, y, out, 1);
 }
 
 }  // namespace
@@ -133,24 +161,20 @@ hipError_t launch_pack_mlp(const uint16_t* w_in, const uint16_t* w_gate, int mlp
     return hipGetLastError();
 }
 
-hipError_t launch_gemv_f32(const float* W, const float* b, const float* x, float* y, int in, int out,
-                           int silu, hipStream_t s) {
-    hipLaunchKernelGGL(gemv_f32_kernel, dim3((out + 3) / 4), dim3(256), 0, s, W, b, x, y, in, out, silu);
-    return hipGetLastError();
-}
-
-hipError_t launch_sinusoid(float t, float* e, int dim, hipStream_t s) {
+hipError_t launch_time_mlp(float t, const float* const w[3], const float* const b[3], float* e1, float* e2, float* emb,
+                           hipStream_t s) {
     // The 256 sinusoid values are formed on the host with the reference's
     // expression (dit_vk.cpp:295-302) and passed by value.
     Sinusoid v{};
-    const int half = dim / 2;
-    for (int j = 0; j < dim && j < 256; j++) {
+    constexpr int half = 128;
+    for (int j = 0; j < 2 * half; j++) {
         // float argument, double exp, rounded to float: as C's exp()
-        const float freq = (j < half) ? (float)::exp((double)(-logf(10000.f) * j / half))
-                                      : (float)::exp((double)(-logf(10000.f) * (j - half) / half));
+        const float freq = (float)::exp((double)(-logf(10000.f) * (j % half) / half));
         v.v[j] = (j < half) ? sinf(t * freq) : cosf(t * freq);
     }
-    hipLaunchKernelGGL(sinusoid_kernel, dim3(1), dim3(256), 0, s, v, e, dim);
+    hipLaunchKernelGGL(time_in_kernel, dim3(DIM / 4), dim3(256), 0, s, v, w[0], b[0], e1, DIM);
+    hipLaunchKernelGGL((gemv_f32_kernel<DIM, 1>), dim3(DIM / 4), dim3(256), 0, s, w[1], b[1], e1, e2, DIM, 1);
+    hipLaunchKernelGGL((gemv_f32_kernel<DIM, 2>), dim3(DIT_EMB / 8), dim3(256), 0, s, w[2], b[2], e2, emb, DIT_EMB, 0);
     return hipGetLastError();
 }
 

@@ -57,10 +57,11 @@ hipError_t launch_ada(const AdaArgs& a, hipStream_t s);
 hipError_t launch_pack_mlp(const uint16_t* w_in, const uint16_t* w_gate, int mlp, uint16_t* w_cat,
                            hipStream_t s);
 
-// y[out] = act(W[out][in] x[in] + b[out]) in fp32; act: 0 none, 1 SiLU.
-hipError_t launch_gemv_f32(const float* W, const float* b, const float* x, float* y, int in, int out,
-                           int silu, hipStream_t s);
-hipError_t launch_sinusoid(float t, float* e, int dim, hipStream_t s);
+// The timestep embedding emb[DIT_EMB] of t: sinusoid [256], then three linears
+// in fp32 ([2560][256], [2560][2560], [DIT_EMB][2560]) with SiLU after the first
+// two; e1 and e2 hold 2560 values each.
+hipError_t launch_time_mlp(float t, const float* const w[3], const float* const b[3], float* e1, float* e2, float* emb,
+                           hipStream_t s);
 
 // The model's ends (dit_ends.hip).  x [Lv + TXT][2560] from the latent grid
 // (T, H, 2 W2, 33) and the text features [TXT][5120].
