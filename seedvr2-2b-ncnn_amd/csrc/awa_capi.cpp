@@ -247,6 +247,7 @@ void plan_schedule(GeomPlan& P, int n_slots) {
             for (int id : best[k]) slot_work[x + XCDS * k].push_back(id);
     }
     P.sched_start.assign(n_slots + 1, 0);
+    P.n_used_slots = 0;
     P.sched_desc.clear();
     std::vector<int32_t> desc_of((size_t)HEADS * P.n_items);
     int n = 0;
@@ -262,26 +263,39 @@ void plan_schedule(GeomPlan& P, int n_slots) {
             n++;
         }
         P.sched_start[sl + 1] = n;
+        if (!slot_work[sl].empty()) P.n_used_slots = sl + 1;
     }
+    P.n_used_slots = (P.n_used_slots + XCDS - 1) / XCDS * XCDS;
 
     // fp32 workgroups: (window, head) groups onto the XCDs as above, each XCD's
     // list longest window first
     std::vector<int> order(P.nwin);
     for (int w = 0; w < P.nwin; w++) order[w] = w;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return win_cost[x] > win_cost[y]; });
-    std::vector<int32_t> list[XCDS];
-    std::fill(xload.begin(), xload.end(), 0);
-    for (int w : order)
-        for (int h = 0; h < HEADS; h++) {
-            const int x = (int)(std::min_element(xload.begin(), xload.end()) - xload.begin());
-            xload[x] += (long)win_cost[w] * (long)items_of[w].size();
-            for (int i : items_of[w]) list[x].push_back(desc_of[h * P.n_items + i]);
-        }
-    size_t len = 0;
-    for (const auto& l : list) len = std::max(len, l.size());
-    P.f32_work.assign(len * XCDS, -1);
-    for (int x = 0; x < XCDS; x++)
-        for (size_t k = 0; k < list[x].size(); k++) P.f32_work[k * XCDS + x] = list[x][k];
+    // (an entry per query tile when those still fit one workgroup per CU: with
+    // 240 rows two query tiles each left 80 workgroups for 256 CUs)
+    for (bool pairs : {false, true}) {
+        std::vector<int32_t> list[XCDS];
+        std::fill(xload.begin(), xload.end(), 0);
+        for (int w : order)
+            for (int h = 0; h < HEADS; h++) {
+                const int x = (int)(std::min_element(xload.begin(), xload.end()) - xload.begin());
+                xload[x] += (long)win_cost[w] * (long)items_of[w].size();
+                for (int i : items_of[w]) {
+                    const int32_t d = desc_of[h * P.n_items + i];
+                    const bool two = P.items[4 * i + 2] >= 0;
+                    if (pairs || !two) list[x].push_back(4 * d);
+                    else for (int t = 1; t <= 2; t++) list[x].push_back(4 * d + t);
+                }
+            }
+        size_t len = 0;
+        for (const auto& l : list) len = std::max(len, l.size());
+        if (!pairs && len * XCDS * 2 > (size_t)n_slots) continue;  // two slots per CU
+        P.f32_work.assign(len * XCDS, -1);
+        for (int x = 0; x < XCDS; x++)
+            for (size_t k = 0; k < list[x].size(); k++) P.f32_work[k * XCDS + x] = list[x][k];
+        break;
+    }
 }
 
 }  // namespace awa
@@ -460,7 +474,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.vsrc_bytes = (uint32_t)std::min<size_t>((size_t)Lv * QKV * es, 0xffffffffu);
     sa.tsrc_bytes = (uint32_t)std::min<size_t>((size_t)P.txt_len * QKV * es, 0xffffffffu);
     sa.items = g->d_items; sa.cumf = g->d_cumf; sa.vidx = g->d_vidx; sa.tile_base = g->d_tile_base;
-    sa.sched_start = g->d_sched_start; sa.sched_desc = g->d_sched_desc; sa.n_slots = P.n_slots;
+    sa.sched_start = g->d_sched_start; sa.sched_desc = g->d_sched_desc; sa.n_slots = P.n_slots; sa.n_used_slots = P.n_used_slots;
     sa.vattn = d_vattn; sa.vattn_bytes = (uint32_t)((size_t)Lv * DIM * es);
     sa.tpart = reinterpret_cast<float*>(base + off_t);
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;

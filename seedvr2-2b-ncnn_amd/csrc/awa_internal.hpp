@@ -156,8 +156,9 @@ struct GeomPlan {
     std::vector<int32_t> tile_win;   // n_vid_tiles, window of each video tile
     std::vector<int32_t> tile_meta;  // n_tiles*2: RoPE-table row of slot 0, valid rows
     std::vector<int32_t> items;      // n_items*4: window, first q tile, second q tile (-1), 0
-    // Workgroups of the fp32 attention kernel: the number of a work item in
-    // sched_desc below (-1: idle).  Consecutive workgroups go to the 8 XCDs
+    // Workgroups of the fp32 attention kernel: 4 x the number of a work item in
+    // sched_desc below, plus 1 or 2 for its first or second query tile alone
+    // (-1: idle).  Consecutive workgroups go to the 8 XCDs
     // in turn, so entry b belongs to XCD b % 8: all items of one (window,
     // head) sit on one XCD, whose L2 holds that window's K and V tiles, and
     // each XCD's list has the windows with more key tiles first (window sizes
@@ -170,6 +171,7 @@ struct GeomPlan {
     // second query tile (-1: none), cumf[window]}, {first video tile of the
     // window, its video tile count, its first text tile, its token count}.
     int n_slots = 0;
+    int n_used_slots = 0;  // slots past it have no items and need no workgroup (a multiple of 8)
     std::vector<int32_t> sched_start;  // n_slots+1
     std::vector<int32_t> sched_desc;   // 8 per item, n_items*HEADS items
 };
@@ -343,7 +345,7 @@ struct SdpaArgs {
     const int32_t* tile_base;
     const int32_t* sched_start;  // bf16 kernel: persistent schedule (GeomPlan)
     const int32_t* sched_desc;
-    int n_slots;
+    int n_slots, n_used_slots;
     void* vattn;
     uint32_t vattn_bytes;  // bf16 kernel: size of vattn (buffer stores drop beyond it)
     float* tpart;          // [nwin][txt_len][2560] fp32 text partials

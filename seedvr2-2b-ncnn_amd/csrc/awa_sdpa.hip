@@ -904,7 +904,8 @@ void sdpa_bf16_kernel(SdpaArgs a) {
 
 hipError_t launch_sdpa(int dtype, const SdpaArgs& a, hipStream_t s) {
     if (dtype != AWA_BF16) return launch_sdpa_f32(a, s);
-    hipLaunchKernelGGL(sdpa_bf16_kernel, dim3(a.n_slots), dim3(128), 0, s, a);
+    if (a.n_used_slots == 0) return hipSuccess;
+    hipLaunchKernelGGL(sdpa_bf16_kernel, dim3(a.n_used_slots), dim3(128), 0, s, a);
     return hipGetLastError();
 }
 

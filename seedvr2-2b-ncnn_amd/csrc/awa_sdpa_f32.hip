@@ -526,10 +526,11 @@ __global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArg
     __shared__ __align__(16) unsigned char lds[(kSplit ? 2 : 1) * STAGE_BYTES];
     const int e = a.f32_work[blockIdx.x];
     if (e < 0) return;  // an idle entry
-    const int4 d0 = reinterpret_cast<const int4*>(a.sched_desc)[2 * e];
-    const int4 d1 = reinterpret_cast<const int4*>(a.sched_desc)[2 * e + 1];
+    const int4 d0 = reinterpret_cast<const int4*>(a.sched_desc)[2 * (e >> 2)];
+    const int4 d1 = reinterpret_cast<const int4*>(a.sched_desc)[2 * (e >> 2) + 1];
+    const int part = e & 3;  // 0: the item's one or two query tiles, 1, 2: one of its two
     Item it;
-    it.h = d0.x & 255; it.w = d0.x >> 8; it.kq0 = d0.y; it.kq1 = d0.z;
+    it.h = d0.x & 255; it.w = d0.x >> 8; it.kq0 = part == 2 ? d0.z : d0.y; it.kq1 = part ? -1 : d0.z;
     it.vbase = d1.x; it.nvt = d1.y; it.tbase = d1.z; it.f = d1.w;
     it.ntt = a.ntt; it.txt = a.txt_len;
     if (it.kq1 >= 0) run_item<2, kSplit>(a, it, lds);
