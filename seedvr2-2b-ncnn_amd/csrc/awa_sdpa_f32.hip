@@ -11,7 +11,7 @@
 // the fp32 one, so three of them still do over five times.  Against 64 bits
 // the result is no further off than a chain of fp32 MFMAs, whose 32 (here 12)
 // roundings of the running sum per score outweigh the operands' last bit
-// (relative error 2.9e-7 against 4.3e-7 on N(0, 1) inputs at 360p, 3.3e-7
+// (relative error 3.2e-7 against 4.3e-7 on N(0, 1) inputs at 360p, 3.6e-7
 // against 5.0e-7 at 1080p).
 //
 // The powers of two 2^a bring every block of 16 rows (K and V: set by the pack
