@@ -7,7 +7,7 @@
 // fp16(x 2^a - hi), which hold 23 of fp32's 24 significand bits (hi's rounding
 // error is a multiple of 2^-24 of it, lo keeps 11 bits of that and a sign), and
 // a product is three MFMAs, lo hi + hi lo + hi hi, accumulated in fp32; the
-// dropped lo lo is 2^-24 of the product.  The fp16 MFMA does 16 times the work of
+// dropped lo lo is at most 2^-22 of the product.  The fp16 MFMA does 16 times the work of
 // the fp32 one, so three of them still do over five times.  Against 64 bits
 // the result is no further off than a chain of fp32 MFMAs, whose 32 (here 12)
 // roundings of the running sum per score outweigh the operands' last bit
