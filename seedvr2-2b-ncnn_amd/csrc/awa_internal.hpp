@@ -69,15 +69,19 @@ __device__ inline float div_by(float x, float r, float rinv) {
 
 // The fp32 path's split operands: x 2^a = hi + lo (two fp16), 2^a =
 // split_scale(largest finite magnitude of the block) bringing that magnitude
-// to [2^14, 2^15).  Infinities take no part in the scale and split into
-// infinity and NaN.
+// to [2^14, 2^15), or less where it is below 2^floor.  Infinities take no part
+// in the scale and split into infinity and NaN.
 __device__ inline float finite_abs(float x) {
     const float v = fabsf(x);
     return v < __builtin_inff() ? v : 0.f;
 }
-__device__ inline float split_scale(float mx) {
-    // exponents below -100 are held there, so that the scale is finite
-    const int e = max((int)(__float_as_uint(mx) >> 23) - 127, -100);
+// V: the scale stays finite.  Q and K: so does the product of two of them, and
+// its inverse, which the scores are multiplied by, stays a normal number (0
+// times a masked score's -infinity is NaN); what a block below 2^-45 loses is
+// under 2^-84.
+constexpr int SPLIT_FLOOR_V = -100, SPLIT_FLOOR_QK = -45;
+__device__ inline float split_scale(float mx, int floor) {
+    const int e = max((int)(__float_as_uint(mx) >> 23) - 127, floor);
     return __uint_as_float((uint32_t)(127 + 14 - e) << 23);
 }
 __device__ inline void split2(float a, float b, uint32_t& hi, uint32_t& lo) {

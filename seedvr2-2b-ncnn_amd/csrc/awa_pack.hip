@@ -236,11 +236,13 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 2 * RT; i++)
-        mx[i] = split_scale(fmaxf(fmaxf(mxs[0][i], mxs[1][i]), fmaxf(mxs[2][i], mxs[3][i])));
+        mx[i] = split_scale(fmaxf(fmaxf(mxs[0][i], mxs[1][i]), fmaxf(mxs[2][i], mxs[3][i])),
+                            i & 1 ? SPLIT_FLOOR_V : SPLIT_FLOOR_QK);
 
     const size_t ht = (size_t)h * a.n_tiles + tile;
     if (tid < 2 * RT) {
-        const float f = split_scale(fmaxf(fmaxf(mxs[0][tid], mxs[1][tid]), fmaxf(mxs[2][tid], mxs[3][tid])));
+        const float f = split_scale(fmaxf(fmaxf(mxs[0][tid], mxs[1][tid]), fmaxf(mxs[2][tid], mxs[3][tid])),
+                                    tid & 1 ? SPLIT_FLOOR_V : SPLIT_FLOOR_QK);
         const size_t b = ht * 4 + qt * RT + (tid >> 1);
         if (tid & 1) a.vexp[b] = (float)(127 - (int)(__float_as_uint(f) >> 23));
         else a.kexp[b] = 1.f / f;

@@ -263,7 +263,7 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
                 mx = fmaxf(mx, fmaxf(fabsf(x[4 * i + p]), fabsf(x[4 * i + p + 1])));
             }
         }
-        const float f = split_scale(finite_abs(max4(mx)));
+        const float f = split_scale(finite_abs(max4(mx)), SPLIT_FLOOR_QK);
         cq[qb] = 1.f / f;
 #pragma unroll
         for (int st = 0; st < 4; st++) {

@@ -78,3 +78,37 @@ def test_mixed_scales(oracle, ctx):
     for a, b in zip(run(ctx, geom, vqkv, tqkv, gains), ref):
         assert np.isfinite(a).all() and rel(a, b) <= 5e-6
     geom.close()
+
+
+# one window (two halves of its units) and sixteen (the unsplit form); 40 and 77
+# text rows leave a partly filled unit
+SPLIT, UNSPLIT = (9, 23, (1, 1, 1), 40), (30, 41, (1, 4, 4), 77)
+
+
+def both(oracle, ctx, shape, change, seed=11):
+    """The op and the oracle on seeded inputs after change(vqkv, tqkv, gains)."""
+    h, w, nw, txt = shape
+    geom = ctx.build_geometry(1, h, w, nw, txt, 0)
+    og = oracle.Geometry(1, h, w, nw, txt, 0)
+    vqkv, tqkv, gains = seeded_awa_inputs(h * w, txt, seed)
+    change(vqkv, tqkv, gains)
+    got = run(ctx, geom, vqkv, tqkv, gains)
+    geom.close()
+    return got, oracle.awa_forward(vqkv, tqkv, og, *gains, eps=1e-5)
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+@pytest.mark.parametrize("zero", ["text_qk", "text", "video_qk", "video", "qk", "all"])
+def test_zero_rows(oracle, ctx, shape, zero):
+    """Whole blocks of zero queries and keys: equal weights, with masked keys at weight 0."""
+    def change(vqkv, tqkv, gains):
+        n = 5120 if zero.endswith("qk") else 7680
+        if not zero.startswith("text"):
+            vqkv[:, :n] = 0
+        if not zero.startswith("video"):
+            tqkv[:, :n] = 0
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        if zero == "all":
+            assert not a.any()
+        else:
+            assert np.isfinite(a).all() and rel(a, b) <= 5e-6
