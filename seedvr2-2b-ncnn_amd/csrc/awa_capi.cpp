@@ -482,6 +482,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size();
     sa.kexp = pa.kexp; sa.vexp = pa.vexp;
     sa.tile_meta = g->d_tile_meta; sa.vcs = g->d_vcs; sa.tcs = g->d_tcs; sa.nq_v = d_nq_v; sa.nq_t = d_nq_t;
+    sa.nk_v = d_nk_v; sa.nk_t = d_nk_t;
     sa.eps = eps; sa.qscale = pa.qscale;
     HIPCK(ctx, launch_sdpa(dtype, sa, s));
     HIPCK(ctx, mark());

@@ -98,6 +98,28 @@ __device__ inline void split8(const float (&x)[8], uint32_t (&hi)[4], uint32_t (
 #pragma unroll
     for (int i = 0; i < 4; i++) split2(x[2 * i], x[2 * i + 1], hi[i], lo[i]);
 }
+// Maximum over the four lanes l % 16 + 16 i (a row of the fragment
+// layouts), without LDS.
+__device__ inline float max4(float v) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Where split V loses nothing: an element keeps 2^-40 of its 16-row block's
+// largest and a probability 2^-33 times the window's largest block over its
+// own (awa_sdpa_f32.hip), so a channel must not be much smaller than the others
+// of its blocks, nor a block than the others of its window.  The pack kernel
+// marks a block wide (VEXP_WIDE in place of its exponent) if the largest value
+// of a channel, zero channels aside, is over 2^SPREAD_CHANNELS below the block's
+// largest (whole blocks only: one or two rows hold small values by chance), or
+// if the block lies below the scales' range; the attention kernel takes the
+// fp32 MFMAs for a window with a wide block, with blocks over 2^SPREAD_BLOCKS
+// apart or without any whole block.
+constexpr int SPREAD_CHANNELS = 10, SPREAD_BLOCKS = 6;
+constexpr float VEXP_WIDE = 1000.f, VEXP_ZERO = -1000.f;
+
 // Fragment order of a packed fp32 tile (32 fragments of 1 KiB, lane l's 16 bytes
 // at 16 l), by 32-key halves of 16 KiB.  K: key block b (16 keys), k32 step s of
 // the channels, hi (0) or lo (1); lane 16 q + r: key 16 b + r, channels
@@ -327,7 +349,8 @@ struct PackArgs {
     void* Qp;              // bf16 storage only (the fp32 attention normalises its own queries)
     void* Kp;
     void* Vp;              // fp32 storage only (the bf16 attention reads V from vqkv / tqkv)
-    // fp32 storage: [HEADS][n_tiles][4], of each 16-row block with split_scale 2^a: 2^-a of K, -a of V
+    // fp32 storage: [HEADS][n_tiles][4], of each 16-row block with split_scale 2^a: 2^-a of K; -a of V,
+    // VEXP_ZERO of a block of zeros, VEXP_WIDE of one that the split does not hold
     float *kexp, *vexp;
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles;
     float eps;
@@ -356,13 +379,13 @@ struct SdpaArgs {
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles, n_items, nwin;
     float scale_log2e;     // multiplier of the scores (1 when Q carries the scale)
     // fp32 kernel: its workgroups, the packed blocks' factors, and what the
-    // queries' normalisation and rotation need (as in PackArgs)
+    // rows' normalisation and rotation need (as in PackArgs)
     const int32_t* f32_work;
     int n_f32_work;
     const float *kexp, *vexp;
     const int32_t* tile_meta;
     const float2 *vcs, *tcs;
-    const float *nq_v, *nq_t;
+    const float *nq_v, *nq_t, *nk_v, *nk_t;
     float eps, qscale;
 };
 hipError_t launch_sdpa(int dtype, const SdpaArgs& a, hipStream_t s);

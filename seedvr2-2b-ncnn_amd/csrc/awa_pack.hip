@@ -69,7 +69,7 @@ template <> struct Io<float> {
 // quad's sum) and in the 16 (the other half's): every lane adds the same
 // two partial sums as with partners lane ^ 4 and lane ^ 8, so the result is
 // the xor butterfly's, bit for bit.
-__device__ inline float dpp_add(float v, int ctrl) {
+__device__ inline float dpp_move(float v, int ctrl) {
     int m;
     switch (ctrl) {  // the control must be a constant
     case 0xB1: m = __builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, false); break;  // [1,0,3,2]
@@ -77,13 +77,19 @@ __device__ inline float dpp_add(float v, int ctrl) {
     case 0x141: m = __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, false); break; // row_half_mirror
     default: m = __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, false); break;    // row_mirror
     }
-    return v + __int_as_float(m);
+    return __int_as_float(m);
 }
 __device__ inline float row_sum16(float v) {
-    v = dpp_add(v, 0xB1);
-    v = dpp_add(v, 0x4E);
-    v = dpp_add(v, 0x141);
-    return dpp_add(v, 0x140);
+    v += dpp_move(v, 0xB1);
+    v += dpp_move(v, 0x4E);
+    v += dpp_move(v, 0x141);
+    return v + dpp_move(v, 0x140);
+}
+__device__ inline float row_min16(float v) {
+    v = fminf(v, dpp_move(v, 0xB1));
+    v = fminf(v, dpp_move(v, 0x4E));
+    v = fminf(v, dpp_move(v, 0x141));
+    return fminf(v, dpp_move(v, 0x140));
 }
 // V staging tile in LDS (fp32), [slot][d] with a row pitch of VP words: four
 // rows apart is 16 banks of 64, so the transposing reads below (16 channels x
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     constexpr int NCS = QR * CS_Q4 / 256;         // table float4 per thread
     __shared__ __align__(16) float vs[QR * VP];
     __shared__ float4 lds_cs[QR * CS_Q4];
-    __shared__ float mxs[4][2 * RT];
+    __shared__ float mxs[4][2 * RT], mns[4][RT];
 
     const int nblk = a.n_tiles * HEADS * NQ;
     const int lid = xcd_remap(nblk);  // a tile's workgroups: neighbouring ids, one XCD
@@ -240,13 +246,6 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
                             i & 1 ? SPLIT_FLOOR_V : SPLIT_FLOOR_QK);
 
     const size_t ht = (size_t)h * a.n_tiles + tile;
-    if (tid < 2 * RT) {
-        const float f = split_scale(fmaxf(fmaxf(mxs[0][tid], mxs[1][tid]), fmaxf(mxs[2][tid], mxs[3][tid])),
-                                    tid & 1 ? SPLIT_FLOOR_V : SPLIT_FLOOR_QK);
-        const size_t b = ht * 4 + qt * RT + (tid >> 1);
-        if (tid & 1) a.vexp[b] = (float)(127 - (int)(__float_as_uint(f) >> 23));
-        else a.kexp[b] = 1.f / f;
-    }
     unsigned char* Kt = reinterpret_cast<unsigned char*>(a.Kp) + ht * (TILE * HEAD_D * 4);
     unsigned char* Vt = reinterpret_cast<unsigned char*>(a.Vp) + ht * (TILE * HEAD_D * 4);
     uint32_t hi[4], lo[4];
@@ -261,15 +260,28 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     }
     // V^T fragments: a 16-row block is half of a lane's eight keys
     const int r16 = tid & 15, q = (tid >> 4) & 3;
+    // the largest magnitude in channel r16 of the block, infinity for zeros only
+    auto channel_max = [](const float* v) __attribute__((always_inline)) {
+        const float m = max4(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        return m > 0.f ? m : INFINITY;
+    };
+    float cmin[RT];  // the smallest of them in each block
+#pragma unroll
+    for (int i = 0; i < RT; i++) cmin[i] = INFINITY;
     if constexpr (RT == 4) {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
             const int u = it * 4 + (tid >> 6), ks = u >> 3, db = u & 7;  // wave-uniform
             float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++)
-                v[e] = vs[(32 * ks + 16 * (e >> 2) + 4 * q + (e & 3)) * VP + 16 * db + r16] *
-                       (ks ? mx[5 + 2 * (e >> 2)] : mx[1 + 2 * (e >> 2)]);
+            for (int e = 0; e < 8; e++) v[e] = vs[(32 * ks + 16 * (e >> 2) + 4 * q + (e & 3)) * VP + 16 * db + r16];
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                float& m = cmin[2 * (it >> 1) + b];  // it >> 1 is ks
+                m = fminf(m, channel_max(v + 4 * b));
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] *= ks ? mx[5 + 2 * (e >> 2)] : mx[1 + 2 * (e >> 2)];
             split8(v, hi, lo);
             unsigned char* d = Vt + f32_vfrag(ks, db, 0) * 1024 + (tid & 63) * 16;
             *reinterpret_cast<uint4*>(d) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
@@ -279,8 +291,10 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         const int db = 2 * (tid >> 6);  // two channel blocks per wave
         float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-            v[e] = vs[(4 * q + (e & 3)) * VP + 16 * (db + (e >> 2)) + r16] * mx[1];
+        for (int e = 0; e < 8; e++) v[e] = vs[(4 * q + (e & 3)) * VP + 16 * (db + (e >> 2)) + r16];
+        cmin[0] = fminf(channel_max(v), channel_max(v + 4));
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] *= mx[1];
         split8(v, hi, lo);
 #pragma unroll
         for (int b = 0; b < 2; b++) {
@@ -288,6 +302,27 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
             *reinterpret_cast<uint2*>(d) = make_uint2(hi[2 * b], hi[2 * b + 1]);
             *reinterpret_cast<uint2*>(d + 1024) = make_uint2(lo[2 * b], lo[2 * b + 1]);
         }
+    }
+    // the blocks' factors
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        cmin[i] = row_min16(cmin[i]);
+        if ((tid & 63) == 0) mns[tid >> 6][i] = cmin[i];
+    }
+    __syncthreads();
+    if (tid < RT) {
+        const int b = qt * RT + tid;  // block of the tile
+        const auto exponent = [](float x) __attribute__((always_inline)) { return (int)(__float_as_uint(x) >> 23) - 127; };
+        auto block_max = [&](int i) __attribute__((always_inline)) {
+            return fmaxf(fmaxf(mxs[0][i], mxs[1][i]), fmaxf(mxs[2][i], mxs[3][i]));
+        };
+        const float vm = block_max(2 * tid + 1);
+        const float vn = fminf(fminf(mns[0][tid], mns[1][tid]), fminf(mns[2][tid], mns[3][tid]));
+        float ve = (float)(exponent(vm) - 14);
+        if (exponent(vm) < SPLIT_FLOOR_V || (nvalid >= 16 * (b + 1) && exponent(vn) < exponent(vm) - SPREAD_CHANNELS))
+            ve = VEXP_WIDE;
+        a.vexp[ht * 4 + b] = vm == 0.f ? VEXP_ZERO : ve;
+        a.kexp[ht * 4 + b] = 1.f / split_scale(block_max(2 * tid), SPLIT_FLOOR_QK);
     }
 }
 

@@ -15,11 +15,16 @@
 // against 5.0e-7 at 1080p).
 //
 // The powers of two 2^a bring every block of 16 rows (K and V: set by the pack
-// kernel per block and head; Q: per row) to at most 2^15, so fp16's range
-// bounds nothing: an element 2^-17 of its block's largest still has its 23
-// bits, and smaller ones are held to 2^-40 of the largest.  They are undone
-// exactly: in the factor of the scores, in P before its split, and in the
-// normalisation of O.  P = exp2(s - m) is split like the rest.
+// kernel per block and head; Q: per row) to at most 2^15: an element 2^-17 of
+// its block's largest still has its 23 bits, smaller ones are held to 2^-40 of
+// the largest.  They are undone exactly: in the factor of the scores, in P
+// before its split, and in the normalisation of O.  P = exp2(s - m) is split
+// like the rest.  Windows whose V spans more than that holds (SPREAD_CHANNELS,
+// SPREAD_BLOCKS) are computed with fp32 MFMAs instead (exact_queries).  Up to
+// there the error is that of N(0, 1) inputs: half of the rows 2^-5 of the others,
+// or a sixteenth of the channels 2^7 times the others, 3.1e-7 to 3.3e-7 at 360p
+// and at most 6.1e-7 in the worst channel, against 4.4e-7 and 9.0e-7 as fp32
+// MFMAs.
 //
 // The query rows are normalised and rotated here (each is read by one
 // workgroup), K and V come from the pack kernel as hi and lo tiles in fragment
@@ -66,14 +71,7 @@ struct Item {
     }
 };
 
-// Maximum / sum over the four lanes l % 16 + 16 i (a row of the fragment
-// layouts), without LDS.
-__device__ inline float max4(float v) {
-    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
+// Sum over the four lanes l % 16 + 16 i, as max4.
 __device__ inline float sum4(float v) {
     auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
@@ -81,12 +79,25 @@ __device__ inline float sum4(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// A wave-uniform value kept in a scalar register.
+__device__ inline float scalar(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+// Maximum over the wave, as a scalar.
+__device__ inline float wave_max(float v) {
+    v = max4(v);
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return scalar(v);
+}
+
 // P is at most 2^M_STALE (the running maximum stays until a tile's exceeds it by
-// more, so that O is rarely rescaled), times 2^P_SHIFT: below 2^16, and down to
-// 2^-22 in fp16's normal range.  A V block is taken as no smaller than 2^V_FLOOR
-// of the window's largest in P's exponent, which keeps P out of fp32's
-// subnormals (the row sum needs it) and lies far below what fp16 holds of V.
-constexpr float P_SHIFT = 8.f, M_STALE = 7.f, V_FLOOR = -60.f;
+// more, so that O is rarely rescaled), times 2^P_SHIFT and the V block's power of
+// two relative to the window's largest (2^-SPREAD_BLOCKS at least, else the
+// window goes to exact_queries): below 2^16, and down to 2^-22 of the largest
+// (2^-16 for the smallest blocks) in fp16's normal range; below that it is held
+// to 2^-33 (2^-27).
+constexpr float P_SHIFT = 8.f, M_STALE = 7.f;
 
 constexpr uint32_t FU_BYTES = 32 * HEAD_D * 4;  // a K or V unit (32 keys): hi and lo, 16 KiB
 constexpr uint32_t V_RING = 2 * FU_BYTES;       // LDS stage: two K units, then two V units
@@ -131,6 +142,208 @@ __device__ inline void mfma_fence(f32x4 (&s)[N][2]) {
     asm volatile("s_nop 1");
 }
 
+// ---- windows whose V the split does not hold (SPREAD_CHANNELS): fp32 MFMAs
+//
+// The same workgroup and the same output for its query tile t, 16 queries a wave, as
+// plain fp32: K and V rows straight from vqkv / tqkv (K normalised and rotated
+// as the pack kernel does) into LDS, 32 keys at a time, and
+// v_mfma_f32_16x16x4_f32 for both products.  The fp32 MFMA's 32 cycles bound it,
+// so it neither pipelines nor shares a unit between two query blocks.  Channels
+// do not depend on each other here and any finite value keeps all its bits.
+// 1080p shifted with every window here: 454 us a pass, 171 on split operands.
+constexpr int EX_P = HEAD_D + 4;  // LDS pitch of a row (floats)
+constexpr int EX_STAGE = 2 * 32 * EX_P;  // K and V rows of a unit
+template <bool kSplit>
+__device__ inline void exact_queries(const SdpaArgs& a, const Item& wt, float* lds, int t) {
+    const int h = wt.h;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // addresses of its own, none held across
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int half = kSplit ? wave >> 2 : 0, w4 = wave & 3, r16 = lane & 15, q = lane >> 4;
+    const int nu = wt.units(), n0 = kSplit ? (nu + 1) >> 1 : nu;
+    const int ubeg = half ? n0 : 0, uend = half ? nu : n0;
+    float* ks = lds + half * EX_STAGE;
+    float* vs = ks + 32 * EX_P;
+
+    // query r16 of the block, channels 32 s + 8 q .. + 7 (k step 8 s + e pairs
+    // channel 32 s + 8 q + e of the four lane groups, in K's fragments alike)
+    const int kq = t ? wt.kq1 : wt.kq0, slot = 16 * w4 + r16;
+    const bool qtxt = kq >= wt.nvt;
+    const uint32_t row_ofs =
+        a.vrow[(size_t)(qtxt ? a.n_vid_tiles + (kq - wt.nvt) : wt.vbase + kq) * TILE + vrow_pos(slot)];
+    const int2 qmeta = reinterpret_cast<const int2*>(a.tile_meta)[wt.tile(kq)];
+    float x[32];
+    {
+        const float* row = reinterpret_cast<const float*>(qtxt ? a.tsrc : a.vsrc) + row_ofs + h * HEAD_D + 8 * q;
+        const float* cs = reinterpret_cast<const float*>(qtxt ? a.tcs : a.vcs) +
+                          ((size_t)qmeta.x + min(slot, qmeta.y - 1)) * (2 * CS_STRIDE) + 8 * q;
+        const float* gain = (qtxt ? a.nq_t : a.nq_v) + 8 * q;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            x[i] = row[32 * (i >> 3) + (i & 7)];
+            ss += x[i] * x[i];
+        }
+        const float n = sqrtf(sum4(ss) / (float)HEAD_D + a.eps), in = 1.f / n;
+#pragma unroll
+        for (int i = 0; i < 32; i += 2) {
+            const int c = 32 * (i >> 3) + (i & 7);
+            const float x0 = div_by(x[i], n, in) * gain[c], x1 = div_by(x[i + 1], n, in) * gain[c + 1];
+            x[i] = (x0 * cs[c] - x1 * cs[c + 1]) * a.qscale;
+            x[i + 1] = (x1 * cs[c] + x0 * cs[c + 1]) * a.qscale;
+        }
+    }
+
+    // a unit's rows: eight threads a row, 16 channels each
+    const int krow = (tid & 255) >> 3, kc = 16 * (tid & 7);
+    float4 rk[4], rv[4], rc[4];
+    auto load_unit = [&](int u) __attribute__((always_inline)) {
+        const int t2 = wt.unit_half(u), tile = t2 >> 1, sl = 32 * (t2 & 1) + krow;
+        const bool txt = u >= wt.vid_units();
+        const uint32_t ofs = a.vrow[(size_t)(txt ? a.n_vid_tiles + (tile - wt.tbase) : tile) * TILE + vrow_pos(sl)];
+        const int2 meta = reinterpret_cast<const int2*>(a.tile_meta)[tile];
+        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + ofs + DIM + h * HEAD_D + kc;
+        const float* cs = reinterpret_cast<const float*>(txt ? a.tcs : a.vcs) +
+                          ((size_t)meta.x + min(sl, meta.y - 1)) * (2 * CS_STRIDE) + kc;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            rk[i] = reinterpret_cast<const float4*>(row)[i];
+            rv[i] = reinterpret_cast<const float4*>(row + DIM)[i];
+            rc[i] = reinterpret_cast<const float4*>(cs)[i];
+        }
+    };
+    auto store_unit = [&](int u) __attribute__((always_inline)) {
+        const float* gain = (u >= wt.vid_units() ? a.nk_t : a.nk_v) + kc;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) ss += rk[i].x * rk[i].x + rk[i].y * rk[i].y + rk[i].z * rk[i].z + rk[i].w * rk[i].w;
+#pragma unroll
+        for (int o = 1; o <= 4; o <<= 1) ss += __shfl_xor(ss, o);
+        const float n = sqrtf(ss / (float)HEAD_D + a.eps), in = 1.f / n;
+        const bool valid = krow < wt.unit_valid(u);  // V of a masked key: 0, whatever its weight's 0 meets
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float k0 = div_by(rk[i].x, n, in) * gain[4 * i], k1 = div_by(rk[i].y, n, in) * gain[4 * i + 1];
+            const float k2 = div_by(rk[i].z, n, in) * gain[4 * i + 2], k3 = div_by(rk[i].w, n, in) * gain[4 * i + 3];
+            *reinterpret_cast<float4*>(ks + krow * EX_P + kc + 4 * i) =
+                make_float4(k0 * rc[i].x - k1 * rc[i].y, k1 * rc[i].x + k0 * rc[i].y, k2 * rc[i].z - k3 * rc[i].w,
+                            k3 * rc[i].z + k2 * rc[i].w);
+            *reinterpret_cast<float4*>(vs + krow * EX_P + kc + 4 * i) = valid ? rv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+
+    f32x4 oacc[8];
+#pragma unroll
+    for (int db = 0; db < 8; db++) oacc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    if (ubeg < uend) load_unit(ubeg);
+    for (int i = 0; i < n0; i++) {  // the same iteration count in both halves
+        const int u = ubeg + i;
+        __syncthreads();  // every wave is done with the unit before
+        if (u < uend) store_unit(u);
+        __syncthreads();
+        if (u + 1 < uend) load_unit(u + 1);
+        if (u >= uend) continue;  // uniform per half
+        f32x4 s[2];
+        const int kv = wt.unit_valid(u);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+            s[kb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < 32; st += 4) {
+                const f32x4 k4 = *reinterpret_cast<const f32x4*>(ks + (16 * kb + r16) * EX_P + 32 * (st >> 3) + 8 * q + (st & 7));
+#pragma unroll
+                for (int e = 0; e < 4; e++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], x[st + e], s[kb], 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (16 * kb + 4 * q + r >= kv) s[kb][r] = -INFINITY;
+                mx = fmaxf(mx, s[kb][r]);
+            }
+        }
+        const float m_new = fmaxf(m, max4(mx));  // finite: every unit has a valid key
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        float psum = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                s[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] - m);
+                psum += s[kb][r];
+            }
+        l = l * alpha + psum;  // this lane's keys; summed over the row at the end
+#pragma unroll
+        for (int db = 0; db < 8; db++) oacc[db] *= alpha;
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int db = 0; db < 8; db++)
+                    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[(16 * kb + 4 * q + r) * EX_P + 16 * db + r16],
+                                                                    s[kb][r], oacc[db], 0, 0, 0);
+    }
+    l = sum4(l);
+    if constexpr (kSplit) {  // half 1 leaves its share past the stages, half 0 merges it
+        f32x4* pub = reinterpret_cast<f32x4*>(lds + 2 * EX_STAGE) + (size_t)w4 * (8 * 64) + lane;
+        float* pml = lds + 2 * EX_STAGE + 4 * 8 * 64 * 4 + w4 * (2 * 64) + lane;
+        if (half == 1) {
+#pragma unroll
+            for (int db = 0; db < 8; db++) pub[64 * db] = oacc[db];
+            pml[0] = m;
+            pml[64] = l;
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float m1 = pml[0], l1 = pml[64], mm = fmaxf(m, m1);
+        const float a0 = __builtin_amdgcn_exp2f(m - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
+        l = l * a0 + l1 * a1;
+#pragma unroll
+        for (int db = 0; db < 8; db++) oacc[db] = oacc[db] * a0 + pub[64 * db] * a1;
+    }
+    if (slot >= wt.nvalid(kq)) return;  // padding
+    float* dst = qtxt ? a.tpart + ((size_t)wt.w * a.txt_len + TILE * (kq - wt.nvt) + slot) * DIM
+                      : reinterpret_cast<float*>(a.vattn) + row_ofs / 3;
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int db = 0; db < 8; db++) *reinterpret_cast<f32x4*>(dst + h * HEAD_D + 16 * db + 4 * q) = oacc[db] * inv;
+}
+
+// The rows of a wave's query blocks nq w4 + qb (nq = 2: blocks 4 .. 7 are of the
+// second query tile): element offsets in vqkv / tqkv, and the tiles' records.
+struct QueryRows {
+    uint32_t ofs[2];
+    int2 meta[2];
+};
+__device__ inline QueryRows query_rows(const SdpaArgs& a, const Item& wt, int nq, int w4, int r16) {
+    QueryRows r;
+#pragma unroll
+    for (int qb = 0; qb < 2; qb++) {
+        const int blk = nq * w4 + min(qb, nq - 1), kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
+        const int row_tile = kq >= wt.nvt ? a.n_vid_tiles + (kq - wt.nvt) : wt.vbase + kq;
+        r.ofs[qb] = a.vrow[(size_t)row_tile * TILE + vrow_pos(slot)];
+        r.meta[qb] = reinterpret_cast<const int2*>(a.tile_meta)[wt.tile(kq)];
+    }
+    return r;
+}
+
+// The largest V exponent of the window, in whose units P V is accumulated, or
+// VEXP_WIDE where the split does not hold the window: the same in every wave.
+__device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane) {
+    const float* ve = a.vexp + (size_t)wt.h * a.n_tiles * 4;
+    float vmax = VEXP_ZERO, vmin = VEXP_WIDE;
+    for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) {
+        const float e = ve[4 * wt.tile(i >> 2) + (i & 3)];
+        vmax = fmaxf(vmax, e);
+        if (e != VEXP_ZERO) vmin = fminf(vmin, e);
+    }
+    vmax = wave_max(vmax);
+    vmin = -wave_max(-vmin);
+    return vmin < vmax - SPREAD_BLOCKS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
+}
+
 // One workgroup per (two query tiles of a window, head), 128 queries: four
 // waves of 32 (or, for an odd window's last tile, of 16).  64 KiB of LDS and at
 // most 256 registers: two workgroups per CU, two waves per SIMD.  Fewer
@@ -170,7 +383,8 @@ __device__ inline void mfma_fence(f32x4 (&s)[N][2]) {
 //     {4 q + e, 16 + 4 q + e}, e = 0..3, which are exactly the lane's score
 //     registers of the unit's two blocks.
 template <int NQ, bool kSplit>
-__device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char* lds) {
+__device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRows& rows, float vmax, unsigned char* lds,
+                                uint32_t* out_ofs) {
     const int h = wt.h;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int half = kSplit ? wave >> 2 : 0, w4 = wave & 3;
@@ -188,7 +402,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
     // units' DMA
     const cfloat2_t* ke = (const cfloat2_t*)(a.kexp) + (size_t)h * a.n_tiles * 2;
     const cfloat2_t* ve2 = (const cfloat2_t*)(a.vexp) + (size_t)h * a.n_tiles * 2;
-    const float* ve = a.vexp + (size_t)h * a.n_tiles * 4;
     // unit u into a ring slot (0, 1: this half's even and odd units)
     auto fetch_k = [&](int u, int slot) __attribute__((always_inline)) {
         if (u < uend)
@@ -202,35 +415,26 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
     fetch_k(ubeg, 0);
     fetch_k(ubeg + 1, 1);
     fetch_v(ubeg, 0);
+    // kept for the end in LDS (as registers they spilled), by the wave that reads it
+    if (half == 0)
+#pragma unroll
+        for (int qb = 0; qb < NQ; qb++) out_ofs[16 * (NQ * w4 + qb) + r16] = rows.ofs[qb];
 
     // ---- this wave's queries: 16-row blocks NQ w4 + qb of the item, every load
     // issued before the first use
-    // element offsets of the queries' rows in vqkv / tqkv
-    uint32_t row_ofs[NQ];
     float4 xr[NQ][8], cs[NQ][8];
-    int2 meta[NQ];
-#pragma unroll
-    for (int qb = 0; qb < NQ; qb++) {
-        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
-        const int row_tile = kq >= wt.nvt ? a.n_vid_tiles + (kq - wt.nvt) : wt.vbase + kq;
-        row_ofs[qb] = a.vrow[(size_t)row_tile * TILE + vrow_pos(slot)];
-        meta[qb] = reinterpret_cast<const int2*>(a.tile_meta)[wt.tile(kq)];
-    }
 #pragma unroll
     for (int qb = 0; qb < NQ; qb++) {
         const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
         const bool txt = kq >= wt.nvt;
-        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + row_ofs[qb] + h * HEAD_D + 8 * q;
+        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + rows.ofs[qb] + h * HEAD_D + 8 * q;
         const float4* cst = reinterpret_cast<const float4*>(txt ? a.tcs : a.vcs) +
-                            ((size_t)meta[qb].x + min(slot, meta[qb].y - 1)) * (CS_STRIDE / 2) + 2 * q;
+                            ((size_t)rows.meta[qb].x + min(slot, rows.meta[qb].y - 1)) * (CS_STRIDE / 2) + 2 * q;
 #pragma unroll
         for (int i = 0; i < 8; i++) xr[qb][i] = *reinterpret_cast<const float4*>(row + 32 * (i >> 1) + 4 * (i & 1));
 #pragma unroll
         for (int i = 0; i < 8; i++) cs[qb][i] = cst[8 * (i >> 1) + (i & 1)];
     }
-    // the largest V exponent of the window: P V is accumulated in its units
-    float vmax = -1000.f;
-    for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) vmax = fmaxf(vmax, ve[4 * wt.tile(i >> 2) + (i & 3)]);
 
     f16x8 qh[NQ][4], ql[NQ][4];
     float cq[NQ];
@@ -277,8 +481,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
         }
         __builtin_amdgcn_sched_barrier(0);  // one block's gains at a time: registers
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
 
     f32x4 oacc[8][NQ];
     float m_i[NQ], l_i[NQ];
@@ -361,13 +563,14 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
         f32x4 (&sn)[2][NQ] = s[sl ^ 1];
         const int un = min(u + 1, uend - 1);  // past the end: any unit's factors
         const f32x2 kcn = ke[wt.unit_half(un)];
-        // P leaves as exp2(s - m + vs): vs puts the block's V scale and
-        // P_SHIFT into the exponent, vi takes them back out of the row sum
+        // P leaves as exp2(s - m + vs): vs puts the block's V scale (of a block
+        // of zeros any) and P_SHIFT into the exponent, vi takes them back out of
+        // the row sum
         f32x2 vs = ve2[wt.unit_half(u)], vi;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
-            vs[kb] = fmaxf(vs[kb] - vmax, V_FLOOR) + P_SHIFT;
-            vi[kb] = __builtin_amdgcn_exp2f(-vs[kb]);  // exact: whole exponents
+            vs[kb] = scalar(fmaxf(vs[kb] - vmax, (float)-SPREAD_BLOCKS) + P_SHIFT);
+            vi[kb] = scalar(__builtin_amdgcn_exp2f(-vs[kb]));  // exact: whole exponents
         }
         uint32_t hi[NQ][4], lo[NQ][4];
         // ---- phase A
@@ -510,7 +713,7 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
         for (int i = 0; i < 8; i++) {
             const int row = 2 * i + (ln >> 5), ch = ln & 31, slot = 16 * (blk & 3) + row;
             const f32x4 v = stg[row * 32 + (ch ^ row)];
-            const uint32_t ofs = __shfl(row_ofs[qb], row);
+            const uint32_t ofs = out_ofs[16 * blk + row];
             if (slot >= wt.nvalid(kq)) continue;  // padding
             // video: the token's row of vattn (a row is a third of its qkv row)
             float* dst = kq < wt.nvt ? reinterpret_cast<float*>(a.vattn) + ofs / 3
@@ -524,6 +727,7 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, unsigned char
 template <bool kSplit>
 __global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArgs a) {
     __shared__ __align__(16) unsigned char lds[(kSplit ? 2 : 1) * STAGE_BYTES];
+    __shared__ uint32_t out_ofs[2 * TILE];
     const int e = a.f32_work[blockIdx.x];
     if (e < 0) return;  // an idle entry
     const int4 d0 = reinterpret_cast<const int4*>(a.sched_desc)[2 * (e >> 2)];
@@ -533,8 +737,16 @@ __global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArg
     it.h = d0.x & 255; it.w = d0.x >> 8; it.kq0 = part == 2 ? d0.z : d0.y; it.kq1 = part ? -1 : d0.z;
     it.vbase = d1.x; it.nvt = d1.y; it.tbase = d1.z; it.f = d1.w;
     it.ntt = a.ntt; it.txt = a.txt_len;
-    if (it.kq1 >= 0) run_item<2, kSplit>(a, it, lds);
-    else run_item<1, kSplit>(a, it, lds);
+    const int nq = it.kq1 >= 0 ? 2 : 1;
+    const QueryRows rows =
+        query_rows(a, it, nq, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3, threadIdx.x & 15);
+    const float vmax = window_vmax(a, it, threadIdx.x & 63);
+    if (vmax == VEXP_WIDE) {
+        for (int t = 0; t < nq; t++) exact_queries<kSplit>(a, it, reinterpret_cast<float*>(lds), t);
+        return;
+    }
+    if (nq == 2) run_item<2, kSplit>(a, it, rows, vmax, lds, out_ofs);
+    else run_item<1, kSplit>(a, it, rows, vmax, lds, out_ofs);
 }
 
 }  // namespace

@@ -112,3 +112,32 @@ def test_zero_rows(oracle, ctx, shape, zero):
             assert not a.any()
         else:
             assert np.isfinite(a).all() and rel(a, b) <= 5e-6
+
+
+def worst_channel(a, b):
+    """Largest relative 2-norm error of one channel of one head over the rows."""
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    return float((np.linalg.norm(a - b, axis=0) / np.linalg.norm(b, axis=0)).max())
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+@pytest.mark.parametrize("e", [0, 6, 12, 24, 32, 60])
+def test_one_large_v(oracle, ctx, shape, e):
+    """Channels do not depend on each other: one element of V 2^e times as large
+    leaves every other channel as accurate as before.  Bar 1e-5 per channel:
+    the 5e-6 above, and a factor of two for the worst of 2,560 channels."""
+    def change(vqkv, tqkv, gains):
+        vqkv[101, 5120 + 128 * 3 + 17] *= np.float32(2.0 ** e)
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert worst_channel(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+def test_small_channels(oracle, ctx, shape):
+    """Channels of V of very different sizes, side by side and from row to row."""
+    def change(vqkv, tqkv, gains):
+        for x in (vqkv, tqkv):
+            x[:, 5120:] *= np.exp2(np.arange(2560) % 40 - 20).astype(np.float32)
+        vqkv[150:170, 5120:] *= np.float32(2.0 ** -18)
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert worst_channel(a, b) <= 1e-5
