@@ -69,8 +69,7 @@ __device__ inline float div_by(float x, float r, float rinv) {
 
 // The fp32 path's split operands: x 2^a = hi + lo (two fp16), 2^a =
 // split_scale(largest finite magnitude of the block) bringing that magnitude
-// to [2^14, 2^15), or less where it is below 2^floor.  Infinities take no part
-// in the scale and split into infinity and NaN.
+// to [2^14, 2^15), or less where it is below 2^floor.
 __device__ inline float finite_abs(float x) {
     const float v = fabsf(x);
     return v < __builtin_inff() ? v : 0.f;
@@ -113,8 +112,9 @@ __device__ inline float max4(float v) {
 // of its blocks, nor a block than the others of its window.  The pack kernel
 // marks a block wide (VEXP_WIDE in place of its exponent) if the largest value
 // of a channel, zero channels aside, is over 2^SPREAD_CHANNELS below the block's
-// largest (whole blocks only: one or two rows hold small values by chance), or
-// if the block lies below the scales' range; the attention kernel takes the
+// largest (whole blocks only: one or two rows hold small values by chance), if
+// the block lies below the scales' range, or if its K or V holds an infinity
+// (which splits into infinity and NaN; a NaN stays one either way); the attention kernel takes the
 // fp32 MFMAs for a window with a wide block, with blocks over 2^SPREAD_BLOCKS
 // apart or without any whole block.
 constexpr int SPREAD_CHANNELS = 10, SPREAD_BLOCKS = 6;

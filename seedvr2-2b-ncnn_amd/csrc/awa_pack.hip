@@ -225,8 +225,8 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         IO::widen(rv[kk], v);
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            mx[2 * kk] = fmaxf(mx[2 * kk], finite_abs(k[kk][i]));
-            mx[2 * kk + 1] = fmaxf(mx[2 * kk + 1], finite_abs(v[i]));
+            mx[2 * kk] = fmaxf(mx[2 * kk], fabsf(k[kk][i]));
+            mx[2 * kk + 1] = fmaxf(mx[2 * kk + 1], fabsf(v[i]));
         }
         float4* vrow = reinterpret_cast<float4*>(vs + lr * VP + c * 8);
         vrow[0] = rv[kk].a;
@@ -316,13 +316,13 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         auto block_max = [&](int i) __attribute__((always_inline)) {
             return fmaxf(fmaxf(mxs[0][i], mxs[1][i]), fmaxf(mxs[2][i], mxs[3][i]));
         };
-        const float vm = block_max(2 * tid + 1);
+        const float km = block_max(2 * tid), vm = block_max(2 * tid + 1);
         const float vn = fminf(fminf(mns[0][tid], mns[1][tid]), fminf(mns[2][tid], mns[3][tid]));
         float ve = (float)(exponent(vm) - 14);
-        if (exponent(vm) < SPLIT_FLOOR_V || (nvalid >= 16 * (b + 1) && exponent(vn) < exponent(vm) - SPREAD_CHANNELS))
+        if (exponent(vm) < SPLIT_FLOOR_V || exponent(vm) == 128 || (nvalid >= 16 * (b + 1) && exponent(vn) < exponent(vm) - SPREAD_CHANNELS))
             ve = VEXP_WIDE;
-        a.vexp[ht * 4 + b] = vm == 0.f ? VEXP_ZERO : ve;
-        a.kexp[ht * 4 + b] = 1.f / split_scale(block_max(2 * tid), SPLIT_FLOOR_QK);
+        a.vexp[ht * 4 + b] = exponent(km) == 128 ? VEXP_WIDE : vm == 0.f ? VEXP_ZERO : ve;
+        a.kexp[ht * 4 + b] = 1.f / split_scale(km, SPLIT_FLOOR_QK);
     }
 }
 

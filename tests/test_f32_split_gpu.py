@@ -141,3 +141,16 @@ def test_small_channels(oracle, ctx, shape):
         vqkv[150:170, 5120:] *= np.float32(2.0 ** -18)
     for a, b in zip(*both(oracle, ctx, shape, change)):
         assert worst_channel(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+def test_infinite_v(oracle, ctx, shape):
+    """An infinity in V is an infinity in its channel of the rows that see it."""
+    def change(vqkv, tqkv, gains):
+        vqkv[101, 5120 + 17] = np.inf
+        vqkv[33, 5120 + 128 * 7 + 90] = -np.inf
+        tqkv[5, 5120 + 128 * 9 + 3] = np.inf
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert np.isinf(b).any() and np.array_equal(np.isinf(a), np.isinf(b)) and not np.isnan(a).any()
+        fin = np.isfinite(b)
+        assert np.array_equal(a[~fin], b[~fin]) and rel(a[fin], b[fin]) <= 5e-6
