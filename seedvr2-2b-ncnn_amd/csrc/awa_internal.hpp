@@ -70,10 +70,6 @@ __device__ inline float div_by(float x, float r, float rinv) {
 // The fp32 path's split operands: x 2^a = hi + lo (two fp16), 2^a =
 // split_scale(largest finite magnitude of the block) bringing that magnitude
 // to [2^14, 2^15), or less where it is below 2^floor.
-__device__ inline float finite_abs(float x) {
-    const float v = fabsf(x);
-    return v < __builtin_inff() ? v : 0.f;
-}
 // V: the scale stays finite.  Q and K: so does the product of two of them, and
 // its inverse, which the scores are multiplied by, stays a normal number (0
 // times a masked score's -infinity is NaN); what a block below 2^-45 loses is

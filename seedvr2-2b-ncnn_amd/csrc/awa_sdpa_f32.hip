@@ -99,6 +99,14 @@ __device__ inline float wave_max(float v) {
 // to 2^-33 (2^-27).
 constexpr float P_SHIFT = 8.f, M_STALE = 7.f;
 
+// The largest query value times the largest key value up to which the split
+// holds the scores.  Values are held to 2^-40 of the largest of their row or
+// block, so a score is off by up to some 2^-36 of this product: far below the
+// rounding of its own sum, unless the gains of q and k cancel channel by channel
+// (2^10 against 2^-10: product 2^21, error 1.8e-6 for 3.2e-7).  2^13 leaves 2^-26
+// (N(0, 1) rows and gains of 1: 2^4).
+constexpr float QK_MAX = 8192.f;
+
 constexpr uint32_t FU_BYTES = 32 * HEAD_D * 4;  // a K or V unit (32 keys): hi and lo, 16 KiB
 constexpr uint32_t V_RING = 2 * FU_BYTES;       // LDS stage: two K units, then two V units
 constexpr uint32_t STAGE_BYTES = 4 * FU_BYTES;  // 64 KiB
@@ -332,16 +340,24 @@ __device__ inline QueryRows query_rows(const SdpaArgs& a, const Item& wt, int nq
 // The largest V exponent of the window, in whose units P V is accumulated, or
 // VEXP_WIDE where the split does not hold the window: the same in every wave.
 __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane) {
-    const float* ve = a.vexp + (size_t)wt.h * a.n_tiles * 4;
-    float vmax = VEXP_ZERO, vmin = VEXP_WIDE;
+    const float *ve = a.vexp + (size_t)wt.h * a.n_tiles * 4, *ke = a.kexp + (size_t)wt.h * a.n_tiles * 4;
+    static_assert(HEAD_D == 128, "two gains per lane");
+    const float g = fmaxf(fmaxf(fabsf(a.nq_v[lane]), fabsf(a.nq_v[lane + 64])),
+                          fmaxf(fabsf(a.nq_t[lane]), fabsf(a.nq_t[lane + 64])));
+    float vmax = VEXP_ZERO, vmin = VEXP_WIDE, kmax = 0.f;
     for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) {
-        const float e = ve[4 * wt.tile(i >> 2) + (i & 3)];
+        const int b = 4 * wt.tile(i >> 2) + (i & 3);
+        const float e = ve[b];
         vmax = fmaxf(vmax, e);
         if (e != VEXP_ZERO) vmin = fminf(vmin, e);
+        kmax = fmaxf(kmax, ke[b]);
     }
     vmax = wave_max(vmax);
     vmin = -wave_max(-vmin);
-    return vmin < vmax - SPREAD_BLOCKS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
+    // a normalised query's largest value is below sqrt(2 128) qscale = 2.05 times
+    // its largest gain, a key's below 2^15 times its block's 2^-a
+    const float qk = wave_max(g) * wave_max(kmax) * 65536.f;
+    return vmin < vmax - SPREAD_BLOCKS || qk > QK_MAX || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
 }
 
 // One workgroup per (two query tiles of a window, head), 128 queries: four
@@ -467,7 +483,7 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
                 mx = fmaxf(mx, fmaxf(fabsf(x[4 * i + p]), fabsf(x[4 * i + p + 1])));
             }
         }
-        const float f = split_scale(finite_abs(max4(mx)), SPLIT_FLOOR_QK);
+        const float f = split_scale(max4(mx), SPLIT_FLOOR_QK);
         cq[qb] = 1.f / f;
 #pragma unroll
         for (int st = 0; st < 4; st++) {

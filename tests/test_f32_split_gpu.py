@@ -154,3 +154,14 @@ def test_infinite_v(oracle, ctx, shape):
         assert np.isinf(b).any() and np.array_equal(np.isinf(a), np.isinf(b)) and not np.isnan(a).any()
         fin = np.isfinite(b)
         assert np.array_equal(a[~fin], b[~fin]) and rel(a[fin], b[fin]) <= 5e-6
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+def test_opposite_gains(oracle, ctx, shape):
+    """Gains of q and k that cancel channel by channel: the scores are as before."""
+    def change(vqkv, tqkv, gains):
+        s = np.exp2(4.0 * (np.arange(128) // 2 % 9 - 4)).astype(np.float32)
+        for i in range(4):
+            gains[i] = (gains[i] * (s if i % 2 == 0 else 1 / s)).astype(np.float32)
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert worst_channel(a, b) <= 1e-5
