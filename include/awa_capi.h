@@ -153,7 +153,7 @@ int awa_forward(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
  * device it runs on until the process ends (awa_create looks up its address).
  * Geometries whose scratch exceeds it are rejected with AWA_EARG (1080p bf16
  * needs 76 MiB, the 71 x 97 grid with 77 text rows 104 MiB; fp32 storage
- * also packs V and needs about 2.6 times as much).  No per-phase timing events
+ * packs K and V and needs about 1.9 times as much).  No per-phase timing events
  * are recorded.  All calls on one device share the array: calls that overlap
  * in time on one device race. */
 enum { AWA_NOALLOC_SCRATCH_MIB = 128 };

@@ -418,11 +418,23 @@ hipError_t timing_mark(awa_ctx* ctx, hipStream_t s) { return event_mark(ctx, ctx
 
 namespace awa {
 
-size_t op_scratch_bytes(const GeomPlan& P, int dtype) {
-    const size_t packed = (size_t)HEADS * P.n_tiles * TILE * HEAD_D * elem_size(dtype);
-    const size_t n_packed = dtype == AWA_BF16 ? 2 : 3;  // Q, K (and V for fp32)
-    return n_packed * align256(packed) + align256((size_t)P.nwin * P.txt_len * DIM * 4);
-}
+namespace {
+// The op's scratch: bf16 Q and K tiles, fp32 the blocks' factors (kexp, then
+// vexp), K and V tiles; then the text partials.
+struct ScratchLayout {
+    size_t off_k, off_v, off_t, bytes;
+    ScratchLayout(const GeomPlan& P, int dtype) {
+        const bool bf16 = dtype == AWA_BF16;
+        const size_t packed = align256((size_t)HEADS * P.n_tiles * TILE * HEAD_D * elem_size(dtype));
+        off_k = bf16 ? packed : align256((size_t)2 * HEADS * P.n_tiles * 4 * sizeof(float));
+        off_v = off_k + packed;
+        off_t = bf16 ? off_v : off_v + packed;
+        bytes = off_t + align256((size_t)P.nwin * P.txt_len * DIM * 4);
+    }
+};
+}  // namespace
+
+size_t op_scratch_bytes(const GeomPlan& P, int dtype) { return ScratchLayout(P, dtype).bytes; }
 
 int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv, const void* d_tqkv,
                  const float* d_nq_v, const float* d_nk_v, const float* d_nq_t, const float* d_nk_t,
@@ -431,9 +443,8 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     const GeomPlan& P = g->plan;
     const int Lv = P.Lv;
     const size_t es = elem_size(dtype);
-    const size_t packed = (size_t)HEADS * P.n_tiles * TILE * HEAD_D * es;
     const bool bf16 = dtype == AWA_BF16;
-    const size_t off_k = align256(packed), off_v = 2 * off_k, off_t = (bf16 ? 2 : 3) * off_k;
+    const ScratchLayout lay(P, dtype);
     // the bf16 kernel addresses vattn with 32-bit buffer offsets (and marks
     // padding rows with offsets from 2^31), and vqkv / tqkv rows through the
     // geometry's 32-bit row table
@@ -443,7 +454,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     }
     char* base = static_cast<char*>(ext_scratch);
     if (!base) {
-        int rc = ensure_scratch(ctx, op_scratch_bytes(P, dtype));
+        int rc = ensure_scratch(ctx, lay.bytes);
         if (rc != AWA_OK) return rc;
         base = static_cast<char*>(ctx->scratch);
     }
@@ -459,8 +470,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     pa.nq_v = d_nq_v; pa.nk_v = d_nk_v; pa.nq_t = d_nq_t; pa.nk_t = d_nk_t;
     pa.tile_meta = g->d_tile_meta; pa.vrow = g->d_vrow;
     pa.vcs = g->d_vcs; pa.tcs = g->d_tcs;
-    // bf16: Q and K; fp32: K, V and the blocks' factors (in Q's place)
-    pa.Qp = bf16 ? base : nullptr; pa.Kp = base + off_k; pa.Vp = bf16 ? nullptr : base + off_v;
+    pa.Qp = bf16 ? base : nullptr; pa.Kp = base + lay.off_k; pa.Vp = bf16 ? nullptr : base + lay.off_v;
     pa.kexp = reinterpret_cast<float*>(base); pa.vexp = pa.kexp + (size_t)HEADS * P.n_tiles * 4;
     pa.n_vid_tiles = P.n_vid_tiles; pa.ntt = P.ntt; pa.txt_sets = P.txt_sets; pa.txt_len = P.txt_len;
     pa.n_tiles = P.n_tiles; pa.eps = eps;
@@ -476,7 +486,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.items = g->d_items; sa.cumf = g->d_cumf; sa.vidx = g->d_vidx; sa.tile_base = g->d_tile_base;
     sa.sched_start = g->d_sched_start; sa.sched_desc = g->d_sched_desc; sa.n_slots = P.n_slots; sa.n_used_slots = P.n_used_slots;
     sa.vattn = d_vattn; sa.vattn_bytes = (uint32_t)((size_t)Lv * DIM * es);
-    sa.tpart = reinterpret_cast<float*>(base + off_t);
+    sa.tpart = reinterpret_cast<float*>(base + lay.off_t);
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;
     sa.n_tiles = P.n_tiles; sa.n_items = P.n_items; sa.nwin = P.nwin;
     sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size();

@@ -302,8 +302,9 @@ int check_forward_args(const char* who, awa_ctx* ctx, const awa_geom* g, int dty
                        const void* d_vqkv, const void* d_tqkv, int Lv, int TXT, const float* d_nq_v,
                        const float* d_nk_v, const float* d_nq_t, const float* d_nk_t, float eps,
                        const void* d_vattn, const void* d_tattn);
-// Bytes of scratch the op needs for a geometry and storage type: packed Q, K
-// and V tiles, then the per-window text partials, each 256-byte aligned.
+// Bytes of scratch the op needs for a geometry and storage type: the packed
+// tiles (bf16 Q and K; fp32 K and V, with their factors), then the per-window
+// text partials, each 256-byte aligned.
 size_t op_scratch_bytes(const GeomPlan& P, int dtype);
 // awa_forward without argument checks (shared with the block).  ext_scratch:
 // nullptr uses the context's scratch (grown on demand, per-phase events when

@@ -12,8 +12,9 @@
 // the host that name is only a stand-in, not a device address): awa_create
 // looks up the current device's address once with hipGetSymbolAddress, and
 // that pointer is what the kernels receive.  The kernels overwrite every byte
-// they later read (padding rows of the packed tiles are written as zeros,
-// every window writes all of its text partial rows), so nothing needs
+// they later read (padding rows of the packed tiles are written, as zeros for
+// bf16 and as the window's last row for fp32, and every window writes all of
+// its text partial rows), so nothing needs
 // clearing between calls.  All calls on one device share the array: calls
 // that overlap in time on one device, on any streams or contexts, race.
 #include <mutex>

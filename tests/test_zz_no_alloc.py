@@ -74,7 +74,7 @@ def test_noalloc_matches_forward(awa):
 
 
 def test_noalloc_refuses_oversized_geometry(awa):
-    """1080p with fp32 storage needs about 200 MiB of scratch, more than the
+    """1080p with fp32 storage needs 138 MiB of scratch, more than the
     fixed array holds: refused before any kernel is enqueued."""
     import torch
     dev = torch.device("cuda:0")
@@ -87,5 +87,22 @@ def test_noalloc_refuses_oversized_geometry(awa):
         ctx.forward(g, vq, tq, *gains, eps=1e-5, noalloc=True)
     assert e.value.code == awa.AWA_EARG
     assert "at most" in str(e.value)
+    g.close()
+    ctx.close()
+
+
+def test_noalloc_f32_scratch_holds_two_tiles(awa):
+    """fp32 storage packs K and V: the unshifted 1080p layer needs 127 MiB and
+    fits (with a third packed tile it would need 185)."""
+    import torch
+    dev = torch.device("cuda:0")
+    ctx = awa.Context(0)
+    g = ctx.build_geometry(1, 68, 80, (4, 3, 3), 58, 0)
+    vqkv, tqkv, gains = seeded_awa_inputs(5440, 58, 43)
+    args = [torch.from_numpy(x).to(dev) for x in (vqkv, tqkv, *gains)]
+    got = ctx.forward(g, *args, eps=1e-5, noalloc=True)
+    ref = ctx.forward(g, *args, eps=1e-5)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
     g.close()
     ctx.close()
