@@ -139,7 +139,11 @@ int awa_reserve(awa_ctx* ctx, const awa_geom* g, int dtype);
  *   Lv, TXT   must equal the geometry's Lv and txt_len
  *   d_nq_v .. d_nk_t  fp32 [128] device vectors
  * Tokens outside every window get zero rows, as the reference's zero-fill
- * (awa_layer.cpp:386-399). */
+ * (awa_layer.cpp:386-399).
+ * d_vattn may lie over d_vqkv or d_tqkv, and d_tattn too (not over each other):
+ * the video rows then go through the scratch and a device copy, which needs
+ * Lv * 2560 elements more of it (reserved by awa_reserve for AWA_F32; for
+ * AWA_BF16 the first such call allocates them). */
 int awa_forward(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
                 const void* d_tqkv, int Lv, int TXT, const float* d_nq_v,
                 const float* d_nk_v, const float* d_nq_t, const float* d_nk_t,

@@ -423,6 +423,7 @@ namespace {
 // vexp), K and V tiles; then the text partials.
 struct ScratchLayout {
     size_t off_k, off_v, off_t, bytes;
+    size_t rows;  // the video rows, past `bytes`: for a call whose vattn lies over its inputs
     ScratchLayout(const GeomPlan& P, int dtype) {
         const bool bf16 = dtype == AWA_BF16;
         const size_t packed = align256((size_t)HEADS * P.n_tiles * TILE * HEAD_D * elem_size(dtype));
@@ -430,11 +431,25 @@ struct ScratchLayout {
         off_v = off_k + packed;
         off_t = bf16 ? off_v : off_v + packed;
         bytes = off_t + align256((size_t)P.nwin * P.txt_len * DIM * 4);
+        rows = align256((size_t)P.Lv * DIM * elem_size(dtype));
     }
 };
+bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+}
 }  // namespace
 
-size_t op_scratch_bytes(const GeomPlan& P, int dtype) { return ScratchLayout(P, dtype).bytes; }
+size_t op_scratch_bytes(const GeomPlan& P, int dtype, bool in_place) {
+    const ScratchLayout lay(P, dtype);
+    return lay.bytes + (in_place ? lay.rows : 0);
+}
+
+bool op_in_place(const GeomPlan& P, int dtype, const void* d_vqkv, const void* d_tqkv, const void* d_vattn) {
+    const size_t es = elem_size(dtype), out = (size_t)P.Lv * DIM * es;
+    return overlaps(d_vattn, out, d_vqkv, (size_t)P.Lv * QKV * es) ||
+           overlaps(d_vattn, out, d_tqkv, (size_t)P.txt_len * QKV * es);
+}
 
 int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv, const void* d_tqkv,
                  const float* d_nq_v, const float* d_nk_v, const float* d_nq_t, const float* d_nk_t,
@@ -452,17 +467,22 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
         set_err(ctx, "awa_forward: Lv=%d video rows exceed the bf16 path's 32-bit addressing", Lv);
         return AWA_EARG;
     }
+    // the attention kernels read rows of vqkv and tqkv while others of its
+    // workgroups already write vattn: over its inputs it is formed in the scratch
+    // and copied at the end
+    const bool in_place = op_in_place(P, dtype, d_vqkv, d_tqkv, d_vattn);
     char* base = static_cast<char*>(ext_scratch);
     if (!base) {
-        int rc = ensure_scratch(ctx, lay.bytes);
+        int rc = ensure_scratch(ctx, lay.bytes + (in_place ? lay.rows : 0));
         if (rc != AWA_OK) return rc;
         base = static_cast<char*>(ctx->scratch);
     }
+    void* const d_rows = in_place ? base + lay.bytes : d_vattn;
     // per-phase events only for the context's own scratch: creating events
     // may allocate, which the caller-provided scratch path must not
     auto mark = [&]() { return ext_scratch ? hipSuccess : timing_mark(ctx, s); };
 
-    if (!P.covers_all) HIPCK(ctx, launch_zero(d_vattn, (size_t)Lv * DIM * es, s));
+    if (!P.covers_all) HIPCK(ctx, launch_zero(d_rows, (size_t)Lv * DIM * es, s));
     HIPCK(ctx, mark());
 
     PackArgs pa{};
@@ -485,7 +505,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.tsrc_bytes = (uint32_t)std::min<size_t>((size_t)P.txt_len * QKV * es, 0xffffffffu);
     sa.items = g->d_items; sa.cumf = g->d_cumf; sa.vidx = g->d_vidx; sa.tile_base = g->d_tile_base;
     sa.sched_start = g->d_sched_start; sa.sched_desc = g->d_sched_desc; sa.n_slots = P.n_slots; sa.n_used_slots = P.n_used_slots;
-    sa.vattn = d_vattn; sa.vattn_bytes = (uint32_t)((size_t)Lv * DIM * es);
+    sa.vattn = d_rows; sa.vattn_bytes = (uint32_t)((size_t)Lv * DIM * es);
     sa.tpart = reinterpret_cast<float*>(base + lay.off_t);
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;
     sa.n_tiles = P.n_tiles; sa.n_items = P.n_items; sa.nwin = P.nwin;
@@ -495,6 +515,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.nk_v = d_nk_v; sa.nk_t = d_nk_t;
     sa.eps = eps; sa.qscale = pa.qscale;
     HIPCK(ctx, launch_sdpa(dtype, sa, s));
+    if (in_place) HIPCK(ctx, hipMemcpyAsync(d_vattn, d_rows, (size_t)Lv * DIM * es, hipMemcpyDeviceToDevice, s));
     HIPCK(ctx, mark());
 
     HIPCK(ctx, launch_coalesce(dtype, sa.tpart, d_tattn, P.nwin, P.txt_len, s));
@@ -677,7 +698,7 @@ int awa_geom_build(awa_ctx* ctx, int t, int h, int w, const int32_t num_windows[
     }
     // the op's scratch for this geometry (bf16 storage), so that a first
     // awa_forward under stream capture does not allocate
-    if (rc == AWA_OK) rc = ensure_scratch(ctx, op_scratch_bytes(P, AWA_BF16));
+    if (rc == AWA_OK) rc = ensure_scratch(ctx, op_scratch_bytes(P, AWA_BF16, false));
     if (rc != AWA_OK) {
         free_geom_buffers(g);
         delete g;
@@ -789,7 +810,7 @@ int geom_inject(awa_ctx* ctx, const char* who, const std::vector<int32_t>& cumf,
     }
     if (rc == AWA_OK) rc = upload_plan(ctx, g, s);
     if (rc == AWA_OK) step(hipStreamSynchronize(s));
-    if (rc == AWA_OK) rc = ensure_scratch(ctx, op_scratch_bytes(P, AWA_BF16));
+    if (rc == AWA_OK) rc = ensure_scratch(ctx, op_scratch_bytes(P, AWA_BF16, false));
     if (rc != AWA_OK) {
         if (e != hipSuccess) set_err(ctx, "%s: %s", who, hipGetErrorString(e));
         free_geom_buffers(g);
@@ -1000,7 +1021,8 @@ int awa_reserve(awa_ctx* ctx, const awa_geom* g, int dtype) {
         return AWA_EARG;
     }
     DeviceGuard dg(ctx->device);
-    return ensure_scratch(ctx, op_scratch_bytes(g->plan, dtype));
+    // fp32: room for the rows of a call in place too
+    return ensure_scratch(ctx, op_scratch_bytes(g->plan, dtype, dtype == AWA_F32));
 }
 
 int awa_timing_enable(awa_ctx* ctx, int enable) {

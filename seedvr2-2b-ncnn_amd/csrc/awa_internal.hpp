@@ -304,8 +304,10 @@ int check_forward_args(const char* who, awa_ctx* ctx, const awa_geom* g, int dty
                        const void* d_vattn, const void* d_tattn);
 // Bytes of scratch the op needs for a geometry and storage type: the packed
 // tiles (bf16 Q and K; fp32 K and V, with their factors), then the per-window
-// text partials, each 256-byte aligned.
-size_t op_scratch_bytes(const GeomPlan& P, int dtype);
+// text partials, each 256-byte aligned; and the video rows of a call in place.
+size_t op_scratch_bytes(const GeomPlan& P, int dtype, bool in_place);
+// Whether vattn lies (partly) over vqkv or tqkv.
+bool op_in_place(const GeomPlan& P, int dtype, const void* d_vqkv, const void* d_tqkv, const void* d_vattn);
 // awa_forward without argument checks (shared with the block).  ext_scratch:
 // nullptr uses the context's scratch (grown on demand, per-phase events when
 // timing is on); otherwise a caller-provided device buffer of at least

@@ -61,7 +61,8 @@ extern "C" int awa_forward_noalloc(awa_ctx* ctx, const awa_geom* g, int dtype, c
     const int rc = check_forward_args("awa_forward_noalloc", ctx, g, dtype, d_vqkv, d_tqkv, Lv, TXT,
                                       d_nq_v, d_nk_v, d_nq_t, d_nk_t, eps, d_vattn, d_tattn);
     if (rc != AWA_OK) return rc;
-    const size_t need = op_scratch_bytes(g->plan, dtype);
+    const size_t need =
+        op_scratch_bytes(g->plan, dtype, op_in_place(g->plan, dtype, d_vqkv, d_tqkv, d_vattn));
     if (need > kScratchBytes) {
         set_err(ctx,
                 "awa_forward_noalloc: this geometry needs %zu bytes of scratch (%s storage); the "

@@ -1,0 +1,33 @@
+"""Outputs that lie over inputs: the same bits as into buffers of their own.
+
+The attention kernels read rows of vqkv and tqkv while other workgroups write
+vattn, so those rows take another way then.
+"""
+import pytest
+
+from conftest import seeded_awa_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("over", ["vqkv", "tqkv"])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_op_in_place(ctx, dtype, over, noalloc):
+    import torch
+    h, w, txt = 30, 41, 77
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    geom = ctx.build_geometry(1, h, w, (1, 4, 4), txt, 1)
+    vqkv, tqkv, gains = seeded_awa_inputs(h * w, txt, 21)
+    inputs = {"vqkv": torch.from_numpy(vqkv).cuda().to(dt), "tqkv": torch.from_numpy(tqkv).cuda().to(dt)}
+    gains = [torch.from_numpy(g).cuda() for g in gains]
+    ref = ctx.forward(geom, inputs["vqkv"], inputs["tqkv"], *gains, eps=1e-5, noalloc=noalloc)
+    n, out = inputs[over].numel(), h * w * 2560
+    buf = torch.empty(max(n, out), dtype=dt, device="cuda")
+    buf[:n] = inputs[over].flatten()
+    inputs[over] = buf[:n].view(-1, 7680)
+    got = ctx.forward(geom, inputs["vqkv"], inputs["tqkv"], *gains, eps=1e-5, vattn=buf[:out].view(-1, 2560),
+                      noalloc=noalloc)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+    geom.close()
