@@ -119,9 +119,9 @@ typedef struct {
     const float* vid_out_b;       /* fp32 [64]                                          */
 } dit_io_weights;
 
-/* Prepared input/output layers: padded device copies of vid_in_w (K 132 ->
- * 192) and vid_out_w / vid_out_b (N 64 -> 256) for the block's GEMM kernel;
- * the other pointers are borrowed and must stay valid. */
+/* Prepared input/output layers: device copies of vid_in_w (K padded 132 ->
+ * 160) and vid_out_w in the order in which the kernels read them, and of
+ * vid_out_b; the other pointers are borrowed and must stay valid. */
 typedef struct dit_io dit_io;
 int dit_io_create(awa_ctx* ctx, const dit_io_weights* w, dit_io** out, awa_stream_t stream);
 void dit_io_destroy(awa_ctx* ctx, dit_io* io);
@@ -129,13 +129,15 @@ void dit_io_destroy(awa_ctx* ctx, dit_io* io);
 /* Input layers: patchify the latent grid d_grid fp32 (T, H, W, 33) (H, W even;
  * dit_vk.cpp:717-733), vid_in_proj to the video rows and txt_in of d_txt fp32
  * [TXT][5120] to the text rows of the residual stream d_x fp32
- * [Lv + TXT][2560], Lv = T (H/2) (W/2).  bf16 GEMM inputs, fp32 out. */
+ * [Lv + TXT][2560], Lv = T (H/2) (W/2).  bf16 GEMM inputs, fp32 out.  d_x may
+ * lie over d_grid or d_txt (those are copied first). */
 int dit_embed(awa_ctx* ctx, const dit_io* io, const float* d_grid, int T, int H, int W,
               const float* d_txt, int TXT, float* d_x, awa_stream_t stream);
 
 /* Output layer: RMSNorm of the video rows of d_x with out_norm_w, times
  * (emb[6d+1] + out_ada_scale) plus (emb[6d] + out_ada_shift), vid_out_proj,
- * unpatchified to d_out fp32 (T, H, W, 16) (dit_vk.cpp:735-750). */
+ * unpatchified to d_out fp32 (T, H, W, 16) (dit_vk.cpp:735-750).  d_out may lie
+ * over d_x or d_emb (it is copied there at the end). */
 int dit_final(awa_ctx* ctx, const dit_io* io, const float* d_emb, const float* d_x, int T, int H,
               int W, float eps, float* d_out, awa_stream_t stream);
 

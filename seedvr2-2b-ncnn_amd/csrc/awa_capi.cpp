@@ -434,10 +434,6 @@ struct ScratchLayout {
         rows = align256((size_t)P.Lv * DIM * elem_size(dtype));
     }
 };
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    return x < y + nb && y < x + na;
-}
 }  // namespace
 
 size_t op_scratch_bytes(const GeomPlan& P, int dtype, bool in_place) {

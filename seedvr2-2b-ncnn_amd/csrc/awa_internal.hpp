@@ -302,6 +302,11 @@ int check_forward_args(const char* who, awa_ctx* ctx, const awa_geom* g, int dty
                        const void* d_vqkv, const void* d_tqkv, int Lv, int TXT, const float* d_nq_v,
                        const float* d_nk_v, const float* d_nq_t, const float* d_nk_t, float eps,
                        const void* d_vattn, const void* d_tattn);
+// Whether the na bytes at a and the nb bytes at b share any.
+inline bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+}
 // Bytes of scratch the op needs for a geometry and storage type: the packed
 // tiles (bf16 Q and K; fp32 K and V, with their factors), then the per-window
 // text partials, each 256-byte aligned; and the video rows of a call in place.

@@ -93,7 +93,15 @@ void dit_io_destroy(awa_ctx* ctx, dit_io* io) {
 
 namespace {
 // workspace bytes of each entry point (the offsets below follow the same layouts)
-size_t embed_ws_bytes(int TXT) { return (size_t)EMBED_TXT_SPLIT * TXT * DIM * 4; }
+// embed: the text's partial products, then copies of inputs that d_x lies over
+size_t embed_part_bytes(int TXT) { return align256((size_t)EMBED_TXT_SPLIT * TXT * DIM * 4); }
+size_t grid_bytes(int Lv) { return (size_t)Lv * 4 * 33 * 4; }
+size_t txt_bytes(int TXT) { return (size_t)TXT * 5120 * 4; }
+size_t embed_ws_bytes(int Lv, int TXT) {
+    return embed_part_bytes(TXT) + align256(grid_bytes(Lv)) + align256(txt_bytes(TXT));
+}
+// final: the output, if it lies over x or the embedding
+size_t final_ws_bytes(int Lv) { return (size_t)Lv * VID_OUT * 4; }
 size_t layer_ws_bytes(int M, int mlp) {
     return align256(12 * DIM * 4) + align256((size_t)M * DIM * 2) + align256((size_t)M * QKV * 2) +
            align256((size_t)M * DIM * 2) + align256((size_t)M * mlp * 2);
@@ -109,7 +117,7 @@ int dit_reserve(awa_ctx* ctx, const awa_geom* g, int mlp) {
     const int Lv = g->plan.Lv, TXT = g->plan.txt_len;
     DeviceGuard dg(ctx->device);
     HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes,
-                             std::max(layer_ws_bytes(Lv + TXT, mlp), embed_ws_bytes(TXT))));
+                             std::max(layer_ws_bytes(Lv + TXT, mlp), std::max(embed_ws_bytes(Lv, TXT), final_ws_bytes(Lv)))));
     return awa_reserve(ctx, g, AWA_BF16);
 }
 
@@ -127,8 +135,21 @@ int dit_embed(awa_ctx* ctx, const dit_io* io, const float* d_grid, int T, int H,
     a.vid_w = io->vid_in_w; a.vid_b = io->vid_in_b;
     a.txt = d_txt; a.txt_w = io->txt_in_w; a.txt_b = io->txt_in_b;
     a.x = d_x;
-    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, embed_ws_bytes(TXT)));
+    HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, embed_ws_bytes(a.Lv, TXT)));
     a.part = static_cast<float*>(ctx->ws);
+    // workgroups write x while others still read the inputs: those under x are
+    // copied first
+    char* copy = static_cast<char*>(ctx->ws) + embed_part_bytes(TXT);
+    const size_t x_bytes = (size_t)(a.Lv + TXT) * DIM * 4;
+    if (overlaps(d_x, x_bytes, d_grid, grid_bytes(a.Lv))) {
+        HIPCK(ctx, hipMemcpyAsync(copy, d_grid, grid_bytes(a.Lv), hipMemcpyDeviceToDevice, s));
+        a.grid = reinterpret_cast<const float*>(copy);
+        copy += align256(grid_bytes(a.Lv));
+    }
+    if (overlaps(d_x, x_bytes, d_txt, txt_bytes(TXT))) {
+        HIPCK(ctx, hipMemcpyAsync(copy, d_txt, txt_bytes(TXT), hipMemcpyDeviceToDevice, s));
+        a.txt = reinterpret_cast<const float*>(copy);
+    }
     HIPCK(ctx, launch_embed(a, s));
     return AWA_OK;
 }
@@ -148,7 +169,17 @@ int dit_final(awa_ctx* ctx, const dit_io* io, const float* d_emb, const float* d
     a.rows = T * (H / 2) * (W / 2); a.H = H; a.W2 = W / 2;
     a.eps = eps;
     a.out = d_out;
+    // workgroups write out while others still read x and the embedding: over
+    // those the output goes through the workspace
+    const size_t out_bytes = final_ws_bytes(a.rows);
+    const bool in_place = overlaps(d_out, out_bytes, d_x, (size_t)a.rows * DIM * 4) ||
+                          overlaps(d_out, out_bytes, d_emb, (size_t)DIT_EMB * 4);
+    if (in_place) {
+        HIPCK(ctx, ensure_buffer(&ctx->ws, &ctx->ws_bytes, out_bytes));
+        a.out = static_cast<float*>(ctx->ws);
+    }
     HIPCK(ctx, launch_final(a, s));
+    if (in_place) HIPCK(ctx, hipMemcpyAsync(d_out, a.out, out_bytes, hipMemcpyDeviceToDevice, s));
     return AWA_OK;
 }
 

@@ -31,3 +31,42 @@ def test_op_in_place(ctx, dtype, over, noalloc):
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
     geom.close()
+
+
+@pytest.mark.parametrize("over", ["grid", "txt"])
+def test_embed_in_place(ctx, over):
+    import torch
+    from test_dit_ends_gpu import make_io
+    g = torch.Generator(device="cuda").manual_seed(5)
+    _, io = make_io(ctx, g)
+    h, w, txt = 40, 50, 90
+    inputs = {"grid": torch.randn((1, 2 * h, 2 * w, 33), generator=g, device="cuda"),
+              "txt": torch.randn((txt, 5120), generator=g, device="cuda")}
+    ref = ctx.embed(io, inputs["grid"], inputs["txt"])
+    buf = torch.empty(ref.numel(), device="cuda")
+    x, n = inputs[over], inputs[over].numel()
+    buf[-n:] = x.flatten()  # under the last rows written
+    inputs[over] = buf[-n:].view(x.shape)
+    got = ctx.embed(io, inputs["grid"], inputs["txt"], x=buf.view(ref.shape))
+    assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("over", ["x", "emb"])
+def test_final_in_place(ctx, over):
+    import torch
+    from test_dit_ends_gpu import make_io
+    g = torch.Generator(device="cuda").manual_seed(6)
+    _, io = make_io(ctx, g)
+    h, w = 40, 50
+    x = torch.randn((h * w, 2560), generator=g, device="cuda")
+    emb = torch.randn(6 * 2560, generator=g, device="cuda") * 0.02
+    ref = ctx.final(io, emb, x, 1, 2 * h, 2 * w)
+    n = ref.numel()
+    if over == "x":
+        out = x.view(-1)[-n:]
+    else:
+        buf = torch.empty(n, device="cuda")
+        buf[n // 2:n // 2 + emb.numel()] = emb
+        emb, out = buf[n // 2:n // 2 + emb.numel()], buf
+    got = ctx.final(io, emb, x, 1, 2 * h, 2 * w, out=out.view(ref.shape))
+    assert torch.equal(got, ref)
