@@ -429,8 +429,9 @@ def test_model_directory_errors(ctx, awa, tmp_path):
     assert "null stream" in awa.lib().awa_last_error(ctx.ptr).decode()
 
 
-# shapes that fall to each tile form of the GEMM (256 x 256 and 256 x 224, 256 x 128,
-# 128 x 256, 128 x 128, 128 x 64), with row counts at and around their edges
+# shapes that fall to each tile form of the GEMM (256 x 256, 256 x 224, 256 x 160,
+# 256 x 128, 128 x 256, 128 x 192, 128 x 128, 128 x 64), with row counts at and
+# around their edges
 @pytest.mark.parametrize("N,K", [(2560, 2560), (7680, 2560), (13824, 2560), (2560, 6912), (256, 64)])
 def test_gemm_tile_forms_agree(ctx, N, K):
     """Every tile form sums an output's products in the same order (K steps of 32 in
@@ -447,3 +448,54 @@ def test_gemm_tile_forms_agree(ctx, N, K):
     assert float((full[-300:].float() - ref).norm() / ref.norm()) <= 2.0 ** -8
     for M in (1, 63, 64, 65, 128, 257, 679, 897, 1418, 2778, 3100):
         assert torch.equal(ctx.gemm(A[:M].contiguous(), W), full[:M]), M
+
+
+@pytest.fixture(scope="module")
+def frame_layers(ctx):
+    """A layer's weights, 18 frames of 300 rows with 20 text rows, and each frame's
+    result by itself (the smallest tiles), for dual and shared branches."""
+    import torch
+    txt, mlp, n = 20, 2048, 18
+    g = torch.Generator(device="cuda").manual_seed(77)
+    r = lambda *s, scale=0.02: torch.randn(s, generator=g, device="cuda") * scale
+
+    def branch():
+        b = {k: r(*s).bfloat16() for k, s in (("qkv_w", (7680, 2560)), ("out_w", (2560, 2560)), ("mlp_out_w", (2560, mlp)))}
+        b["mlp_w"] = ctx.pack_mlp(r(mlp, 2560).bfloat16(), r(mlp, 2560).bfloat16())
+        b.update(out_b=r(2560), nq=1 + r(128), nk=1 + r(128))
+        for k in ("attn_shift", "attn_scale", "attn_gate", "mlp_shift", "mlp_scale", "mlp_gate"):
+            b[k] = r(2560, scale=0.5 if "gate" in k else 0.02) + ("scale" in k)
+        return b
+
+    vid, text = branch(), branch()
+    emb = r(6 * 2560)
+    frames, trows = r(n, 300, 2560, scale=1.0), r(txt, 2560, scale=1.0)
+
+    def run(tb, t0, t1):
+        nt = t1 - t0
+        geom = ctx.build_geometry(nt, 15, 20, (nt, 1, 1), txt, 0)  # a window per frame
+        assert geom.info()["nwin"] == nt
+        x = torch.cat([frames[t0:t1].reshape(-1, 2560), trows])
+        ctx.layer(geom, vid, tb, emb, x, 300 * nt, txt, mlp=mlp)
+        geom.close()
+        return x[:300 * nt].view(nt, 300, 2560)
+
+    alone = {k: torch.cat([run(tb, t, t + 1) for t in range(n)]) for k, tb in (("dual", text), ("shared", vid))}
+    return lambda kind, nt: run(text if kind == "dual" else vid, 0, nt), alone
+
+
+@pytest.mark.parametrize("kind", ["dual", "shared"])
+@pytest.mark.parametrize("frames", [2, 3, 5, 6, 7, 8, 10, 11, 12, 13, 16, 18])
+def test_layer_tile_forms_agree(frame_layers, kind, frames):
+    """The fused epilogues (residual, SwiGLU) in every tile form: the video rows of
+    a frame do not depend on the other frames (a window each, the same RoPE), nor
+    do their bits on the tiles.  On 256 CUs the residual GEMMs take 128 x 64 at 2
+    frames, 128 x 128 at 3 and 5, 128 x 192 at 6 and 7, 128 x 256 at 8 and 10
+    (shared), 256 x 128 at 10 (dual), 256 x 160 at 11 to 13, 256 x 224 at 16, 256 x
+    256 at 18 (dual); SwiGLU 128 x 128 at 2 and 3, 128 x 256 at 5 (dual) and 6
+    (shared), 256 x 128 at 6 (dual), 256 x 160 at 7 and 8, 256 x 224 at 11, 256 x
+    256 at 12, 128 x 192 at 10 (shared)."""
+    import torch
+    note(f"layer tile forms {kind} {frames}")
+    run, alone = frame_layers
+    assert torch.equal(run(kind, frames), alone[kind][:frames])
