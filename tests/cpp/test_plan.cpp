@@ -1,4 +1,4 @@
-// test_plan.cpp — the host planner of the bf16 attention kernel (awa::plan_tiles,
+// test_plan.cpp — the host planner of the attention kernels (awa::plan_tiles,
 // awa::plan_schedule in seedvr2-2b-ncnn_amd/csrc/awa_capi.cpp) on the CPU.
 //
 // Usage: test_plan t h w nw_t nw_h nw_w txt shifted n_slots [empty_at]
@@ -8,7 +8,12 @@
 // schedule, then checks:
 //   - every (head, work item) appears in exactly one slot, once;
 //   - every descriptor matches its item (window, query tiles, tile ranges);
-//   - all items of one (window, head) sit on slots of one XCD (slot % 8);
+//   - all items of one (window, head) sit on slots of one XCD (slot % 8), and
+//     no slot past n_used_slots has any;
+//   - the fp32 kernel's workgroups (f32_work): every (head, query tile) once, all
+//     of one (window, head) on one XCD (entry % 8), longest windows first and
+//     idle entries last on each; single query tiles if and only if those fit
+//     one workgroup per CU (two slots);
 //   - the kernel's DMA stream (stream_tiles, stream_tile, stream_fetch): in
 //     every slot, replaying the prologue and each tile's fetch into the K
 //     ring (3 slots) and the V ring (2 slots), the tile an item reads at key
@@ -97,6 +102,53 @@ int main(int argc, char** argv) {
     }
     for (size_t i = 0; i < seen.size(); i++)
         if (seen[i] != 1) return fail("item not scheduled", (long)i, seen[i]);
+
+    if (P.n_used_slots % 8 != 0 || P.n_used_slots < 8 || P.n_used_slots > S)
+        return fail("used slot count", P.n_used_slots, S);
+    int last_used = 0;
+    for (int s = 0; s < S; s++)
+        if (P.sched_start[s + 1] > P.sched_start[s]) last_used = s;
+    if (last_used / 8 != P.n_used_slots / 8 - 1) return fail("used slots", last_used, P.n_used_slots);
+
+    // fp32: sched_desc number and part of each entry
+    std::vector<int> q_seen((size_t)NI * H * 2, 0);
+    std::vector<long> prev(8, 1L << 40), tiles_on(8, 0);
+    std::vector<char> idle(8, 0);
+    bool singles = false, pairs = false;
+    group_xcd.clear();
+    if (P.f32_work.empty() || P.f32_work.size() % 8 != 0) return fail("f32 list size", (long)P.f32_work.size(), 0);
+    for (size_t b = 0; b < P.f32_work.size(); b++) {
+        const int e = P.f32_work[b], x = (int)(b % 8);
+        if (e < 0) { idle[x] = 1; continue; }
+        if (idle[x]) return fail("f32 entry after an idle one", (long)b, e);
+        const int k = e >> 2, part = e & 3;
+        if (k >= NI * H || part > 2) return fail("f32 entry", (long)b, e);
+        const int32_t* d = &P.sched_desc[(size_t)k * 8];
+        const bool two = d[2] >= 0;
+        if (part && !two) return fail("f32 part of a single tile", (long)b, e);
+        if (part) singles = true;
+        else if (two) pairs = true;
+        for (int t = 0; t < 2; t++)
+            if (part ? t == part - 1 : (t == 0 || two)) {
+                if (q_seen[(size_t)k * 2 + t]++) return fail("f32 query tile twice", k, t);
+                tiles_on[x]++;
+            }
+        const long g = (long)(d[0] >> 8) * H + (d[0] & 255), nk = awa::stream_tiles(d[5], P.ntt);
+        auto it = group_xcd.find(g);
+        if (it == group_xcd.end()) group_xcd[g] = x;
+        else if (it->second != x) return fail("f32 group split over XCDs", g, (long)b);
+        if (nk > prev[x]) return fail("f32 order", (long)b, nk);
+        prev[x] = nk;
+    }
+    for (int k = 0; k < NI * H; k++)
+        for (int t = 0; t < 2; t++)
+            if (q_seen[(size_t)k * 2 + t] != (t == 0 || P.sched_desc[(size_t)k * 8 + 2] >= 0))
+                return fail("f32 query tile missing", k, t);
+    const long single_len = *std::max_element(tiles_on.begin(), tiles_on.end()) * 8;
+    if (singles && pairs) return fail("f32 forms mixed", 0, 0);
+    if (singles && single_len * 2 > S) return fail("f32 single tiles on a full device", single_len, S);
+    if (pairs && single_len * 2 <= S) return fail("f32 pairs where single tiles fit", single_len, S);
+    std::printf("f32 entries %zu %s\n", P.f32_work.size(), singles ? "single" : "pairs");
 
     // The DMA stream of every slot, replayed as the kernel issues it: a ring
     // entry is (head, tile); -1 marks a fetch past the slot's last item (an

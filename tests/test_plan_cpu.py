@@ -8,7 +8,8 @@ worse than plain longest-first (on the 1080p unshifted layer, where first fit
 decreasing packs the few item sizes better, strictly lower), and the kernel's
 DMA stream replayed slot by slot: every key tile an item reads is the one its
 fetch two (K) or one (V) tiles earlier put into the ring, including items of
-a window without video rows (one text tile of its own, padded to two).
+a window without video rows (one text tile of its own, padded to two); and the
+fp32 kernel's list of workgroups, either side of its single-tile rule.
 """
 import os
 import re
@@ -90,3 +91,12 @@ def test_schedule_on_random_shapes(driver):
     for t, h, w, nw, txt, sh in random_shapes():
         mk, lpt, mean = run(driver, t, h, w, nw, txt, sh, 512)
         assert mk <= lpt and mk >= mean, (t, h, w, nw, txt, sh)
+
+
+@pytest.mark.parametrize("slots,form", [(512, "single"), (240, "single"), (232, "pairs"), (8, "pairs")])
+def test_f32_single_tiles_at_their_edge(driver, slots, form):
+    """12 x 20 rows with 9 text rows are one window of five query tiles; three of the
+    20 heads share an XCD, so 8 x 15 entries of one tile need 240 slots."""
+    r = subprocess.run([driver] + "1 12 20 1 2 2 9 0".split() + [str(slots)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip().endswith("rc=0"), r.stdout[-2000:] + r.stderr[-2000:]
+    assert re.search(r"f32 entries \d+ (\w+)", r.stdout).group(1) == form, r.stdout
