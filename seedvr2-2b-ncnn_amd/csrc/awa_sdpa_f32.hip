@@ -132,24 +132,6 @@ __device__ inline void dma_quarter(const void* unit, uint32_t part, uint32_t lan
 // This wave's DMA has landed and its LDS reads are done, then the barrier.
 __device__ inline void unit_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Eighteen wait states between MFMAs and the first use of their results, tied to
-// the registers (the compiler places the eight or so that this MFMA needs by
-// itself; next to a unit's MFMAs the rest is nothing).
-template <int N>
-__device__ inline void mfma_fence(f32x4 (&s)[N][1]) {
-#pragma unroll
-    for (int i = 0; i < N; i += 2)
-        asm volatile("s_nop %c2" : "+v"(s[i][0]), "+v"(s[i + 1][0]) : "n"(i ? 0 : 15));
-    asm volatile("s_nop 1");
-}
-template <int N>
-__device__ inline void mfma_fence(f32x4 (&s)[N][2]) {
-#pragma unroll
-    for (int i = 0; i < N; i += 2)
-        asm volatile("s_nop %c4" : "+v"(s[i][0]), "+v"(s[i][1]), "+v"(s[i + 1][0]), "+v"(s[i + 1][1]) : "n"(i ? 0 : 15));
-    asm volatile("s_nop 1");
-}
-
 // ---- windows whose V the split does not hold (SPREAD_CHANNELS): fp32 MFMAs
 //
 // The same workgroup and the same output for its query tile t, 16 queries a wave, as
@@ -560,7 +542,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
 #pragma unroll
         for (int qb = 0; qb < NQ; qb++) up |= mloc[qb] > m_i[qb] + M_STALE;
         if (!__any(up)) return;
-        mfma_fence(oacc);
 #pragma unroll
         for (int qb = 0; qb < NQ; qb++) {
             const float m_new = fmaxf(m_i[qb], mloc[qb]);
@@ -616,7 +597,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        mfma_fence(sn);
         mask(sn, un);
         f16x8 ph[NQ], pl[NQ];
 #pragma unroll
@@ -659,7 +639,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
             if (st < 3) read_k(0, st + 1);
             score_step(s[0], st);
         }
-        mfma_fence(s[0]);
         mask(s[0], ubeg);
         float mloc[NQ];
 #pragma unroll
@@ -679,7 +658,6 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
     // not held in registers across the loop
     int ln = lane;
     asm volatile("" : "+v"(ln));
-    mfma_fence(oacc);
     float l[NQ];
 #pragma unroll
     for (int qb = 0; qb < NQ; qb++) l[qb] = sum4(l_i[qb]);

@@ -282,10 +282,10 @@ def test_m0_written_only_by_the_kernels_asm(sdpa_asm):
 # Wait states a read needs after the write of its register (gfx950), as the
 # compiler inserts them for its own instructions: a VALU, memory or MFMA
 # source read of a v_mfma_f32_32x32x16_bf16 result 12 (s_nop 11), of a
-# v_mfma_f32_16x16x32_bf16 result 8, of a v_mfma_f32_32x32x2_f32 result 18;
+# v_mfma_f32_16x16x32_bf16 (or _f16) result 8, of a v_mfma_f32_32x32x2_f32 result 18;
 # a read of a transcendental result one.
 MFMA_READ_WAIT = {"v_mfma_f32_32x32x16_bf16": 12, "v_mfma_f32_16x16x32_bf16": 8, "v_mfma_f32_32x32x2_f32": 18,
-                  "v_mfma_f32_16x16x4_f32": 10}
+                  "v_mfma_f32_16x16x32_f16": 8, "v_mfma_f32_16x16x4_f32": 10}
 TRANS_READ_WAIT = 1
 VREG = re.compile(r"\b([va])\[(\d+):(\d+)\]|\b([va])(\d+)\b")
 TRANS = re.compile(r"^v_(exp|log|rcp|rsq|sqrt|sin|cos)_f32")
@@ -416,10 +416,10 @@ def test_mfma_results_read_after_enough_wait_states(sdpa_asm):
     assert not any("v255, v255" in ins for _, ins, _ in wait_state_violations(fenced))
 
 
-@pytest.mark.parametrize("src", ["awa_sdpa_f32", "dit_gemm"])
+@pytest.mark.parametrize("src", ["awa_sdpa_f32", "dit_gemm", "dit_ends"])
 def test_other_mfma_kernels_wait_states(tmp_path, src):
     """The same wait-state check over the library's other MFMA kernels (the
-    fp32 attention kernel and every GEMM instantiation), whose epilogues read
+    fp32 attention kernel, every GEMM instantiation and the ends), whose epilogues read
     accumulators after asm fences."""
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not present")
