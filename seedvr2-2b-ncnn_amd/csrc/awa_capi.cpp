@@ -89,7 +89,7 @@ hipError_t dalloc(T** p, size_t n) {
 
 void free_geom_buffers(awa_geom* g) {
     void* ptrs[] = {g->d_slices, g->d_cumf, g->d_vidx, g->d_tile_base, g->d_tile_win,
-                    g->d_items, g->d_f32_work, g->d_sched_start, g->d_sched_desc, g->d_vfreq, g->d_tfreq,
+                    g->d_f32_work, g->d_sched_start, g->d_sched_desc, g->d_vfreq, g->d_tfreq,
                     g->d_vcs, g->d_tcs, g->d_tile_meta, g->d_vrow};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -316,7 +316,6 @@ int upload_plan(awa_ctx* ctx, awa_geom* g, hipStream_t s) {
                                   hipMemcpyHostToDevice, s));
     HIPCK(ctx, dalloc(&g->d_tile_base, P.tile_base.size()));
     HIPCK(ctx, dalloc(&g->d_tile_win, P.tile_win.size()));
-    HIPCK(ctx, dalloc(&g->d_items, P.items.size()));
     HIPCK(ctx, dalloc(&g->d_f32_work, P.f32_work.size()));
     if (!P.f32_work.empty())
         HIPCK(ctx, hipMemcpyAsync(g->d_f32_work, P.f32_work.data(), P.f32_work.size() * 4,
@@ -325,9 +324,6 @@ int upload_plan(awa_ctx* ctx, awa_geom* g, hipStream_t s) {
                               hipMemcpyHostToDevice, s));
     if (!P.tile_win.empty())
         HIPCK(ctx, hipMemcpyAsync(g->d_tile_win, P.tile_win.data(), P.tile_win.size() * 4,
-                                  hipMemcpyHostToDevice, s));
-    if (!P.items.empty())
-        HIPCK(ctx, hipMemcpyAsync(g->d_items, P.items.data(), P.items.size() * 4,
                                   hipMemcpyHostToDevice, s));
     HIPCK(ctx, dalloc(&g->d_tile_meta, P.tile_meta.size()));
     HIPCK(ctx, hipMemcpyAsync(g->d_tile_meta, P.tile_meta.data(), P.tile_meta.size() * 4,
@@ -499,12 +495,12 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.vrow = g->d_vrow; sa.vsrc = d_vqkv; sa.tsrc = d_tqkv;
     sa.vsrc_bytes = (uint32_t)std::min<size_t>((size_t)Lv * QKV * es, 0xffffffffu);
     sa.tsrc_bytes = (uint32_t)std::min<size_t>((size_t)P.txt_len * QKV * es, 0xffffffffu);
-    sa.items = g->d_items; sa.cumf = g->d_cumf; sa.vidx = g->d_vidx; sa.tile_base = g->d_tile_base;
+    sa.vidx = g->d_vidx;
     sa.sched_start = g->d_sched_start; sa.sched_desc = g->d_sched_desc; sa.n_slots = P.n_slots; sa.n_used_slots = P.n_used_slots;
     sa.vattn = d_rows; sa.vattn_bytes = (uint32_t)((size_t)Lv * DIM * es);
     sa.tpart = reinterpret_cast<float*>(base + lay.off_t);
-    sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_sets = P.txt_sets; sa.txt_len = P.txt_len;
-    sa.n_tiles = P.n_tiles; sa.n_items = P.n_items; sa.nwin = P.nwin;
+    sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_len = P.txt_len;
+    sa.n_tiles = P.n_tiles;
     sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size();
     sa.kexp = pa.kexp; sa.vexp = pa.vexp;
     sa.tile_meta = g->d_tile_meta; sa.vcs = g->d_vcs; sa.tcs = g->d_tcs; sa.nq_v = d_nq_v; sa.nq_t = d_nq_t;

@@ -7,11 +7,11 @@
 // Per head h and tile k the packed buffers hold
 //   Qp[h][k][slot 0..63][d 0..127]   normalised + rotated queries
 //   Kp[h][k][slot 0..63][d 0..127]   normalised + rotated keys
-// in bf16.  Unused slots are zero.  Queries carry the softmax scale times
+// in bf16, unused slots zero.  Queries carry the softmax scale times
 // log2(e), so scores come out in log2 units.  The bf16 attention kernel reads V
 // from vqkv / tqkv itself, through the geometry's row table
 // (awa_geom::d_vrow).  For fp32 storage only K and V are packed, as split fp16
-// tiles in fragment order (f32_kfrag).
+// tiles in fragment order (f32_kfrag); unused slots repeat the window's last row.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -271,7 +271,6 @@ struct awa_geom {
     int32_t* d_vidx = nullptr;
     int32_t* d_tile_base = nullptr;
     int32_t* d_tile_win = nullptr;
-    int32_t* d_items = nullptr;
     int32_t* d_f32_work = nullptr;  // GeomPlan::f32_work
     int32_t* d_sched_start = nullptr;
     int32_t* d_sched_desc = nullptr;
@@ -370,18 +369,14 @@ struct SdpaArgs {
     const void* vsrc;            // bf16 kernel: vqkv and tqkv, whose V columns it reads
     const void* tsrc;
     uint32_t vsrc_bytes, tsrc_bytes;
-    const int32_t* items;
-    const int32_t* cumf;
     const int32_t* vidx;
-    const int32_t* tile_base;
     const int32_t* sched_start;  // bf16 kernel: persistent schedule (GeomPlan)
     const int32_t* sched_desc;
     int n_slots, n_used_slots;
     void* vattn;
     uint32_t vattn_bytes;  // bf16 kernel: size of vattn (buffer stores drop beyond it)
     float* tpart;          // [nwin][txt_len][2560] fp32 text partials
-    int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles, n_items, nwin;
-    float scale_log2e;     // multiplier of the scores (1 when Q carries the scale)
+    int n_vid_tiles, ntt, txt_len, n_tiles;
     // fp32 kernel: its workgroups, the packed blocks' factors, and what the
     // rows' normalisation and rotation need (as in PackArgs)
     const int32_t* f32_work;

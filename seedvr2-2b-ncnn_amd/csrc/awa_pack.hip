@@ -52,14 +52,9 @@ template <> struct Io<float> {
     static __device__ inline Raw load(const float* p) {
         return {*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4)};
     }
-    static __device__ inline Raw zero() { return {make_float4(0, 0, 0, 0), make_float4(0, 0, 0, 0)}; }
     static __device__ inline void widen(const Raw& r, float* x) {
         x[0] = r.a.x; x[1] = r.a.y; x[2] = r.a.z; x[3] = r.a.w;
         x[4] = r.b.x; x[5] = r.b.y; x[6] = r.b.z; x[7] = r.b.w;
-    }
-    static __device__ inline void store8(float* p, const float* x) {
-        *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
-        *reinterpret_cast<float4*>(p + 4) = make_float4(x[4], x[5], x[6], x[7]);
     }
 };
 
