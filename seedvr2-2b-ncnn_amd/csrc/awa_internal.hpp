@@ -108,13 +108,16 @@ __device__ inline float max4(float v) {
 // of its blocks, nor a block than the others of its window.  The pack kernel
 // marks a block wide (VEXP_WIDE in place of its exponent) if the largest value
 // of a channel, zero channels aside, is over 2^SPREAD_CHANNELS below the block's
-// largest (whole blocks only: one or two rows hold small values by chance), if
-// the block lies below the scales' range, or if its K or V holds an infinity
-// (which splits into infinity and NaN; a NaN stays one either way); the attention kernel takes the
-// fp32 MFMAs for a window with a wide block, with blocks over 2^SPREAD_BLOCKS
-// apart or without any whole block.
+// largest (whole blocks only: one or two rows hold small values by chance); the
+// attention kernel takes operands of three bf16 values for a window with a wide
+// block, with blocks over 2^SPREAD_BLOCKS apart or without any whole block.
+// VEXP_FULL marks a block with an infinity in K or V (which splits into infinity
+// and NaN; a NaN stays one either way) or with values at the ends of fp32's
+// range (2^127, where a bf16 may round to infinity; below 2^SPLIT_FLOOR_V, the
+// channels of a wide block too, whose last bits would be subnormal): its windows
+// take fp32 MFMAs.
 constexpr int SPREAD_CHANNELS = 10, SPREAD_BLOCKS = 6;
-constexpr float VEXP_WIDE = 1000.f, VEXP_ZERO = -1000.f;
+constexpr float VEXP_WIDE = 1000.f, VEXP_FULL = 2000.f, VEXP_ZERO = -1000.f;
 
 // Fragment order of a packed fp32 tile (32 fragments of 1 KiB, lane l's 16 bytes
 // at 16 l), by 32-key halves of 16 KiB.  K: key block b (16 keys), k32 step s of
@@ -353,7 +356,7 @@ struct PackArgs {
     void* Kp;
     void* Vp;              // fp32 storage only (the bf16 attention reads V from vqkv / tqkv)
     // fp32 storage: [HEADS][n_tiles][4], of each 16-row block with split_scale 2^a: 2^-a of K; -a of V,
-    // VEXP_ZERO of a block of zeros, VEXP_WIDE of one that the split does not hold
+    // VEXP_ZERO of a block of zeros, VEXP_WIDE or VEXP_FULL of one that the split does not hold
     float *kexp, *vexp;
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles;
     float eps;

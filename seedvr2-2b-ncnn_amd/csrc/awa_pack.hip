@@ -313,10 +313,13 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         };
         const float km = block_max(2 * tid), vm = block_max(2 * tid + 1);
         const float vn = fminf(fminf(mns[0][tid], mns[1][tid]), fminf(mns[2][tid], mns[3][tid]));
+        const bool whole = nvalid >= 16 * (b + 1);
         float ve = (float)(exponent(vm) - 14);
-        if (exponent(vm) < SPLIT_FLOOR_V || exponent(vm) == 128 || (nvalid >= 16 * (b + 1) && exponent(vn) < exponent(vm) - SPREAD_CHANNELS))
-            ve = VEXP_WIDE;
-        a.vexp[ht * 4 + b] = exponent(km) == 128 ? VEXP_WIDE : vm == 0.f ? VEXP_ZERO : ve;
+        if (whole && exponent(vn) < exponent(vm) - SPREAD_CHANNELS)
+            ve = exponent(vn) < SPLIT_FLOOR_V ? VEXP_FULL : VEXP_WIDE;
+        if (vm == 0.f) ve = VEXP_ZERO;
+        else if (exponent(vm) < SPLIT_FLOOR_V || exponent(vm) >= 127) ve = VEXP_FULL;
+        a.vexp[ht * 4 + b] = exponent(km) >= 127 ? VEXP_FULL : ve;
         a.kexp[ht * 4 + b] = 1.f / split_scale(km, SPLIT_FLOOR_QK);
     }
 }

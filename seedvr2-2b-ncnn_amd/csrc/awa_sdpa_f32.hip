@@ -20,11 +20,12 @@
 // the largest.  They are undone exactly: in the factor of the scores, in P
 // before its split, and in the normalisation of O.  P = exp2(s - m) is split
 // like the rest.  Windows whose V spans more than that holds (SPREAD_CHANNELS,
-// SPREAD_BLOCKS) are computed with fp32 MFMAs instead (exact_queries).  Up to
-// there the error is that of N(0, 1) inputs: half of the rows 2^-5 of the others,
-// or a sixteenth of the channels 2^7 times the others, 3.1e-7 to 3.3e-7 at 360p
-// and at most 6.1e-7 in the worst channel, against 4.4e-7 and 9.0e-7 as fp32
-// MFMAs.
+// SPREAD_BLOCKS) take three bf16 values of V and P instead (wide_item), those with
+// infinities, the ends of fp32's range or gains that cancel fp32 MFMAs
+// (full_queries).  Up to there the error is that of N(0, 1) inputs: half of the
+// rows 2^-5 of the others, or a sixteenth of the channels 2^7 times the others,
+// 3.1e-7 to 3.3e-7 at 360p and at most 6.1e-7 in the worst channel, against 4.4e-7
+// and 9.0e-7 as fp32 MFMAs.
 //
 // The query rows are normalised and rotated here (each is read by one
 // workgroup), K and V come from the pack kernel as hi and lo tiles in fragment
@@ -94,7 +95,7 @@ __device__ inline float wave_max(float v) {
 // P is at most 2^M_STALE (the running maximum stays until a tile's exceeds it by
 // more, so that O is rarely rescaled), times 2^P_SHIFT and the V block's power of
 // two relative to the window's largest (2^-SPREAD_BLOCKS at least, else the
-// window goes to exact_queries): below 2^16, and down to 2^-22 of the largest
+// window goes to wide_item): below 2^16, and down to 2^-22 of the largest
 // (2^-16 for the smallest blocks) in fp16's normal range; below that it is held
 // to 2^-33 (2^-27).
 constexpr float P_SHIFT = 8.f, M_STALE = 7.f;
@@ -132,19 +133,19 @@ __device__ inline void dma_quarter(const void* unit, uint32_t part, uint32_t lan
 // This wave's DMA has landed and its LDS reads are done, then the barrier.
 __device__ inline void unit_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// ---- windows whose V the split does not hold (SPREAD_CHANNELS): fp32 MFMAs
+// ---- windows with infinities, values at the ends of fp32's range or gains of q
+// and k that cancel (VEXP_FULL, QK_MAX): fp32 MFMAs
 //
 // The same workgroup and the same output for its query tile t, 16 queries a wave, as
 // plain fp32: K and V rows straight from vqkv / tqkv (K normalised and rotated
 // as the pack kernel does) into LDS, 32 keys at a time, and
 // v_mfma_f32_16x16x4_f32 for both products.  The fp32 MFMA's 32 cycles bound it,
-// so it neither pipelines nor shares a unit between two query blocks.  Channels
-// do not depend on each other here and any finite value keeps all its bits.
-// 1080p shifted with every window here: 454 us a pass, 171 on split operands.
+// so it neither pipelines nor shares a unit between two query blocks.
+// 1080p shifted with every window here: 454 us a pass, 360p 129.
 constexpr int EX_P = HEAD_D + 4;  // LDS pitch of a row (floats)
 constexpr int EX_STAGE = 2 * 32 * EX_P;  // K and V rows of a unit
 template <bool kSplit>
-__device__ inline void exact_queries(const SdpaArgs& a, const Item& wt, float* lds, int t) {
+__device__ inline void full_queries(const SdpaArgs& a, const Item& wt, float* lds, int t) {
     const int h = wt.h;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // addresses of its own, none held across
@@ -319,8 +320,74 @@ __device__ inline QueryRows query_rows(const SdpaArgs& a, const Item& wt, int nq
     return r;
 }
 
-// The largest V exponent of the window, in whose units P V is accumulated, or
-// VEXP_WIDE where the split does not hold the window: the same in every wave.
+// This wave's queries, 16-row blocks NQ w4 + qb of the item, normalised, rotated and
+// split (2^-a to cq): every load issued before the first use.
+template <int NQ>
+__device__ inline void load_queries(const SdpaArgs& a, const Item& wt, const QueryRows& rows, int w4, int lane,
+                                    f16x8 (&qh)[NQ][4], f16x8 (&ql)[NQ][4], float (&cq)[NQ]) {
+    const int h = wt.h, r16 = lane & 15, q = lane >> 4;
+    float4 xr[NQ][8], cs[NQ][8];
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
+        const bool txt = kq >= wt.nvt;
+        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + rows.ofs[qb] + h * HEAD_D + 8 * q;
+        const float4* cst = reinterpret_cast<const float4*>(txt ? a.tcs : a.vcs) +
+                            ((size_t)rows.meta[qb].x + min(slot, rows.meta[qb].y - 1)) * (CS_STRIDE / 2) + 2 * q;
+#pragma unroll
+        for (int i = 0; i < 8; i++) xr[qb][i] = *reinterpret_cast<const float4*>(row + 32 * (i >> 1) + 4 * (i & 1));
+#pragma unroll
+        for (int i = 0; i < 8; i++) cs[qb][i] = cst[8 * (i >> 1) + (i & 1)];
+    }
+
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        float x[32];
+        float ss = 0.f;
+        const float* gain = ((NQ * w4 + qb < 4 ? wt.kq0 : wt.kq1) >= wt.nvt ? a.nq_t : a.nq_v) + 8 * q;
+        float gr[32];
+#pragma unroll
+        for (int i = 0; i < 32; i++) gr[i] = gain[32 * (i >> 3) + (i & 7)];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            x[4 * i] = xr[qb][i].x; x[4 * i + 1] = xr[qb][i].y; x[4 * i + 2] = xr[qb][i].z; x[4 * i + 3] = xr[qb][i].w;
+        }
+#pragma unroll
+        for (int i = 0; i < 32; i++) ss += x[i] * x[i];
+        ss = sum4(ss);
+        // x / n g, rotated, times the softmax scale
+        const float in = a.qscale / sqrtf(ss / (float)HEAD_D + a.eps);
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float c4[4] = {cs[qb][i].x, cs[qb][i].y, cs[qb][i].z, cs[qb][i].w};
+#pragma unroll
+            for (int p = 0; p < 4; p += 2) {
+                const float x0 = x[4 * i + p] * in * gr[4 * i + p], x1 = x[4 * i + p + 1] * in * gr[4 * i + p + 1];
+                x[4 * i + p] = x0 * c4[p] - x1 * c4[p + 1];
+                x[4 * i + p + 1] = x1 * c4[p] + x0 * c4[p + 1];
+                mx = fmaxf(mx, fmaxf(fabsf(x[4 * i + p]), fabsf(x[4 * i + p + 1])));
+            }
+        }
+        const float f = split_scale(max4(mx), SPLIT_FLOOR_QK);
+        cq[qb] = 1.f / f;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            float y[8];
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = x[8 * st + i] * f;
+            split8(y, hi, lo);
+            qh[qb][st] = __builtin_bit_cast(f16x8, hi);
+            ql[qb][st] = __builtin_bit_cast(f16x8, lo);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one block's gains at a time: registers
+    }
+}
+
+// The largest V exponent of the window, in whose units P V is accumulated, or,
+// where the split does not hold the window, VEXP_WIDE (wide_item) or VEXP_FULL
+// (full_queries): the same in every wave.
 __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane) {
     const float *ve = a.vexp + (size_t)wt.h * a.n_tiles * 4, *ke = a.kexp + (size_t)wt.h * a.n_tiles * 4;
     static_assert(HEAD_D == 128, "two gains per lane");
@@ -338,8 +405,214 @@ __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane)
     vmin = -wave_max(-vmin);
     // a normalised query's largest value is below sqrt(2 128) qscale = 2.05 times
     // its largest gain, a key's below 2^15 times its block's 2^-a
-    const float qk = wave_max(g) * wave_max(kmax) * 65536.f;
-    return vmin < vmax - SPREAD_BLOCKS || qk > QK_MAX || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
+    if (vmax == VEXP_FULL || !(wave_max(g) * wave_max(kmax) * 65536.f <= QK_MAX)) return VEXP_FULL;
+    return vmin < vmax - SPREAD_BLOCKS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
+}
+
+// ---- windows whose V the split does not hold
+//
+// run_item with P V formed from three bf16 values of V and of P (split3: all 24
+// significand bits and fp32's exponents; six MFMAs a product, the dropped ones
+// below 2^-25 of it).  Nothing of V is scaled, so channels do not depend on each
+// other and any finite value keeps all its bits.  K comes by DMA as there; V rows
+// are gathered from vqkv / tqkv a unit ahead, each thread the eight keys of two
+// channels, and reach LDS as three planes of fragments.  Not pipelined between
+// units.
+// With every window here 1080p shifted takes 219 us a pass and 360p 60 (the fp32 MFMA
+// kernel that the split replaced 371 and 60, split operands 171 and 45), with less
+// error than either: 3.1e-7 at 360p, worst channel 4.3e-7.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+// eight floats = the sum of three bf16 vectors, largest first
+__device__ inline void split3(const float* x, bf16x8 (&f)[3]) {
+    u32x4 u[3];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            u[p][i] = bf16x2_rne(a, b);
+            a -= __uint_as_float(u[p][i] << 16);
+            b -= __uint_as_float(u[p][i] & 0xffff0000u);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) f[p] = __builtin_bit_cast(bf16x8, u[p]);
+}
+
+template <int NQ, bool kSplit>
+__device__ inline void wide_item(const SdpaArgs& a, const Item& wt, const QueryRows& rows, unsigned char* lds) {
+    const int h = wt.h;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // addresses of its own, none held across
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int half = kSplit ? wave >> 2 : 0, w4 = wave & 3, r16 = lane & 15, q = lane >> 4;
+    const int nu = wt.units(), n0 = kSplit ? (nu + 1) >> 1 : nu;
+    const int ubeg = half ? n0 : 0, uend = half ? nu : n0;
+    // LDS of a half: two K units, then V's planes [plane][channel block][lane]
+    static_assert(V_RING + 3 * 8 * 1024 <= STAGE_BYTES, "the planes fit");
+    unsigned char* stage = lds + half * STAGE_BYTES;
+    const uint32_t ldsb = (uint32_t)(uintptr_t)(lptr_t)lds + half * STAGE_BYTES;
+    const f16x8* kf = reinterpret_cast<const f16x8*>(stage) + lane;
+    bf16x8* vf = reinterpret_cast<bf16x8*>(stage + V_RING) + lane;
+    const unsigned char* Kh = reinterpret_cast<const unsigned char*>(a.Kp) + (size_t)h * a.n_tiles * (2 * FU_BYTES);
+    const cfloat2_t* ke = (const cfloat2_t*)(a.kexp) + (size_t)h * a.n_tiles * 2;
+    auto fetch_k = [&](int u, int slot) __attribute__((always_inline)) {
+        if (u < uend)
+            dma_quarter(Kh + (size_t)wt.unit_half(u) * FU_BYTES, 4096u * w4, 16u * lane, ldsb + slot * FU_BYTES);
+    };
+    // V of a unit: keys {4 q + e, 16 + 4 q + e} of channels 16 (w4 + 4 j) + r16
+    uint32_t vofs[8];  // rows of the unit after the one in rv
+    float rv[16];
+    auto load_rows = [&](int u) __attribute__((always_inline)) {
+        const int t2 = wt.unit_half(u), tile = t2 >> 1;
+        const uint32_t* vr = a.vrow + (size_t)(u >= wt.vid_units() ? a.n_vid_tiles + (tile - wt.tbase) : tile) * TILE;
+#pragma unroll
+        for (int e = 0; e < 8; e++) vofs[e] = vr[vrow_pos(32 * (t2 & 1) + 16 * (e >> 2) + 4 * q + (e & 3))];
+    };
+    auto load_v = [&](int u) __attribute__((always_inline)) {
+        const float* src =
+            reinterpret_cast<const float*>(u >= wt.vid_units() ? a.tsrc : a.vsrc) + 2 * DIM + h * HEAD_D + 16 * w4 + r16;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) rv[8 * j + e] = src[vofs[e] + 64 * j];
+    };
+    fetch_k(ubeg, 0);
+    if (ubeg < uend) load_rows(ubeg);
+    f16x8 qh[NQ][4], ql[NQ][4];
+    float cq[NQ];
+    load_queries(a, wt, rows, w4, lane, qh, ql, cq);
+    if (ubeg < uend) {
+        load_v(ubeg);
+        if (ubeg + 1 < uend) load_rows(ubeg + 1);
+    }
+
+    f32x4 oacc[8][NQ];
+    float m[NQ], l[NQ];
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        m[qb] = -INFINITY;
+        l[qb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < 8; db++) oacc[db][qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    for (int i = 0; i < n0; i++) {  // the same iteration count in both halves
+        const int u = ubeg + i, slot = i & 1;
+        unit_barrier();  // K(u) has landed, every wave is done with V(u - 1) and K(u - 1)
+        fetch_k(u + 1, slot ^ 1);
+        bf16x8 pf[NQ][3];
+        if (u < uend) {  // uniform per half
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                bf16x8 f[3];
+                split3(rv + 8 * j, f);
+#pragma unroll
+                for (int p = 0; p < 3; p++) vf[64 * (8 * p + w4 + 4 * j)] = f[p];
+            }
+            if (u + 1 < uend) load_v(u + 1);
+            if (u + 2 < uend) load_rows(u + 2);
+            // scores: lane has keys 16 kb + 4 q + r of query r16
+            f32x4 s[2][NQ];
+#pragma unroll
+            for (int st = 0; st < 4; st++) {
+                f16x8 f[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[e] = kf[slot * (FU_BYTES / 16) + 64 * f32_kfrag(e >> 1, st, e & 1)];
+#pragma unroll
+                for (int pr = 0; pr < 3; pr++)
+#pragma unroll
+                    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                        for (int qb = 0; qb < NQ; qb++)
+                            s[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                f[2 * kb + (pr == 0)], pr == 1 ? ql[qb][st] : qh[qb][st],
+                                st == 0 && pr == 0 ? (f32x4){0.f, 0.f, 0.f, 0.f} : s[kb][qb], 0, 0, 0);
+            }
+            const int kv = wt.unit_valid(u);
+            const f32x2 kc = ke[wt.unit_half(u)];
+#pragma unroll
+            for (int qb = 0; qb < NQ; qb++) {
+                float p[8], mx = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    p[e] = 16 * (e >> 2) + 4 * q + (e & 3) < kv ? s[e >> 2][qb][e & 3] * (cq[qb] * kc[e >> 2]) : -INFINITY;
+                    mx = fmaxf(mx, p[e]);
+                }
+                mx = max4(mx);
+                if (__any(mx > m[qb])) {
+                    const float m_new = fmaxf(m[qb], mx), alpha = __builtin_amdgcn_exp2f(m[qb] - m_new);
+                    m[qb] = m_new;
+                    l[qb] *= alpha;
+#pragma unroll
+                    for (int db = 0; db < 8; db++) oacc[db][qb] *= alpha;
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    p[e] = __builtin_amdgcn_exp2f(p[e] - m[qb]);
+                    l[qb] += p[e];  // this lane's keys; summed over the row at the end
+                }
+                split3(p, pf[qb]);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // V(u)'s planes are complete
+        if (u < uend) {
+            constexpr int order[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // small products first
+#pragma unroll
+            for (int db = 0; db < 8; db += 2) {
+                bf16x8 f[2][3];
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int p = 0; p < 3; p++) f[e][p] = vf[64 * (8 * p + db + e)];
+#pragma unroll
+                for (int o = 0; o < 6; o++)
+#pragma unroll
+                    for (int e = 0; e < 2; e++)
+#pragma unroll
+                        for (int qb = 0; qb < NQ; qb++)
+                            oacc[db + e][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[e][order[o][0]], pf[qb][order[o][1]],
+                                                                                       oacc[db + e][qb], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) l[qb] = sum4(l[qb]);
+    if constexpr (kSplit) {  // half 1 leaves its share in its stage, half 0 merges it (as run_item)
+        __syncthreads();
+        f32x4* pub = reinterpret_cast<f32x4*>(lds + STAGE_BYTES) + (size_t)w4 * (8 * NQ * 64) + lane;
+        float* pml = reinterpret_cast<float*>(lds) + (size_t)w4 * (2 * NQ * 64) + lane;  // half 0's stage is free
+        if (half == 1) {
+#pragma unroll
+            for (int qb = 0; qb < NQ; qb++) {
+#pragma unroll
+                for (int db = 0; db < 8; db++) pub[64 * (8 * qb + db)] = oacc[db][qb];
+                pml[64 * (2 * qb)] = m[qb];
+                pml[64 * (2 * qb + 1)] = l[qb];
+            }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int qb = 0; qb < NQ; qb++) {
+            const float m1 = pml[64 * (2 * qb)], l1 = pml[64 * (2 * qb + 1)], mm = fmaxf(m[qb], m1);
+            const float a0 = __builtin_amdgcn_exp2f(m[qb] - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
+            l[qb] = l[qb] * a0 + l1 * a1;
+#pragma unroll
+            for (int db = 0; db < 8; db++) oacc[db][qb] = oacc[db][qb] * a0 + pub[64 * (8 * qb + db)] * a1;
+        }
+    }
+#pragma unroll
+    for (int qb = 0; qb < NQ; qb++) {
+        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
+        if (slot >= wt.nvalid(kq)) continue;  // padding
+        float* dst = kq < wt.nvt ? reinterpret_cast<float*>(a.vattn) + rows.ofs[qb] / 3
+                                 : a.tpart + ((size_t)wt.w * a.txt_len + TILE * (kq - wt.nvt) + slot) * DIM;
+        const float inv = 1.f / l[qb];
+#pragma unroll
+        for (int db = 0; db < 8; db++)
+            *reinterpret_cast<f32x4*>(dst + h * HEAD_D + 16 * db + 4 * q) = oacc[db][qb] * inv;
+    }
 }
 
 // One workgroup per (two query tiles of a window, head), 128 queries: four
@@ -418,67 +691,9 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
 #pragma unroll
         for (int qb = 0; qb < NQ; qb++) out_ofs[16 * (NQ * w4 + qb) + r16] = rows.ofs[qb];
 
-    // ---- this wave's queries: 16-row blocks NQ w4 + qb of the item, every load
-    // issued before the first use
-    float4 xr[NQ][8], cs[NQ][8];
-#pragma unroll
-    for (int qb = 0; qb < NQ; qb++) {
-        const int blk = NQ * w4 + qb, kq = blk < 4 ? wt.kq0 : wt.kq1, slot = 16 * (blk & 3) + r16;
-        const bool txt = kq >= wt.nvt;
-        const float* row = reinterpret_cast<const float*>(txt ? a.tsrc : a.vsrc) + rows.ofs[qb] + h * HEAD_D + 8 * q;
-        const float4* cst = reinterpret_cast<const float4*>(txt ? a.tcs : a.vcs) +
-                            ((size_t)rows.meta[qb].x + min(slot, rows.meta[qb].y - 1)) * (CS_STRIDE / 2) + 2 * q;
-#pragma unroll
-        for (int i = 0; i < 8; i++) xr[qb][i] = *reinterpret_cast<const float4*>(row + 32 * (i >> 1) + 4 * (i & 1));
-#pragma unroll
-        for (int i = 0; i < 8; i++) cs[qb][i] = cst[8 * (i >> 1) + (i & 1)];
-    }
-
     f16x8 qh[NQ][4], ql[NQ][4];
     float cq[NQ];
-#pragma unroll
-    for (int qb = 0; qb < NQ; qb++) {
-        float x[32];
-        float ss = 0.f;
-        const float* gain = ((NQ * w4 + qb < 4 ? wt.kq0 : wt.kq1) >= wt.nvt ? a.nq_t : a.nq_v) + 8 * q;
-        float gr[32];
-#pragma unroll
-        for (int i = 0; i < 32; i++) gr[i] = gain[32 * (i >> 3) + (i & 7)];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            x[4 * i] = xr[qb][i].x; x[4 * i + 1] = xr[qb][i].y; x[4 * i + 2] = xr[qb][i].z; x[4 * i + 3] = xr[qb][i].w;
-        }
-#pragma unroll
-        for (int i = 0; i < 32; i++) ss += x[i] * x[i];
-        ss = sum4(ss);
-        // x / n g, rotated, times the softmax scale
-        const float in = a.qscale / sqrtf(ss / (float)HEAD_D + a.eps);
-        float mx = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float c4[4] = {cs[qb][i].x, cs[qb][i].y, cs[qb][i].z, cs[qb][i].w};
-#pragma unroll
-            for (int p = 0; p < 4; p += 2) {
-                const float x0 = x[4 * i + p] * in * gr[4 * i + p], x1 = x[4 * i + p + 1] * in * gr[4 * i + p + 1];
-                x[4 * i + p] = x0 * c4[p] - x1 * c4[p + 1];
-                x[4 * i + p + 1] = x1 * c4[p] + x0 * c4[p + 1];
-                mx = fmaxf(mx, fmaxf(fabsf(x[4 * i + p]), fabsf(x[4 * i + p + 1])));
-            }
-        }
-        const float f = split_scale(max4(mx), SPLIT_FLOOR_QK);
-        cq[qb] = 1.f / f;
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            float y[8];
-            uint32_t hi[4], lo[4];
-#pragma unroll
-            for (int i = 0; i < 8; i++) y[i] = x[8 * st + i] * f;
-            split8(y, hi, lo);
-            qh[qb][st] = __builtin_bit_cast(f16x8, hi);
-            ql[qb][st] = __builtin_bit_cast(f16x8, lo);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one block's gains at a time: registers
-    }
+    load_queries(a, wt, rows, w4, lane, qh, ql, cq);
 
     f32x4 oacc[8][NQ];
     float m_i[NQ], l_i[NQ];
@@ -735,12 +950,16 @@ __global__ __launch_bounds__(kSplit ? 512 : 256, 2) void sdpa_f32_kernel(SdpaArg
     const QueryRows rows =
         query_rows(a, it, nq, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3, threadIdx.x & 15);
     const float vmax = window_vmax(a, it, threadIdx.x & 63);
-    if (vmax == VEXP_WIDE) {
-        for (int t = 0; t < nq; t++) exact_queries<kSplit>(a, it, reinterpret_cast<float*>(lds), t);
-        return;
+    const int mode = __builtin_amdgcn_readfirstlane(vmax == VEXP_FULL ? 2 : vmax == VEXP_WIDE);  // a scalar branch
+    if (mode == 0) {
+        if (nq == 2) run_item<2, kSplit>(a, it, rows, vmax, lds, out_ofs);
+        else run_item<1, kSplit>(a, it, rows, vmax, lds, out_ofs);
+    } else if (mode == 1) {
+        if (nq == 2) wide_item<2, kSplit>(a, it, rows, lds);
+        else wide_item<1, kSplit>(a, it, rows, lds);
+    } else {
+        for (int t = 0; t < nq; t++) full_queries<kSplit>(a, it, reinterpret_cast<float*>(lds), t);
     }
-    if (nq == 2) run_item<2, kSplit>(a, it, rows, vmax, lds, out_ofs);
-    else run_item<1, kSplit>(a, it, rows, vmax, lds, out_ofs);
 }
 
 }  // namespace

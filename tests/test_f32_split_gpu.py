@@ -165,3 +165,34 @@ def test_opposite_gains(oracle, ctx, shape):
             gains[i] = (gains[i] * (s if i % 2 == 0 else 1 / s)).astype(np.float32)
     for a, b in zip(*both(oracle, ctx, shape, change)):
         assert worst_channel(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+@pytest.mark.parametrize("small,large", [(-98, 0), (-110, 0), (-60, 60), (-112, -112)])
+def test_ends_of_the_range(oracle, ctx, shape, small, large):
+    """Channels of V near both ends of fp32's range, alone and side by side."""
+    def change(vqkv, tqkv, gains):
+        for x in (vqkv, tqkv):
+            x[:, 5120::2] *= np.float32(2.0 ** small)
+            x[:, 5121::2] *= np.float32(2.0 ** large)
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert worst_channel(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("h,w,nw,txt", [(1, 1, (1, 1, 1), 1), (1, 31, (1, 1, 1), 32), (4, 8, (1, 1, 1), 33),
+                                        (3, 11, (1, 1, 1), 64), (8, 16, (1, 1, 1), 65), (13, 5, (1, 1, 1), 31),
+                                        (10, 29, (1, 2, 2), 58), (30, 41, (1, 4, 4), 77)])
+@pytest.mark.parametrize("kind", ["wide", "full"])
+def test_wide_edges(oracle, ctx, h, w, nw, txt, kind):
+    """The paths of windows that the split does not hold, at the edges of their
+    units and halves: channels of V 2^24 apart, and gains that cancel."""
+    def change(vqkv, tqkv, gains):
+        s = np.exp2(12.0 * (np.arange(128) // 2 % 3 - 1)).astype(np.float32)
+        if kind == "wide":
+            for x in (vqkv, tqkv):
+                x[:, 5120:] *= np.tile(s, 20)
+        else:
+            for i in range(4):
+                gains[i] = (gains[i] * (s if i % 2 == 0 else 1 / s)).astype(np.float32)
+    for a, b in zip(*both(oracle, ctx, (h, w, nw, txt), change, seed=100 * h + w)):
+        assert rel(a, b) <= 5e-6
