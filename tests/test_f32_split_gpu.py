@@ -196,3 +196,30 @@ def test_wide_edges(oracle, ctx, h, w, nw, txt, kind):
                 gains[i] = (gains[i] * (s if i % 2 == 0 else 1 / s)).astype(np.float32)
     for a, b in zip(*both(oracle, ctx, (h, w, nw, txt), change, seed=100 * h + w)):
         assert rel(a, b) <= 5e-6
+
+
+@pytest.mark.parametrize("txt", [9, 77])
+@pytest.mark.parametrize("kind", ["split", "wide", "full"])
+def test_text_tables_per_window(oracle, ctx, txt, kind):
+    """Windows with a text RoPE table (and so text tiles) of their own, one of them
+    without video rows, on each path."""
+    import types
+    og = oracle.Geometry(1, 23, 27, (4, 3, 3), txt, 0)
+    sl = np.insert(og.slices, 2, [0, 1, 5, 5, 0, 27], axis=0).astype(np.int32)
+    nwin = og.nwin + 1
+    tf = np.concatenate([og.txt_freq[:txt] * np.float32(1 + 0.25 * w) for w in range(nwin)])
+    geo = types.SimpleNamespace(t=1, h=23, w=27, Lv=og.Lv, txt_len=txt, slices=sl, nwin=nwin, vid_freq=og.vid_freq,
+                                txt_freq=np.ascontiguousarray(tf))
+    g = ctx.geometry_from_win(1, 23, 27, sl, og.vid_freq, geo.txt_freq, txt)
+    vqkv, tqkv, gains = seeded_awa_inputs(og.Lv, txt, 90 + txt)
+    s = np.exp2(12.0 * (np.arange(128) // 2 % 3 - 1)).astype(np.float32)
+    if kind == "wide":
+        for x in (vqkv, tqkv):
+            x[:, 5120:] *= np.tile(s, 20)
+    elif kind == "full":
+        for i in range(4):
+            gains[i] = (gains[i] * (s if i % 2 == 0 else 1 / s)).astype(np.float32)
+    ref = oracle.awa_forward(vqkv, tqkv, geo, *gains, eps=1e-5)
+    for a, b in zip(run(ctx, g, vqkv, tqkv, gains), ref):
+        assert np.isfinite(a).all() and rel(a, b) <= 5e-6
+    g.close()
