@@ -125,8 +125,11 @@ __device__ inline void store_cs(float4* lds_cs, const float4 (&t)[CS_PT], int ti
 // leave as split fp16 tiles in fragment order (f32_kfrag), each 16-row block
 // scaled by its own power of two (split_scale of its largest finite
 // magnitude), whose inverse or exponent goes to kexp / vexp; V is transposed through LDS.
-// whole-tile workgroups from this many (tile, head) pairs on (measured: quarters
-// faster up to 1,200 pairs, whole tiles from 1,900)
+// The blocks' ranges are checked on the way (SPREAD_CHANNELS; 1080p 53 -> 56 us).
+// whole-tile workgroups from this many (tile, head) pairs on (measured on the whole
+// op: quarters 98 against 105 us at 1,260 pairs, equal within the runs at 1,340, whole
+// tiles 129 against 131 at 1,540 and 167 against 169 at 1,980; the kernel alone, its
+// inputs in the memory-side cache, would have quarters up to 1,660)
 constexpr long F32_WHOLE_MIN = 1536;
 template <int QR>
 __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
