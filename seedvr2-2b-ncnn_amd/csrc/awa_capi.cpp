@@ -415,15 +415,15 @@ hipError_t timing_mark(awa_ctx* ctx, hipStream_t s) { return event_mark(ctx, ctx
 namespace awa {
 
 namespace {
-// The op's scratch: bf16 Q and K tiles, fp32 the blocks' factors (kexp, then
-// vexp), K and V tiles; then the text partials.
+// The op's scratch: bf16 Q and K tiles, fp32 the blocks' factors (kexp, vexp,
+// vrmin), K and V tiles; then the text partials.
 struct ScratchLayout {
     size_t off_k, off_v, off_t, bytes;
     size_t rows;  // the video rows, past `bytes`: for a call whose vattn lies over its inputs
     ScratchLayout(const GeomPlan& P, int dtype) {
         const bool bf16 = dtype == AWA_BF16;
         const size_t packed = align256((size_t)HEADS * P.n_tiles * TILE * HEAD_D * elem_size(dtype));
-        off_k = bf16 ? packed : align256((size_t)2 * HEADS * P.n_tiles * 4 * sizeof(float));
+        off_k = bf16 ? packed : align256((size_t)3 * HEADS * P.n_tiles * 4 * sizeof(float));
         off_v = off_k + packed;
         off_t = bf16 ? off_v : off_v + packed;
         bytes = off_t + align256((size_t)P.nwin * P.txt_len * DIM * 4);
@@ -484,6 +484,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     pa.vcs = g->d_vcs; pa.tcs = g->d_tcs;
     pa.Qp = bf16 ? base : nullptr; pa.Kp = base + lay.off_k; pa.Vp = bf16 ? nullptr : base + lay.off_v;
     pa.kexp = reinterpret_cast<float*>(base); pa.vexp = pa.kexp + (size_t)HEADS * P.n_tiles * 4;
+    pa.vrmin = pa.vexp + (size_t)HEADS * P.n_tiles * 4;
     pa.n_vid_tiles = P.n_vid_tiles; pa.ntt = P.ntt; pa.txt_sets = P.txt_sets; pa.txt_len = P.txt_len;
     pa.n_tiles = P.n_tiles; pa.eps = eps;
     pa.qscale = (1.0f / std::sqrt(128.0f)) * 1.4426950408889634f;
@@ -502,7 +503,7 @@ int forward_impl(awa_ctx* ctx, const awa_geom* g, int dtype, const void* d_vqkv,
     sa.n_vid_tiles = P.n_vid_tiles; sa.ntt = P.ntt; sa.txt_len = P.txt_len;
     sa.n_tiles = P.n_tiles;
     sa.f32_work = g->d_f32_work; sa.n_f32_work = (int)P.f32_work.size();
-    sa.kexp = pa.kexp; sa.vexp = pa.vexp;
+    sa.kexp = pa.kexp; sa.vexp = pa.vexp; sa.vrmin = pa.vrmin;
     sa.tile_meta = g->d_tile_meta; sa.vcs = g->d_vcs; sa.tcs = g->d_tcs; sa.nq_v = d_nq_v; sa.nq_t = d_nq_t;
     sa.nk_v = d_nk_v; sa.nk_t = d_nk_t;
     sa.eps = eps; sa.qscale = pa.qscale;

@@ -105,18 +105,20 @@ __device__ inline float max4(float v) {
 // Where split V loses nothing: an element keeps 2^-40 of its 16-row block's
 // largest and a probability 2^-33 times the window's largest block over its
 // own (awa_sdpa_f32.hip), so a channel must not be much smaller than the others
-// of its blocks, nor a block than the others of its window.  The pack kernel
+// of its blocks, nor a row than the others of its window (a large row of small
+// weight would lose that weight's bits).  The pack kernel
 // marks a block wide (VEXP_WIDE in place of its exponent) if the largest value
 // of a channel, zero channels aside, is over 2^SPREAD_CHANNELS below the block's
 // largest (whole blocks only: one or two rows hold small values by chance); the
 // attention kernel takes operands of three bf16 values for a window with a wide
-// block, with blocks over 2^SPREAD_BLOCKS apart or without any whole block.
+// block, with rows (their largest values; zero rows aside) over 2^SPREAD_ROWS apart
+// or without any whole block.
 // VEXP_FULL marks a block with an infinity in K or V (which splits into infinity
 // and NaN; a NaN stays one either way) or with values at the ends of fp32's
 // range (2^127, where a bf16 may round to infinity; below 2^SPLIT_FLOOR_V, the
 // channels of a wide block too, whose last bits would be subnormal): its windows
 // take fp32 MFMAs.
-constexpr int SPREAD_CHANNELS = 10, SPREAD_BLOCKS = 6;
+constexpr int SPREAD_CHANNELS = 10, SPREAD_ROWS = 6;
 constexpr float VEXP_WIDE = 1000.f, VEXP_FULL = 2000.f, VEXP_ZERO = -1000.f;
 
 // Fragment order of a packed fp32 tile (32 fragments of 1 KiB, lane l's 16 bytes
@@ -357,7 +359,8 @@ struct PackArgs {
     void* Vp;              // fp32 storage only (the bf16 attention reads V from vqkv / tqkv)
     // fp32 storage: [HEADS][n_tiles][4], of each 16-row block with split_scale 2^a: 2^-a of K; -a of V,
     // VEXP_ZERO of a block of zeros, VEXP_WIDE or VEXP_FULL of one that the split does not hold
-    float *kexp, *vexp;
+    // and of V's rows that are not zero the smallest -a (by the row's own largest value)
+    float *kexp, *vexp, *vrmin;
     int n_vid_tiles, ntt, txt_sets, txt_len, n_tiles;
     float eps;
     float qscale;          // folded into Q: softmax scale 1/sqrt(128) times log2(e)
@@ -384,7 +387,7 @@ struct SdpaArgs {
     // rows' normalisation and rotation need (as in PackArgs)
     const int32_t* f32_work;
     int n_f32_work;
-    const float *kexp, *vexp;
+    const float *kexp, *vexp, *vrmin;
     const int32_t* tile_meta;
     const float2 *vcs, *tcs;
     const float *nq_v, *nq_t, *nk_v, *nk_t;

@@ -80,6 +80,12 @@ __device__ inline float row_sum16(float v) {
     v += dpp_move(v, 0x141);
     return v + dpp_move(v, 0x140);
 }
+__device__ inline float row_max16(float v) {
+    v = fmaxf(v, dpp_move(v, 0xB1));
+    v = fmaxf(v, dpp_move(v, 0x4E));
+    v = fmaxf(v, dpp_move(v, 0x141));
+    return fmaxf(v, dpp_move(v, 0x140));
+}
 __device__ inline float row_min16(float v) {
     v = fminf(v, dpp_move(v, 0xB1));
     v = fminf(v, dpp_move(v, 0x4E));
@@ -139,7 +145,7 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
     constexpr int NCS = QR * CS_Q4 / 256;         // table float4 per thread
     __shared__ __align__(16) float vs[QR * VP];
     __shared__ float4 lds_cs[QR * CS_Q4];
-    __shared__ float mxs[4][2 * RT], mns[4][RT];
+    __shared__ float mxs[4][2 * RT], mns[4][RT], rms[4][RT];
 
     const int nblk = a.n_tiles * HEADS * NQ;
     const int lid = xcd_remap(nblk);  // a tile's workgroups: neighbouring ids, one XCD
@@ -230,11 +236,15 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         vrow[0] = rv[kk].a;
         vrow[1] = rv[kk].b;
     }
-    // block maxima: 16 rows, so all four waves
+    // block maxima, and V's smallest row maximum: 16 rows, so all four waves
 #pragma unroll
     for (int i = 0; i < 2 * RT; i++) {
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], o));
+        mx[i] = row_max16(mx[i]);
+        if (i & 1) {
+            const float rm = -max4(mx[i] > 0.f ? -mx[i] : -INFINITY);
+            if ((tid & 63) == 0) rms[tid >> 6][i >> 1] = rm;
+        }
+        mx[i] = max4(mx[i]);
         if ((tid & 63) == 0) mxs[tid >> 6][i] = mx[i];
     }
     __syncthreads();
@@ -323,6 +333,8 @@ __global__ __launch_bounds__(256) void pack_f32_kernel(PackArgs a) {
         if (vm == 0.f) ve = VEXP_ZERO;
         else if (exponent(vm) < SPLIT_FLOOR_V || exponent(vm) >= 127) ve = VEXP_FULL;
         a.vexp[ht * 4 + b] = exponent(km) >= 127 ? VEXP_FULL : ve;
+        a.vrmin[ht * 4 + b] =
+            (float)(exponent(fminf(fminf(rms[0][tid], rms[1][tid]), fminf(rms[2][tid], rms[3][tid]))) - 14);
         a.kexp[ht * 4 + b] = 1.f / split_scale(km, SPLIT_FLOOR_QK);
     }
 }

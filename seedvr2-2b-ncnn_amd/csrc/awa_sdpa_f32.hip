@@ -20,12 +20,13 @@
 // the largest.  They are undone exactly: in the factor of the scores, in P
 // before its split, and in the normalisation of O.  P = exp2(s - m) is split
 // like the rest.  Windows whose V spans more than that holds (SPREAD_CHANNELS,
-// SPREAD_BLOCKS) take three bf16 values of V and P instead (wide_item), those with
+// SPREAD_ROWS) take three bf16 values of V and P instead (wide_item), those with
 // infinities, the ends of fp32's range or gains that cancel fp32 MFMAs
 // (full_queries).  Up to there the error is that of N(0, 1) inputs: half of the
 // rows 2^-5 of the others, or a sixteenth of the channels 2^7 times the others,
 // 3.1e-7 to 3.3e-7 at 360p and at most 6.1e-7 in the worst channel, against 4.4e-7
-// and 9.0e-7 as fp32 MFMAs.
+// and 9.0e-7 as fp32 MFMAs.  Scores that one channel carries (15 in log2 units) show
+// the missing bit: 9.8e-7 against 6.8e-7.
 //
 // The query rows are normalised and rotated here (each is read by one
 // workgroup), K and V come from the pack kernel as hi and lo tiles in fragment
@@ -94,7 +95,7 @@ __device__ inline float wave_max(float v) {
 
 // P is at most 2^M_STALE (the running maximum stays until a tile's exceeds it by
 // more, so that O is rarely rescaled), times 2^P_SHIFT and the V block's power of
-// two relative to the window's largest (2^-SPREAD_BLOCKS at least, else the
+// two relative to the window's largest (2^-SPREAD_ROWS at least, else the
 // window goes to wide_item): below 2^16, and down to 2^-22 of the largest
 // (2^-16 for the smallest blocks) in fp16's normal range; below that it is held
 // to 2^-33 (2^-27).
@@ -389,16 +390,16 @@ __device__ inline void load_queries(const SdpaArgs& a, const Item& wt, const Que
 // where the split does not hold the window, VEXP_WIDE (wide_item) or VEXP_FULL
 // (full_queries): the same in every wave.
 __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane) {
-    const float *ve = a.vexp + (size_t)wt.h * a.n_tiles * 4, *ke = a.kexp + (size_t)wt.h * a.n_tiles * 4;
+    const size_t head = (size_t)wt.h * a.n_tiles * 4;
+    const float *ke = a.kexp + head, *ve = a.vexp + head, *vr = a.vrmin + head;
     static_assert(HEAD_D == 128, "two gains per lane");
     const float g = fmaxf(fmaxf(fabsf(a.nq_v[lane]), fabsf(a.nq_v[lane + 64])),
                           fmaxf(fabsf(a.nq_t[lane]), fabsf(a.nq_t[lane + 64])));
     float vmax = VEXP_ZERO, vmin = VEXP_WIDE, kmax = 0.f;
     for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) {
         const int b = 4 * wt.tile(i >> 2) + (i & 3);
-        const float e = ve[b];
-        vmax = fmaxf(vmax, e);
-        if (e != VEXP_ZERO) vmin = fminf(vmin, e);
+        vmax = fmaxf(vmax, ve[b]);
+        vmin = fminf(vmin, vr[b]);
         kmax = fmaxf(kmax, ke[b]);
     }
     vmax = wave_max(vmax);
@@ -406,7 +407,7 @@ __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane)
     // a normalised query's largest value is below sqrt(2 128) qscale = 2.05 times
     // its largest gain, a key's below 2^15 times its block's 2^-a
     if (vmax == VEXP_FULL || !(wave_max(g) * wave_max(kmax) * 65536.f <= QK_MAX)) return VEXP_FULL;
-    return vmin < vmax - SPREAD_BLOCKS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
+    return vmin < vmax - SPREAD_ROWS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
 }
 
 // ---- windows whose V the split does not hold
@@ -781,7 +782,7 @@ __device__ inline void run_item(const SdpaArgs& a, const Item& wt, const QueryRo
         f32x2 vs = ve2[wt.unit_half(u)], vi;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
-            vs[kb] = scalar(fmaxf(vs[kb] - vmax, (float)-SPREAD_BLOCKS) + P_SHIFT);
+            vs[kb] = scalar(fmaxf(vs[kb] - vmax, (float)-SPREAD_ROWS) + P_SHIFT);
             vi[kb] = scalar(__builtin_amdgcn_exp2f(-vs[kb]));  // exact: whole exponents
         }
         uint32_t hi[NQ][4], lo[NQ][4];

@@ -223,3 +223,20 @@ def test_text_tables_per_window(oracle, ctx, txt, kind):
     for a, b in zip(run(ctx, g, vqkv, tqkv, gains), ref):
         assert np.isfinite(a).all() and rel(a, b) <= 5e-6
     g.close()
+
+
+@pytest.mark.parametrize("shape", [SPLIT, UNSPLIT])
+@pytest.mark.parametrize("e", [5, 12, 20, 28])
+def test_large_rows_of_small_weight(oracle, ctx, shape, e):
+    """Rows of V 2^e times the others, every eighth (so in every block), that all
+    queries give a weight of about 2^-30: q and k agree in channel 126 (which no
+    rotation touches), those rows' k has the other sign.  Scores of 15 in log2 units,
+    rounded at 2^-20, leave up to 3e-5 in the worst channel of either side: bar 1e-4."""
+    def change(vqkv, tqkv, gains):
+        for x in (vqkv, tqkv):
+            x[:, 126:2560:128] = 40
+            x[:, 2560 + 126:5120:128] = 40
+            x[::8, 2560 + 126:5120:128] = -40
+            x[::8, 5120:] *= np.float32(2.0 ** e)
+    for a, b in zip(*both(oracle, ctx, shape, change)):
+        assert worst_channel(a, b) <= 1e-4
