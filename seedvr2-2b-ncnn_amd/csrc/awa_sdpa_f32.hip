@@ -25,8 +25,10 @@
 // (full_queries).  Up to there the error is that of N(0, 1) inputs: half of the
 // rows 2^-5 of the others, or a sixteenth of the channels 2^7 times the others,
 // 3.1e-7 to 3.3e-7 at 360p and at most 6.1e-7 in the worst channel, against 4.4e-7
-// and 9.0e-7 as fp32 MFMAs.  Scores that one channel carries (15 in log2 units) show
-// the missing bit: 9.8e-7 against 6.8e-7.
+// and 9.0e-7 as fp32 MFMAs; with 1 % of the inputs 8 times as large 5.3e-7 against
+// 6.7e-7, with gains of 4 6.4e-7 against 1.1e-6.  Scores that a single channel carries
+// (15 in log2 units) show the missing bit and the dropped lo lo: 9.8e-7 against
+// 6.8e-7 (8.8e-7 with lo lo as a fourth MFMA, at 5 % of the op's time).
 //
 // The query rows are normalised and rotated here (each is read by one
 // workgroup), K and V come from the pack kernel as hi and lo tiles in fragment
