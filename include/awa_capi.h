@@ -52,8 +52,9 @@ enum { AWA_OK = 0, AWA_EARG = -1, AWA_EHIP = -2 };
  * error against 64 bits is below that of a chain of fp32 MFMAs (3.2e-7 for
  * 4.3e-7 on N(0, 1) inputs at 360p; where a single channel carries the scores up
  * to 1.5 times it) and channels do not depend on each other.
- * Windows with infinities, with values near the ends of fp32's range or with q
- * and k gains whose largest values multiply to over some 2^9 take fp32 MFMAs. */
+ * Windows with infinities, with values near the ends of fp32's range or with
+ * large q and k gains (over some 2^9 multiplied) that cancel channel by channel
+ * take fp32 MFMAs. */
 enum { AWA_F32 = 0, AWA_BF16 = 1 };
 
 enum { AWA_HEADS = 20, AWA_HEAD_D = 128, AWA_DIM = 2560, AWA_QKV = 7680,

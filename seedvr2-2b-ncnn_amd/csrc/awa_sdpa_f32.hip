@@ -104,12 +104,13 @@ __device__ inline float wave_max(float v) {
 constexpr float P_SHIFT = 8.f, M_STALE = 7.f;
 
 // The largest query value times the largest key value up to which the split
-// holds the scores.  Values are held to 2^-40 of the largest of their row or
-// block, so a score is off by up to some 2^-36 of this product: far below the
-// rounding of its own sum, unless the gains of q and k cancel channel by channel
-// (2^10 against 2^-10: product 2^21, error 1.8e-6 for 3.2e-7).  2^13 leaves 2^-26
-// (N(0, 1) rows and gains of 1: 2^4).
-constexpr float QK_MAX = 8192.f;
+// holds the scores whatever the gains.  Values are held to 2^-40 of the largest of
+// their row or block, so a score is off by up to some 2^-36 of this product: far
+// below the rounding of its own sum, unless the gains of q and k cancel channel by
+// channel (2^10 against 2^-10: product 2^21, error 1.8e-6 for 3.2e-7).  2^13 leaves
+// 2^-26 (N(0, 1) rows and gains of 1: 2^4).  Above it the largest gains must meet
+// in one channel, to GAIN_SPREAD.
+constexpr float QK_MAX = 8192.f, GAIN_SPREAD = 64.f;
 
 constexpr uint32_t FU_BYTES = 32 * HEAD_D * 4;  // a K or V unit (32 keys): hi and lo, 16 KiB
 constexpr uint32_t V_RING = 2 * FU_BYTES;       // LDS stage: two K units, then two V units
@@ -137,7 +138,7 @@ __device__ inline void dma_quarter(const void* unit, uint32_t part, uint32_t lan
 __device__ inline void unit_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // ---- windows with infinities, values at the ends of fp32's range or gains of q
-// and k that cancel (VEXP_FULL, QK_MAX): fp32 MFMAs
+// and k that cancel (VEXP_FULL, QK_MAX, GAIN_SPREAD): fp32 MFMAs
 //
 // The same workgroup and the same output for its query tile t, 16 queries a wave, as
 // plain fp32: K and V rows straight from vqkv / tqkv (K normalised and rotated
@@ -394,9 +395,17 @@ __device__ inline void load_queries(const SdpaArgs& a, const Item& wt, const Que
 __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane) {
     const size_t head = (size_t)wt.h * a.n_tiles * 4;
     const float *ke = a.kexp + head, *ve = a.vexp + head, *vr = a.vrmin + head;
+    // the largest gains of q and of k, and their largest product in one channel
     static_assert(HEAD_D == 128, "two gains per lane");
-    const float g = fmaxf(fmaxf(fabsf(a.nq_v[lane]), fabsf(a.nq_v[lane + 64])),
-                          fmaxf(fabsf(a.nq_t[lane]), fabsf(a.nq_t[lane + 64])));
+    float gq = 0.f, gk = 0.f, gqk = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float x = fmaxf(fabsf(a.nq_v[lane + 64 * i]), fabsf(a.nq_t[lane + 64 * i]));
+        const float y = fmaxf(fabsf(a.nk_v[lane + 64 * i]), fabsf(a.nk_t[lane + 64 * i]));
+        gq = fmaxf(gq, x);
+        gk = fmaxf(gk, y);
+        gqk = fmaxf(gqk, x * y);
+    }
     float vmax = VEXP_ZERO, vmin = VEXP_WIDE, kmax = 0.f;
     for (int i = lane; i < 4 * (wt.nvt + wt.ntt); i += 64) {
         const int b = 4 * wt.tile(i >> 2) + (i & 3);
@@ -408,7 +417,10 @@ __device__ inline float window_vmax(const SdpaArgs& a, const Item& wt, int lane)
     vmin = -wave_max(-vmin);
     // a normalised query's largest value is below sqrt(2 128) qscale = 2.05 times
     // its largest gain, a key's below 2^15 times its block's 2^-a
-    if (vmax == VEXP_FULL || !(wave_max(g) * wave_max(kmax) * 65536.f <= QK_MAX)) return VEXP_FULL;
+    gq = wave_max(gq);
+    const float qk = gq * wave_max(kmax) * 65536.f;
+    if (vmax == VEXP_FULL || !(qk < 0x1p100f) || (qk > QK_MAX && gq * wave_max(gk) > GAIN_SPREAD * wave_max(gqk)))
+        return VEXP_FULL;
     return vmin < vmax - SPREAD_ROWS || (wt.f < 16 && wt.txt < 16) ? VEXP_WIDE : vmax;
 }
 

@@ -240,3 +240,22 @@ def test_large_rows_of_small_weight(oracle, ctx, shape, e):
             x[::8, 5120:] *= np.float32(2.0 ** e)
     for a, b in zip(*both(oracle, ctx, shape, change)):
         assert worst_channel(a, b) <= 1e-4
+
+
+@pytest.mark.parametrize("gain", [1, 8, 48])
+def test_large_gains(ctx, gain):
+    """Gains far from 1 in every channel stay on the split operands.  Against the
+    fp32 path, which an infinity in one V channel of every head takes (the oracle's
+    exponentials overflow here): scores of up to 6 gain^2 in log2 units, off by a few
+    2^-24 of that on both sides, in a softmax that few keys share."""
+    h, w, nw, txt = SPLIT
+    geom = ctx.build_geometry(1, h, w, nw, txt, 0)
+    vqkv, tqkv, gains = seeded_awa_inputs(h * w, txt, 13)
+    gains = [g * np.float32(gain) for g in gains]
+    a = run(ctx, geom, vqkv, tqkv, gains)
+    vqkv[101, 5120::128] = np.inf
+    b = run(ctx, geom, vqkv, tqkv, gains)
+    keep = np.arange(2560) % 128 != 0
+    for x, y in zip(a, b):
+        assert np.isfinite(x).all() and rel(x[:, keep], y[:, keep]) <= 2e-6 * gain
+    geom.close()
