@@ -93,8 +93,11 @@ void dit_io_destroy(awa_ctx* ctx, dit_io* io) {
 
 namespace {
 // workspace bytes of each entry point (the offsets below follow the same layouts)
-// embed: the text's partial products, then copies of inputs that d_x lies over
-size_t embed_part_bytes(int TXT) { return align256((size_t)EMBED_TXT_SPLIT * TXT * DIM * 4); }
+// embed: the text's partial products, or a long text in bf16, then copies of inputs
+// that d_x lies over
+size_t embed_part_bytes(int TXT) {
+    return align256(TXT <= EMBED_TXT_MAX ? (size_t)EMBED_TXT_SPLIT * TXT * DIM * 4 : (size_t)TXT * 5120 * 2);
+}
 size_t grid_bytes(int Lv) { return (size_t)Lv * 4 * 33 * 4; }
 size_t txt_bytes(int TXT) { return (size_t)TXT * 5120 * 4; }
 size_t embed_ws_bytes(int Lv, int TXT) {
@@ -150,7 +153,22 @@ int dit_embed(awa_ctx* ctx, const dit_io* io, const float* d_grid, int T, int H,
         HIPCK(ctx, hipMemcpyAsync(copy, d_txt, txt_bytes(TXT), hipMemcpyDeviceToDevice, s));
         a.txt = reinterpret_cast<const float*>(copy);
     }
+    if (TXT <= EMBED_TXT_MAX) {
+        HIPCK(ctx, launch_embed(a, s));
+        return AWA_OK;
+    }
+    // a long text: x = A W^T + b by the residual epilogue on zeroed rows, gate 1
+    uint16_t* txt16 = static_cast<uint16_t*>(ctx->ws);
+    float* x_txt = d_x + (size_t)a.Lv * DIM;
+    HIPCK(ctx, launch_cast_f32_bf16(a.txt, txt16, (int64_t)TXT * 5120, s));
+    a.TXT = 0;
     HIPCK(ctx, launch_embed(a, s));
+    HIPCK(ctx, launch_zero(x_txt, (size_t)TXT * DIM * 4, s));
+    GemmBatch b{};
+    b.nprob = 1;
+    b.p[0] = problem(txt16, 5120, io->txt_in_w, 5120, TXT, DIM, 5120, x_txt, DIM);
+    b.p[0].bias = io->txt_in_b;
+    HIPCK(ctx, launch_gemm(EPI_RESID, b, s));
     return AWA_OK;
 }
 

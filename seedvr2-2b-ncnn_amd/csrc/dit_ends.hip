@@ -219,7 +219,8 @@ __global__ __launch_bounds__(256) void embed_weights_kernel(const uint16_t* __re
 // workgroups at once and are read once; fp32 partial products to the
 // workspace, summed in K order.  (Whole K per workgroup, 32 rows x 32 features
 // over eight waves, re-reads the text in every feature block: 28 us against 14
-// for the text alone.)
+// for the text alone.)  Up to EMBED_TXT_MAX rows; longer texts are left to the block's
+// GEMM and TXT is 0 here.
 constexpr int EMB_K = 160, EMB_LP = EMB_K + 8;  // k (padded) and LDS pitch of a patch row, bf16
 constexpr int EW = 8;  // waves of a workgroup
 constexpr int EMB_ROWS = 64, EMB_COLS = 64 * EW;
@@ -373,6 +374,7 @@ hipError_t launch_embed(const EmbedArgs& args, hipStream_t s) {
     a.txt_blocks = (a.TXT + TXT_ROWS - 1) / TXT_ROWS * (DIM / TXT_COLS) * EMBED_TXT_SPLIT;
     const int vid = (a.Lv + EMB_ROWS - 1) / EMB_ROWS * (DIM / EMB_COLS);
     hipLaunchKernelGGL(embed_kernel, dim3(a.txt_blocks + vid), dim3(64 * EW), 0, s, a);
+    if (a.TXT == 0) return hipGetLastError();
     const int n4 = a.TXT * (DIM / 4);
     hipLaunchKernelGGL(embed_sum_kernel, dim3((n4 + 255) / 256), dim3(256), 0, s, a.part, a.txt_b,
                        a.x + (size_t)a.Lv * DIM, n4);

@@ -67,10 +67,15 @@ hipError_t launch_time_mlp(float t, const float* const w[3], const float* const 
 // (T, H, 2 W2, 33) and the text features [TXT][5120].
 constexpr int EMBED_K = 160;  // 132 patch channels and zeros up to whole k32 steps
 constexpr int EMBED_TXT_SPLIT = 16;  // parts of the text projection's K
+// Up to this many text rows the embedding projects them itself; longer texts take the
+// block's GEMM, since the partial products are 160 KB a row.  On 400 video rows: 58 text
+// rows 17 us against 40, 320 44.3 against 45.3, 384 50.4 against 45.6, 2000 254
+// against 85; the same point with 5440 video rows.
+constexpr int EMBED_TXT_MAX = 320;
 struct EmbedArgs {
     const float* grid;
     int H, W2;
-    int Lv, TXT;
+    int Lv, TXT;  // TXT = 0: the video rows only
     const uint16_t* vid_w;  // [2560][EMBED_K] in fragment order
     const float* vid_b;
     const float* txt;

@@ -64,3 +64,20 @@ def test_final_edges(ctx, t, h, w):
     y = y @ wts["vid_out_w"].double().T + wts["vid_out_b"].double()
     ref = y.reshape(t, h, w, 2, 2, 16).permute(0, 1, 3, 2, 4, 5).reshape(t, 2 * h, 2 * w, 16)
     assert rel(out, ref) <= 1e-4
+
+
+@pytest.mark.parametrize("txt", [320, 321, 700])
+def test_embed_long_text(ctx, txt):
+    """Either side of the length from which the block's GEMM projects the text."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(txt)
+    wts, io = make_io(ctx, g)
+    grid = torch.randn((1, 6, 14, 33), generator=g, device="cuda")
+    text = torch.randn((txt, 5120), generator=g, device="cuda")
+    x = torch.full((21 + txt + 1, DIM), 7.0, device="cuda")  # one guard row
+    ctx.embed(io, grid, text, x=x)
+    p = grid.reshape(1, 3, 2, 7, 2, 33).permute(0, 1, 3, 2, 4, 5).reshape(-1, 132).bfloat16().double()
+    ref = torch.cat([p @ wts["vid_in_w"].double().T + wts["vid_in_b"].double(),
+                     text.bfloat16().double() @ wts["txt_in_w"].double().T + wts["txt_in_b"].double()])
+    assert rel(x[:21], ref[:21]) <= 1e-5 and rel(x[21:-1], ref[21:]) <= 1e-5
+    assert bool((x[-1] == 7.0).all())

@@ -34,12 +34,13 @@ def test_op_in_place(ctx, dtype, over, noalloc):
 
 
 @pytest.mark.parametrize("over", ["grid", "txt"])
-def test_embed_in_place(ctx, over):
+@pytest.mark.parametrize("txt", [90, 500])
+def test_embed_in_place(ctx, over, txt):
     import torch
     from test_dit_ends_gpu import make_io
     g = torch.Generator(device="cuda").manual_seed(5)
     _, io = make_io(ctx, g)
-    h, w, txt = 40, 50, 90
+    h, w = 40, 50
     inputs = {"grid": torch.randn((1, 2 * h, 2 * w, 33), generator=g, device="cuda"),
               "txt": torch.randn((txt, 5120), generator=g, device="cuda")}
     ref = ctx.embed(io, inputs["grid"], inputs["txt"])
